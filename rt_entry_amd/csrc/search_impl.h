@@ -20,7 +20,18 @@
 //  - neighbour ids that pass the filter are compacted before the gathers, so
 //    one iteration issues its loads together and only for points that need a
 //    distance; a lane reads its half-wave's ids in 16-byte LDS reads and
-//    forms each row address with one 32x32->64 multiply-add.
+//    forms each row address with one 32x32->64 multiply-add;
+//  - a batch of which few elements enter the beam is merged by ranks through
+//    LDS instead of by the networks (rank_merge);
+//  - the FAST kernels (one row per iteration, whole 32-dim groups, 32-bit row
+//    offsets) have the graph row expected next on its way while the current
+//    distances are gathered.
+// Against kernels that ran both networks on every step, formed 64-bit row
+// addresses and requested each row when its node was taken: 1M x 128, 10k
+// queries at beam 256 877 -> 826 us and 20k uneven ones at 96-d 2504 -> 2396 us
+// (of waiting and issue in about equal parts), 100k x 128 with 1k queries 170
+// -> 156 us (latency), 10k at 64-d with rerank 631 -> 566 us; 10k at beam 64
+// unchanged at 571 us, which reads 3.9 GB through the L2s at 7.1 TB/s.
 // Parity decisions P1-P7 match the CPU oracle (zeroed filter, all-ones first
 // mask, snapshot filter test per row, no row read for ids >= np,
 // barrier-separated substeps, REF/TUNED comparators).
@@ -168,6 +179,17 @@ constexpr uint64_t want_larger_mask(int r) {
   return m;
 }
 
+// A 64-bit constant made where it is used.  As a plain constant the compiler
+// keeps every mask of every network in scalar registers across the query
+// loop, runs out of them and moves them through VGPR lanes.
+template <uint64_t M>
+__device__ __forceinline__ uint64_t lane_mask_const() {
+  uint32_t lo, hi;
+  asm volatile("s_mov_b32 %0, %1" : "=s"(lo) : "i"((int)(uint32_t)M));
+  asm volatile("s_mov_b32 %0, %1" : "=s"(hi) : "i"((int)(uint32_t)(M >> 32)));
+  return ((uint64_t)hi << 32) | lo;
+}
+
 // Lane mask of "the partner's key is strictly larger / smaller" under the
 // configured comparator (P7).
 template <bool TUNED>
@@ -191,7 +213,7 @@ __device__ __forceinline__ void key_masks(float md, int mi, float pd, int pi, ui
 template <bool TUNED, int SUB, class Dir, int R, int RA, int r>
 __device__ __forceinline__ void stage_reg(float (&d)[R], int (&id)[R], int lane) {
   if constexpr (r < RA) {
-    constexpr uint64_t W = want_larger_mask<SUB, Dir>(r);
+    const uint64_t W = lane_mask_const<want_larger_mask<SUB, Dir>(r)>();
     const float pd = xor_lane<SUB>(d[r], lane);
     const int pi = xor_lane<SUB>(id[r], lane);
     uint64_t pgt, plt;
@@ -281,8 +303,12 @@ struct WaveLds {
   float* cdist;     // 64*MR compacted distances
   float* sbd;       // 64*MR sorted batch distances
   int* sbi;         // 64*MR sorted batch ids
-  float* qd;        // 64*NR beam distances (beam held in LDS)
-  int* qi;          // 64*NR beam ids (beam held in LDS)
+  float* ed;        // kRankMax + 4 distances of a rank merge's elements, then
+  int* eo;          // kRankMax owners by rank,
+  int2* es;         // kRankMax (distance, id) by rank and, for a beam in VGPRs,
+  int2* mbuf;       // 64*NR + 1 slots: laid over cid .. cdist, dead by then
+  float* qd;        // 64*NR + 1 beam distances (beam held in LDS)
+  int* qi;          // 64*NR + 1 beam ids (beam held in LDS)
 };
 
 // Expansion-flag ballots of the beam (graph_search.cuh:1014-1031): bf has
@@ -301,7 +327,7 @@ __device__ __forceinline__ void flag_ballots(const int (&li)[NR], int lane, int 
     // slot r*64 + lane < n, compared as lane < n - r*64 so that no slot
     // index per register stays live in a VGPR
     const bool in = lane < n - r * 64;
-    bf[r] = __ballot(in && li[r] > 0 && (int64_t)li[r] < np);
+    bf[r] = __ballot(in && (uint32_t)li[r] - 1u < (uint32_t)np - 1u);  // 0 < id < np
     bz[r] = __ballot(in && li[r] == 0);
   }
 }
@@ -355,6 +381,14 @@ struct Beam<NR, false> {
       }
     return v;
   }
+  // id of slot sl (uniform)
+  __device__ __forceinline__ int peek(int sl) const {
+    int v = 0;
+#pragma unroll
+    for (int r = 0; r < NR; ++r)
+      if ((sl >> 6) == r) v = __builtin_amdgcn_readlane(i[r], sl & 63);
+    return v;
+  }
   __device__ __forceinline__ void ballots(int lane, int n, int64_t np, uint64_t (&bf)[NR],
                                           uint64_t (&bz)[NR]) const {
     flag_ballots<NR>(i, lane, n, np, bf, bz);
@@ -362,6 +396,41 @@ struct Beam<NR, false> {
   // slot r*64 + lane
   __device__ __forceinline__ int id_at(int r, int) const { return i[r]; }
   __device__ __forceinline__ float dist_at(int r, int) const { return d[r]; }
+  // rank merge: the slots go through the wave's merge buffer into new
+  // registers, so a merge that is given up has changed nothing
+  __device__ __forceinline__ void load(int, int, float (&od)[NR], int (&oi)[NR]) const {
+#pragma unroll
+    for (int r = 0; r < NR; ++r) {
+      od[r] = d[r];
+      oi[r] = i[r];
+    }
+  }
+  __device__ __forceinline__ void put(const WaveLds& s, int s0, int slot, float v, int id) const {
+    s.mbuf[s0 + slot] = make_int2(__float_as_int(v), id);
+  }
+  __device__ __forceinline__ void hole(const WaveLds& s, int s0, int slot) const {
+    s.mbuf[s0 + slot].x = __float_as_int(-1.0f);  // below every distance
+  }
+  __device__ __forceinline__ void get(const WaveLds& s, int s0, int slot, float& v,
+                                      int& id) const {
+    const int2 x = s.mbuf[s0 + slot];
+    v = __int_as_float(x.x);
+    id = x.y;
+  }
+  __device__ __forceinline__ float dist_in(const WaveLds& s, int s0, int slot) const {
+    return __int_as_float(s.mbuf[s0 + slot].x);
+  }
+  __device__ __forceinline__ void undo(int, int, const float (&)[NR], const int (&)[NR]) const {}
+  __device__ __forceinline__ void take_merged(int n, int lane, const float (&nd)[NR],
+                                              const int (&ni)[NR]) {
+#pragma unroll
+    for (int r = 0; r < NR; ++r) {
+      if (r * 64 >= n) continue;
+      const bool in = lane < n - r * 64;  // lanes past the beam stay kMaxD
+      d[r] = in ? nd[r] : d[r];
+      i[r] = in ? ni[r] : i[r];
+    }
+  }
 };
 
 template <int NR>
@@ -385,6 +454,9 @@ struct Beam<NR, true> {
     wave_sync();
     return v;
   }
+  __device__ __forceinline__ int peek(int sl) const {
+    return __builtin_amdgcn_readfirstlane(qi[sl]);
+  }
   __device__ __forceinline__ void ballots(int lane, int n, int64_t np, uint64_t (&bf)[NR],
                                           uint64_t (&bz)[NR]) const {
     int x[NR];
@@ -402,6 +474,35 @@ struct Beam<NR, true> {
       i[r] = in ? qi[r * 64 + lane] : 0;
     }
   }
+  // rank merge: in place (the old slots are in the caller's registers)
+  __device__ __forceinline__ void put(const WaveLds&, int s0, int slot, float v, int id) const {
+    qd[s0 + slot] = v;
+    qi[s0 + slot] = id;
+  }
+  __device__ __forceinline__ void hole(const WaveLds&, int s0, int slot) const {
+    qd[s0 + slot] = -1.0f;
+  }
+  __device__ __forceinline__ void get(const WaveLds&, int s0, int slot, float& v, int& id) const {
+    v = qd[s0 + slot];
+    id = qi[s0 + slot];
+  }
+  __device__ __forceinline__ float dist_in(const WaveLds&, int s0, int slot) const {
+    return qd[s0 + slot];
+  }
+  __device__ __forceinline__ void undo(int n, int lane, const float (&d)[NR],
+                                       const int (&i)[NR]) {
+    store(n, lane, d, i);
+  }
+  __device__ __forceinline__ void take_merged(int n, int lane, const float (&nd)[NR],
+                                              const int (&ni)[NR]) {
+#pragma unroll
+    for (int r = 0; r < NR; ++r) {
+      if (lane >= n - r * 64) continue;
+      qd[r * 64 + lane] = nd[r];
+      qi[r * 64 + lane] = ni[r];
+    }
+    wave_sync();
+  }
   __device__ __forceinline__ void store(int n, int lane, const float (&d)[NR],
                                         const int (&i)[NR]) {
 #pragma unroll
@@ -418,6 +519,16 @@ struct Beam<NR, true> {
 template <int CTRL>
 __device__ __forceinline__ float dpp_f(float v) {
   return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), CTRL, 0xF, 0xF, true));
+}
+
+// v of the lane below / above; `end` in lane 0 / 63 (DPP wave_shr / wave_shl)
+__device__ __forceinline__ float prev_lane(float v, float end) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(end), __float_as_int(v), 0x138,
+                                                    0xF, 0xF, false));
+}
+__device__ __forceinline__ float next_lane(float v, float end) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(end), __float_as_int(v), 0x130,
+                                                    0xF, 0xF, false));
 }
 
 // One level of the lane-pair sum at distance O inside each 32-lane
@@ -476,9 +587,13 @@ __device__ __forceinline__ float treduce(const float (&v)[CNT], int lane) {
   }
 }
 
+// entering elements up to which a rank merge is the shorter path (a multiple
+// of four)
+constexpr int kRankMax = 24;
+
 constexpr int ilog2c(int x) { return x <= 1 ? 0 : 1 + ilog2c(x / 2); }
 
-template <bool TUNED, int NR, int MR, int J, int WPQ>
+template <bool TUNED, int NR, int MR, int J, int WPQ, bool FAST>
 struct SearchCore {
   // points per half-wave in one load group: all 16 when the vectors fit in
   // 64 VGPRs, so one iteration's gathers are issued together; with WPQ
@@ -517,11 +632,25 @@ struct SearchCore {
   // past d reads its row's first dim instead (in bounds) and takes 0, with
   // no branch.  J = 2 and 8 also serve smaller d (1..32, 129..224): every
   // dim group is masked there.
+  //
+  // FAST (d == 32 * J, every row offset below 2^32 bytes, ids below 2^24): a
+  // row's byte offset is one full-rate 24-bit multiply-add into one VGPR,
+  // added to the scalar base by the load itself, and no dim is masked.  The
+  // 64-bit form needs a quarter-rate multiply-add and two VGPRs per point,
+  // and an addition for the last dim group.
   static __device__ __forceinline__ void group_rows(const SearchArgs& a, const int (&ids)[PB],
                                                     int l32, float (&v)[PB][J]) {
     const char* bp = reinterpret_cast<const char*>(a.base) + 4 * l32;
     const uint32_t rowb = (uint32_t)a.stride * 4u;
-    if constexpr (J == 2 || J == 8) {
+    if constexpr (FAST) {
+#pragma unroll
+      for (int pb = 0; pb < PB; ++pb) {
+        const uint32_t off = __umul24((uint32_t)ids[pb], rowb) + 4u * (uint32_t)l32;
+        const char* row = reinterpret_cast<const char*>(a.base) + off;
+#pragma unroll
+        for (int j = 0; j < J; ++j) v[pb][j] = *reinterpret_cast<const float*>(row + 128 * j);
+      }
+    } else if constexpr (J == 2 || J == 8) {
 #pragma unroll
       for (int pb = 0; pb < PB; ++pb) {
         const float* row = reinterpret_cast<const float*>(
@@ -560,7 +689,7 @@ struct SearchCore {
 #pragma unroll
     for (int r = 0; r < MR; ++r) {
       const int slot = r * 64 + lane;
-      const bool valid = slot < m && bi[r] >= 0 && (int64_t)bi[r] < a.np;
+      const bool valid = slot < m && (uint32_t)bi[r] < (uint32_t)a.np;  // 0 <= id < np
       const uint64_t bal = __ballot(valid);
       const int ci = total + (int)__builtin_amdgcn_mbcnt_hi(
                                  (uint32_t)(bal >> 32),
@@ -609,34 +738,138 @@ struct SearchCore {
     return total;
   }
 
-  // True when no batch element can enter the beam, so the step below would
-  // leave L as it is.  The half-cleaner cascade that produced L leaves every
-  // comparator relation of all its stages true (its first stage puts each
-  // lower element at or below its partner, and comparator networks keep
-  // element-wise order, so the recursion keeps it), hence a second pass
-  // swaps nothing and L[n-1] is the beam's largest key.  Every element of
-  // B not below L[n-1] therefore loses its min-exchange, and with no swap the
-  // merge is that second pass.  Distances are non-negative floats, so their
-  // bit patterns order as unsigned integers.
-  static __device__ __forceinline__ bool batch_cannot_enter(float last, const float (&bd)[MR],
-                                                            int lane) {
-    int mn = -1;  // 0xffffffff: no valid element
+  // Merge by ranks, for a batch of which few elements enter the beam.  The
+  // exchange and cascade below leave the n smallest of L and B in ascending
+  // order; when no two of the keys concerned are equal that order is unique,
+  // so any way of merging gives the networks' result.  The entering elements
+  // (masks em, cnt of them) go to LDS; every beam slot counts those below it,
+  // which is how far it moves up, and every entering element its rank among
+  // them.  The beam slots, moved, leave holes, which the elements fill in
+  // their order.  Returns false, with L as it was, when the result may depend
+  // on the networks' own order: equal keys among the entering elements, or one
+  // equal to a beam key (the smallest dropped key, slot n, included), or a
+  // NaN in the batch.  L itself has no equal keys but empty slots (kMaxD) while
+  // `plain` holds; those differ at most in the sign of the padding id, which
+  // nothing reads.
+  //
+  // Bound by instruction issue: 2 VALU instructions per entering element and
+  // register of L and B, against the full sort of B and merge of L whatever
+  // enters.  Elements that enter per step, measured on the CPU over mixtures
+  // of integer and of normalised vectors: 5 at beam 64, 8 at beam 256 (median
+  // 3 to 5; none in 6 to 40% of the steps).  At beam 256 a launch issues 472M
+  // VALU instructions without this path and 390M with it.
+  template <class BeamT>
+  static __device__ __forceinline__ bool rank_merge(const WaveLds& s, int lane, BeamT& L,
+                                                    const float (&bd)[MR], const int (&bi)[MR],
+                                                    const uint64_t (&em)[MR], int cnt, int n) {
+    uint64_t odd = 0;  // lanes that rule this path out
+#pragma unroll
+    for (int r = 0; r < MR; ++r) odd |= __builtin_amdgcn_ballot_w64(bd[r] != bd[r]);
+    if (odd) return false;
+    float ld[NR];
+    int li[NR];
+    L.load(n, lane, ld, li);
+    int ci[MR], up[NR], rk[MR];
+    int base = 0;
 #pragma unroll
     for (int r = 0; r < MR; ++r) {
-      const uint32_t u = bd[r] != kMaxD ? __float_as_uint(bd[r]) : 0xffffffffu;
-      mn = (int)min((uint32_t)mn, u);
+      ci[r] = base + (int)__builtin_amdgcn_mbcnt_hi(
+                         (uint32_t)(em[r] >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)em[r], 0u));
+      if (__builtin_amdgcn_inverse_ballot_w64(em[r])) s.ed[ci[r]] = bd[r];
+      base += __popcll(em[r]);
     }
-    mn = (int)min((uint32_t)mn, (uint32_t)xor_lane<1>(mn, lane));
-    mn = (int)min((uint32_t)mn, (uint32_t)xor_lane<2>(mn, lane));
-    mn = (int)min((uint32_t)mn, (uint32_t)xor_lane<4>(mn, lane));
-    mn = (int)min((uint32_t)mn, (uint32_t)xor_lane<8>(mn, lane));
-    mn = (int)min((uint32_t)mn, (uint32_t)xor_lane<16>(mn, lane));
-    mn = (int)min((uint32_t)mn, (uint32_t)xor_lane<32>(mn, lane));
-    const uint32_t bmin = (uint32_t)__builtin_amdgcn_readfirstlane(mn);
-    if (bmin == 0xffffffffu) return true;
-    // REF swaps on a strictly larger distance; TUNED also on an equal
-    // distance with a larger id, so only a strictly smaller L[n-1] is safe
-    return TUNED ? last < __uint_as_float(bmin) : last <= __uint_as_float(bmin);
+    if (lane < 4) s.ed[cnt + lane] = __builtin_inff();  // the last group of four
+#pragma unroll
+    for (int r = 0; r < NR; ++r) {
+      up[r] = 0;
+      if (r * 64 < n) L.hole(s, r * 64, lane);
+    }
+    if (lane == 0) L.hole(s, n, 0);
+#pragma unroll
+    for (int r = 0; r < MR; ++r) rk[r] = 0;
+    wave_sync();
+    for (int j = 0; j < cnt; j += 4) {
+      const float4 c4 = *reinterpret_cast<const float4*>(s.ed + j);
+      const float c[4] = {c4.x, c4.y, c4.z, c4.w};
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        // registers past the beam hold kMaxD or nothing that is used
+#pragma unroll
+        for (int r = 0; r < NR; ++r) up[r] += c[t] < ld[r] ? 1 : 0;
+#pragma unroll
+        for (int r = 0; r < MR; ++r) rk[r] += c[t] < bd[r] ? 1 : 0;
+      }
+    }
+#pragma unroll
+    for (int r = 0; r < NR; ++r)
+      if (r * 64 < n && up[r] + lane <= n - r * 64)
+        L.put(s, r * 64, up[r] + lane, ld[r], li[r]);
+#pragma unroll
+    for (int r = 0; r < MR; ++r)
+      if (__builtin_amdgcn_inverse_ballot_w64(em[r])) {
+        s.es[rk[r]] = make_int2(__float_as_int(bd[r]), bi[r]);
+        s.eo[rk[r]] = ci[r];
+      }
+    wave_sync();
+    // equal entering elements share a rank: one of them does not find itself
+#pragma unroll
+    for (int r = 0; r < MR; ++r) {
+      const bool in = __builtin_amdgcn_inverse_ballot_w64(em[r]);
+      const int o = in ? s.eo[rk[r]] : 0;
+      odd |= __builtin_amdgcn_ballot_w64(in && o != ci[r]);
+    }
+    int holes = 0;
+    float nd[NR], top = -1.0f;  // top: slot r*64 - 1
+    int ni[NR];
+#pragma unroll
+    for (int r = 0; r < NR; ++r) {
+      if (r * 64 >= n) continue;
+      float f;
+      int fi;
+      L.get(s, r * 64, lane, f, fi);
+      const bool hole = lane < n - r * 64 && f < 0.0f;
+      const uint64_t hm = __builtin_amdgcn_ballot_w64(hole);
+      const int k = holes + (int)__builtin_amdgcn_mbcnt_hi(
+                                (uint32_t)(hm >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)hm, 0u));
+      holes += __popcll(hm);
+      // read by every lane (k <= cnt is inside the buffers), used by the holes
+      const int2 x = s.es[k];
+      nd[r] = hole ? __int_as_float(x.x) : f;
+      ni[r] = hole ? x.y : fi;
+      // a beam key equal to the element in a hole is in the slot below it
+      const float below = prev_lane(f, top);
+      odd |= __builtin_amdgcn_ballot_w64(hole && below == nd[r]);
+      top = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(f), 63));
+    }
+    // slot n, the first that drops out
+    if (L.dist_in(s, n, 0) < 0.0f)
+      odd |= __builtin_amdgcn_ballot_w64(L.dist_in(s, n - 1, 0) == __int_as_float(s.es[holes].x));
+    wave_sync();  // the slots are read before anything is written over them
+    if (odd) {
+      L.undo(n, lane, ld, li);
+      return false;
+    }
+    L.take_merged(n, lane, nd, ni);
+    return true;
+  }
+
+  // No two beam keys are equal, empty slots apart (after a network step).
+  template <class BeamT>
+  static __device__ __forceinline__ bool distinct(int lane, const BeamT& L, int n) {
+    float ld[NR];
+    int li[NR];
+    L.load(n, lane, ld, li);
+    uint64_t same = 0;
+#pragma unroll
+    for (int r = 0; r < NR; ++r) {
+      if (r * 64 >= n) continue;
+      const float top = r + 1 < NR ? __int_as_float(__builtin_amdgcn_readfirstlane(
+                                         __float_as_int(ld[r + 1 < NR ? r + 1 : r])))
+                                   : kMaxD;
+      same |= __builtin_amdgcn_ballot_w64(lane < n - 1 - r * 64 && ld[r] != kMaxD &&
+                                          next_lane(ld[r], top) == ld[r]);
+    }
+    return same == 0;
   }
 
   // min-exchange of L's last c = min(n, m) slots with the sorted batch's
@@ -665,12 +898,48 @@ struct SearchCore {
     merge_asc<TUNED, NR>(ld, li, n, lane);
   }
 
-  // sort B descending, min-exchange into L, merge L ascending
+  // B into L: nothing when no element can enter, a rank merge when few do,
+  // else sort B descending, min-exchange into L, merge L ascending.
+  //
+  // The step leaves L as it is when no element enters: the half-cleaner
+  // cascade that produced L leaves every comparator relation of all its
+  // stages true (its first stage puts each lower element at or below its
+  // partner, and comparator networks keep element-wise order, so the
+  // recursion keeps it), hence a second pass swaps nothing and L[n-1] is the
+  // beam's largest key.  Every element of B not below L[n-1] therefore loses
+  // its min-exchange, and with no swap the merge is that second pass.  REF
+  // swaps on a strictly larger distance; TUNED also on an equal distance with
+  // a larger id, so there an element equal to L[n-1] may enter and goes to
+  // the networks (as does a point at distance kMaxD while seeding).
+  //
+  // `plain` is per query: false once a merge met equal keys or a NaN, after
+  // which the networks take every step (L may hold the tie, or be unsorted).
   template <class BeamT>
   static __device__ __forceinline__ void merge_batch(const WaveLds& s, int lane, BeamT& L,
                                                      float (&bd)[MR], int (&bi)[MR], int n, int m,
-                                                     bool skip_max) {
-    if (batch_cannot_enter(L.last(n), bd, lane)) return;
+                                                     int32_t npi, bool skip_max, bool& plain) {
+    const float last = L.last(n);
+    uint64_t em[MR], any = 0;
+    int cnt = 0;
+    bool ranks = plain;
+#pragma unroll
+    for (int r = 0; r < MR; ++r) {
+      em[r] = __builtin_amdgcn_ballot_w64(bd[r] < last);
+      cnt += __popcll(em[r]);
+      if constexpr (TUNED) {
+        const uint64_t le = __builtin_amdgcn_ballot_w64(bd[r] <= last && bd[r] != kMaxD);
+        any |= le;
+        if (le != em[r]) ranks = false;
+        if (!skip_max && __builtin_amdgcn_ballot_w64(bd[r] == kMaxD && bi[r] != npi)) ranks = false;
+      } else {
+        any |= em[r];
+      }
+    }
+    if (!any) return;
+    if (ranks && cnt <= kRankMax) {
+      if (rank_merge(s, lane, L, bd, bi, em, cnt, n)) return;
+      plain = false;
+    }
     sort_desc<TUNED, MR>(bd, bi, m, lane);
 #pragma unroll
     for (int r = 0; r < MR; ++r) {
@@ -687,6 +956,7 @@ struct SearchCore {
     } else {
       exchange_merge(s, lane, L.d, L.i, n, m, skip_max);
     }
+    if (plain) plain = distinct(lane, L, n);
   }
 };
 
@@ -803,11 +1073,24 @@ __device__ __forceinline__ float* dist_buf_t(const WaveLds& s, uint32_t* qshared
 __host__ __device__ constexpr int filter_words(int w) { return (w + 3) & ~3; }
 
 // LDS words of one wave's private region past the filter: compacted ids,
-// sorted batch (ids, dists), for one wave per query the distances, and for
-// a beam held in LDS its queue of 64*NR (distance, id) slots
+// sorted batch (ids, dists), for one wave per query the distances -- the
+// buffers of a rank merge (kRankWords, and 64*NR + 1 pairs for a beam in VGPRs)
+// lie over them -- and for a beam held in LDS its queue of 64*NR (distance, id)
+// slots and one more, each array in whole 16 bytes
+constexpr int kRankWords = (kRankMax + 4) + kRankMax + 2 * kRankMax;
+template <int NR>
+__host__ __device__ constexpr int queue_words() {
+  return 64 * NR + 4;
+}
+template <int MR, int WPQ, int NR, bool LQ>
+__host__ __device__ constexpr int batch_words() {
+  constexpr int batch = (WPQ > 1 ? 3 : 4) * 64 * MR;
+  constexpr int merge = kRankWords + (LQ ? 0 : 2 * 64 * NR + 4);
+  return batch > merge ? batch : merge;
+}
 template <int MR, int WPQ, int NR, bool LQ>
 __host__ __device__ constexpr int lds_words_wave() {
-  return (WPQ > 1 ? 3 : 4) * 64 * MR + (LQ ? 2 * 64 * NR : 0);
+  return batch_words<MR, WPQ, NR, LQ>() + (LQ ? 2 * queue_words<NR>() : 0);
 }
 // LDS words a query shares between its waves (WPQ > 1): two distance
 // buffers (alternating batches) and the broadcast slot of the work queue
@@ -816,12 +1099,23 @@ __host__ __device__ constexpr int lds_words_query() {
   return WPQ > 1 ? 2 * 64 * MR + 4 : 0;
 }
 
-template <bool TUNED, int NR, int MR, int J, int WPQ, bool LQ>
-__global__ __launch_bounds__(256) void search_kernel(SearchArgs a) {
-  using Core = SearchCore<TUNED, NR, MR, J, WPQ>;
+// Waves per SIMD asked of the compiler: four of the FAST kernels with up to
+// 256 beam slots and 128 dims, which need just over the 128 VGPRs of four
+// waves when left alone (131 at beam 256, d = 128) and then run three.  At
+// 128 only values used once per query go to scratch.
+template <int NR, int J, bool FAST>
+constexpr int min_waves() {
+  return FAST && NR <= 4 && J <= 4 ? 4 : 1;
+}
+
+template <bool TUNED, int NR, int MR, int J, int WPQ, bool LQ, bool FAST>
+__global__ __launch_bounds__(256, (min_waves<NR, J, FAST>())) void search_kernel(SearchArgs a) {
+  using Core = SearchCore<TUNED, NR, MR, J, WPQ, FAST>;
   extern __shared__ uint32_t smem[];
   const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
+  // one value per wave: as a scalar it keeps the query's slot, its addresses
+  // and its LDS region out of VGPRs
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int sub = wave % WPQ;  // this wave's share of the query's distances
   const int fwords = filter_words(a.bloom_words_max);
   const int region = fwords + lds_words_wave<MR, WPQ, NR, LQ>();
@@ -832,7 +1126,8 @@ __global__ __launch_bounds__(256) void search_kernel(SearchArgs a) {
   int parity = 0;  // alternates the shared distance buffers
   const int shift = a.shift;
   const int D = 1 << shift;
-  const int W = a.width;
+  constexpr int KW = FAST ? 1 : kMaxWidth;  // rows expanded per iteration
+  const int W = FAST ? 1 : a.width;
   const int m = W << shift;
   const int64_t np = a.np;
   const int32_t npi = (int32_t)np;
@@ -867,9 +1162,12 @@ __global__ __launch_bounds__(256) void search_kernel(SearchArgs a) {
     s.sbd = (float*)(s.cid + 64 * MR);
     s.sbi = (int*)(s.sbd + 64 * MR);
     s.cdist = WPQ > 1 ? nullptr : (float*)(s.sbi + 64 * MR);
-    s.qd = LQ ? (float*)(base_lds + fwords + lds_words_wave<MR, WPQ, 0, false>())
-              : nullptr;
-    s.qi = LQ ? (int*)(s.qd + 64 * NR) : nullptr;
+    s.ed = (float*)(base_lds + fwords);
+    s.eo = (int*)(s.ed + kRankMax + 4);
+    s.es = (int2*)(s.eo + kRankMax);
+    s.mbuf = LQ ? nullptr : s.es + kRankMax;
+    s.qd = LQ ? (float*)(base_lds + fwords + batch_words<MR, WPQ, NR, LQ>()) : nullptr;
+    s.qi = LQ ? (int*)(s.qd + queue_words<NR>()) : nullptr;
     // the hash count is fixed per mode (kHashes), checked on the host
     Bloom<kHashes<TUNED>> bl{s.bloom, (uint32_t)bwords, (uint32_t)(31 - __clz(bwords)),
                              (uint32_t)bwords * 32u};
@@ -900,6 +1198,8 @@ __global__ __launch_bounds__(256) void search_kernel(SearchArgs a) {
     const int32_t* prow = a.pids + (int64_t)hit * a.cap;
     uint32_t seed = (uint32_t)(q * 64 + lane);  // :66
     int nE = 0, nX = 0;
+    bool plain = true;  // no equal keys met yet (merge_batch)
+    int vpre = -1, gpre = npi;  // FAST: node whose graph row gpre holds or awaits
 
     // ---- entry seeding, :479-959
     const int nch = (n + m - 1) / m;
@@ -923,7 +1223,7 @@ __global__ __launch_bounds__(256) void search_kernel(SearchArgs a) {
       }
       wave_sync();
       nE += Core::batch_dists(a, s, dist_buf(s, qshared, parity), qv, lane, sub, bi, bd, m);
-      Core::merge_batch(s, lane, L, bd, bi, n, m, false);
+      Core::merge_batch(s, lane, L, bd, bi, n, m, npi, false, plain);
     }
 
     // ---- main loop, :964-1532
@@ -938,15 +1238,15 @@ __global__ __launch_bounds__(256) void search_kernel(SearchArgs a) {
       for (int r = 0; r < MR; ++r) bi[r] = npi;
       // pick up to W slots (:985-1031)
       int cnt = 0;
-      int vrow[kMaxWidth];
+      int vrow[KW];
 #pragma unroll
-      for (int x = 0; x < kMaxWidth; ++x) vrow[x] = 0;
+      for (int x = 0; x < KW; ++x) vrow[x] = 0;
       while (cnt < W && mask != 0u) {
         const int b = __builtin_ctz(mask);
         const int sl = chunk * 32 + b;
         const int v = L.take(sl, lane);
 #pragma unroll
-        for (int x = 0; x < kMaxWidth; ++x)
+        for (int x = 0; x < KW; ++x)
           if (x == cnt) vrow[x] = v < 0 ? -v : v;
         mask &= ~(1u << b);
         ++cnt;
@@ -959,23 +1259,35 @@ __global__ __launch_bounds__(256) void search_kernel(SearchArgs a) {
         }
       }
       if (cnt == 0) break;
-      // graph rows into B (rows past np are not read, P4)
+      if constexpr (FAST) {
+        // the row of this iteration is on its way since the last one if the
+        // slot expected then is the one taken now
+        const int v0 = vrow[0];
+        if (v0 == vpre) {
+          bi[0] = lane < m ? gpre : npi;
+        } else if (lane < m) {
+          bi[0] = (uint32_t)v0 < (uint32_t)np
+                      ? a.graph[((uint64_t)(uint32_t)v0 << shift) + lane] : npi;
+        }
+      } else {
+        // graph rows into B (rows past np are not read, P4)
 #pragma unroll
-      for (int r = 0; r < MR; ++r) {
-        const int i = r * 64 + lane;
-        const int w = i >> shift;
-        if (i < m && w < cnt) {
-          int vv = 0;
+        for (int r = 0; r < MR; ++r) {
+          const int i = r * 64 + lane;
+          const int w = i >> shift;
+          if (i < m && w < cnt) {
+            int vv = 0;
 #pragma unroll
-          for (int x = 0; x < kMaxWidth; ++x)
-            if (x == w) vv = vrow[x];
-          bi[r] = (int64_t)vv < np ? a.graph[((int64_t)vv << shift) + (i & (D - 1))] : npi;
+            for (int x = 0; x < KW; ++x)
+              if (x == w) vv = vrow[x];
+            bi[r] = (int64_t)vv < np ? a.graph[((int64_t)vv << shift) + (i & (D - 1))] : npi;
+          }
         }
       }
       // filter test per row against the filter as it was before that row's
       // own adds (P3), then the adds
 #pragma unroll
-      for (int w = 0; w < kMaxWidth; ++w) {
+      for (int w = 0; w < KW; ++w) {
         if (w >= cnt) break;
         nX += (int64_t)vrow[w] < np ? 1 : 0;
         uint32_t pos[MR][kHashes<TUNED>];
@@ -983,7 +1295,7 @@ __global__ __launch_bounds__(256) void search_kernel(SearchArgs a) {
 #pragma unroll
         for (int r = 0; r < MR; ++r) {
           const int i = r * 64 + lane;
-          const bool mine = i < m && (i >> shift) == w;
+          const bool mine = i < m && (FAST || (i >> shift) == w);
           const int t = bi[r];
           bl.positions((uint32_t)t, pos[r]);
           const bool seen = bl.test_pos(pos[r]);
@@ -993,15 +1305,28 @@ __global__ __launch_bounds__(256) void search_kernel(SearchArgs a) {
 #pragma unroll
         for (int r = 0; r < MR; ++r) {
           const int i = r * 64 + lane;
-          const bool mine = i < m && (i >> shift) == w;
+          const bool mine = i < m && (FAST || (i >> shift) == w);
           bl.add_pos(pos[r], pass[r]);
           bi[r] = (mine && !pass[r]) ? npi : bi[r];
         }
         wave_sync();
       }
+      if constexpr (FAST) {
+        // The row expected next is requested just before this iteration's
+        // gathers and travels with them.  (Requested with this iteration's own
+        // row, it would be waited for together with that.)
+        vpre = -1;
+        if (mask != 0u) {
+          vpre = L.peek(chunk * 32 + __builtin_ctz(mask));
+          vpre = vpre < 0 ? -vpre : vpre;
+          if (lane < m)
+            gpre = (uint32_t)vpre < (uint32_t)np
+                       ? a.graph[((uint64_t)(uint32_t)vpre << shift) + lane] : npi;
+        }
+      }
       nE += Core::batch_dists(a, s, dist_buf(s, qshared, parity), qv, lane, sub, bi, bd,
                               cnt << shift);
-      Core::merge_batch(s, lane, L, bd, bi, n, m, true);
+      Core::merge_batch(s, lane, L, bd, bi, n, m, npi, true, plain);
       // rescan (:1495-1516)
       {
         uint64_t bf[NR], bz[NR];
@@ -1055,16 +1380,29 @@ size_t search_lds_bytes(int bloom_words_max, int wpb) {
           lds_words_query<MR, WPQ>()) * 4;
 }
 
-template <bool TUNED, int NR, int MR, int J, int WPQ, bool LQ>
-hipError_t launch_t(const SearchArgs& a, int grid, int wpb, hipStream_t st, int* occ) {
+template <bool TUNED, int NR, int MR, int J, int WPQ, bool LQ, bool FAST>
+hipError_t launch_f(const SearchArgs& a, int grid, int wpb, hipStream_t st, int* occ) {
   const size_t lds = search_lds_bytes<MR, WPQ, NR, LQ>(a.bloom_words_max, wpb);
   if (occ) {  // resident workgroups per CU for this shape
     return hipOccupancyMaxActiveBlocksPerMultiprocessor(
-        occ, search_kernel<TUNED, NR, MR, J, WPQ, LQ>, 64 * wpb, lds);
+        occ, search_kernel<TUNED, NR, MR, J, WPQ, LQ, FAST>, 64 * wpb, lds);
   }
-  hipLaunchKernelGGL((search_kernel<TUNED, NR, MR, J, WPQ, LQ>), dim3(grid), dim3(64 * wpb), lds,
-                     st, a);
+  hipLaunchKernelGGL((search_kernel<TUNED, NR, MR, J, WPQ, LQ, FAST>), dim3(grid), dim3(64 * wpb),
+                     lds, st, a);
   return hipGetLastError();
+}
+
+// The FAST kernels: one row per iteration, whole 32-dim groups, 32-bit row
+// offsets from 24-bit ids.  The rest (wider search, other dims, bases of 4
+// GiB or 16.7M rows and more, several waves per query) takes the general form.
+template <bool TUNED, int NR, int MR, int J, int WPQ, bool LQ>
+hipError_t launch_t(const SearchArgs& a, int grid, int wpb, hipStream_t st, int* occ) {
+  if constexpr (MR == 1 && WPQ == 1) {
+    if (a.width == 1 && a.d == 32 * J && a.np < (1 << 24) &&
+        (uint64_t)a.np * (uint64_t)a.stride <= (1ull << 30))
+      return launch_f<TUNED, NR, MR, J, WPQ, LQ, true>(a, grid, wpb, st, occ);
+  }
+  return launch_f<TUNED, NR, MR, J, WPQ, LQ, false>(a, grid, wpb, st, occ);
 }
 
 template <int NR, int MR, int WPQ, bool LQ>
