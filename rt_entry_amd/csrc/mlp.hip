@@ -48,136 +48,233 @@ __device__ __forceinline__ floatx4 mfma_k32(uint4 a, uint4 b, floatx4 c) {
 
 enum Epi { EPI_RELU = 0, EPI_LINEAR = 1, EPI_RELU_BWD = 2, EPI_STORE = 3 };
 
-// 64 x 32 (rows x k) tile of a bf16 matrix whose element (row, k) sits at
-// P[row * srow + k * sk], for LDS T[64][40] ([row][k], rows 80 bytes apart so
-// every 16-byte MFMA operand read is aligned).  KC: k is the contiguous
-// dimension (sk == 1); thread t takes the 8 k values 8 * (t & 3) + 0..7 of
-// row t >> 2 as one 16-byte load.  Otherwise rows are contiguous (srow ==
-// 1); thread t takes rows 8 * (t & 7) + 0..7 of k value t >> 3 as one
-// 16-byte load and spreads them over 8 LDS rows.  Runs that cross the
-// matrix edge, or strides that break 16-byte alignment (vec false), are
-// loaded element by element with zeros outside.
-template <bool KC>
-__device__ __forceinline__ uint4 tile_load(const uint16_t* __restrict__ P, int64_t srow,
-                                           int64_t sk, int R, int K, int r0, int k0, int t,
-                                           bool vec) {
-  const int r = KC ? r0 + (t >> 2) : r0 + 8 * (t & 7);
-  const int k = KC ? k0 + 8 * (t & 3) : k0 + (t >> 3);
-  const bool full = KC ? (r < R && k + 8 <= K) : (r + 8 <= R && k < K);
+// ---- training GEMMs ----
+// A stage of the training GEMMs: T x kStageK (rows x k) of a bf16 matrix whose
+// element (row, k) sits at P[row * srow + k * sk], in LDS as rows of sixteen
+// 16-byte units (8 k each), unit q of a row at q ^ stage_swz(row).  The 16 rows
+// of an MFMA operand read then lie in distinct banks, and so do the 4-byte
+// stores of four 8-row runs by 16 k pairs.
+//  KC: k is the contiguous dimension (sk == 1); a 16-byte load is 8 k values
+//  of one row and one 16-byte LDS store.
+//  Otherwise rows are contiguous (srow == 1); a thread loads 8 rows of k and
+//  of k + 1 and stores 8 pairs (k, k + 1), one 4-byte store per row.
+// Inside the matrix a stage's loads are issued together without a branch; at
+// its edges, or with strides that break 16-byte alignment (vec false), each
+// run is checked, and loaded element by element with zeros outside.
+constexpr int kStageK = 128;
+
+__device__ __forceinline__ int stage_swz(int row) { return (row & 15) ^ ((row & 16) >> 2); }
+// 16-bit word of (row, k)
+__device__ __forceinline__ int stage_at(int row, int k) {
+  return row * kStageK + ((((k >> 3) ^ stage_swz(row)) << 3) | (k & 7));
+}
+
+__device__ __forceinline__ uint4 run_load(const uint16_t* __restrict__ P, int64_t srow,
+                                          int64_t sk, int R, int K, int r, int k, bool kc,
+                                          bool vec) {
+  const bool full = kc ? (r < R && k + 8 <= K) : (r + 8 <= R && k < K);
   if (vec && full) return *reinterpret_cast<const uint4*>(P + (int64_t)r * srow + (int64_t)k * sk);
   uint16_t e[8];
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
-    const int ri = KC ? r : r + i, ki = KC ? k + i : k;
+    const int ri = kc ? r : r + i, ki = kc ? k + i : k;
     e[i] = (ri < R && ki < K) ? P[(int64_t)ri * srow + (int64_t)ki * sk] : (uint16_t)0;
   }
   uint4 v;
   memcpy(&v, e, 16);
   return v;
 }
+// this thread's i-th run of a stage: row and k
 template <bool KC>
-__device__ __forceinline__ void tile_store(uint16_t (*T)[40], int t, uint4 v) {
-  if constexpr (KC) {
-    *reinterpret_cast<uint4*>(&T[t >> 2][8 * (t & 3)]) = v;
+__device__ __forceinline__ void stage_run(int t, int i, int& r, int& k) {
+  if (KC) {
+    r = (t >> 4) + 16 * i;
+    k = 8 * (t & 15);
   } else {
-    uint16_t e[8];
-    memcpy(e, &v, 16);
+    r = 8 * ((t & 3) + 4 * (i >> 1));
+    k = 2 * (t >> 2) + (i & 1);
+  }
+}
+template <bool KC, int T>
+__device__ __forceinline__ void stage_load(const uint16_t* __restrict__ P, int64_t srow,
+                                           int64_t sk, int R, int K, int r0, int k0, int t,
+                                           bool vec, uint4 (&v)[T / 16]) {
+  if (vec && r0 + T <= R && k0 + kStageK <= K) {
 #pragma unroll
-    for (int i = 0; i < 8; ++i) T[8 * (t & 7) + i][t >> 3] = e[i];
+    for (int i = 0; i < T / 16; ++i) {
+      int r, k;
+      stage_run<KC>(t, i, r, k);
+      v[i] = *reinterpret_cast<const uint4*>(P + (int64_t)(r0 + r) * srow + (int64_t)(k0 + k) * sk);
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < T / 16; ++i) {
+      int r, k;
+      stage_run<KC>(t, i, r, k);
+      v[i] = run_load(P, srow, sk, R, K, r0 + r, k0 + k, KC, vec);
+    }
+  }
+}
+template <bool KC, int T>
+__device__ __forceinline__ void stage_store(uint16_t* S, int t, const uint4 (&v)[T / 16]) {
+#pragma unroll
+  for (int i = 0; i < T / 16; i += KC ? 1 : 2) {
+    int r, k;
+    stage_run<KC>(t, i, r, k);
+    if constexpr (KC) {
+      *reinterpret_cast<uint4*>(S + stage_at(r, k)) = v[i];
+    } else {
+      const uint32_t lo[4] = {v[i].x, v[i].y, v[i].z, v[i].w};
+      const uint32_t hi[4] = {v[i + 1].x, v[i + 1].y, v[i + 1].z, v[i + 1].w};
+#pragma unroll
+      for (int w = 0; w < 4; ++w) {
+        *reinterpret_cast<uint32_t*>(S + stage_at(r + 2 * w, k)) =
+            (lo[w] & 0xffffu) | (hi[w] << 16);
+        *reinterpret_cast<uint32_t*>(S + stage_at(r + 2 * w + 1, k)) =
+            (lo[w] >> 16) | (hi[w] & 0xffff0000u);
+      }
+    }
   }
 }
 
-// C[M x N] = op(A)[M x K] . op(B)[K x N] with bf16 operands addressed by
-// strides (element (m,k) of A at A[m*sam + k*sak], (k,n) of B at
-// B[k*sbk + n*sbn]); AK / BK: k is A's / B's contiguous dimension (else m /
-// n is).  Workgroup tile 64x64, four waves of 32x32 (2x2 tiles of
-// v_mfma_f32_16x16x32_bf16), K staged through LDS 32 at a time with 16-byte
-// loads, the next K tile's loads in flight while the current one is
-// multiplied.  Epilogues:
+// One product C[M x N] = op(A)[M x K] . op(B)[K x N] with bf16 operands
+// addressed by strides (element (m,k) of A at A[m*sam + k*sak], (k,n) of B at
+// B[k*sbk + n*sbn]).
+struct Gemm {
+  const uint16_t* A;
+  int64_t sam, sak;
+  const uint16_t* B;
+  int64_t sbk, sbn;
+  int M, N, K;
+  const float* bias;
+  const float* act;
+  float* out;
+  uint16_t* out16;
+};
+// Up to three products of one kind in one launch (workgroups in their order).
+struct GemmGroup {
+  Gemm g[3];
+  int tiles[3];  // workgroups of each product (0: none)
+};
+
+// AK / BK: k is A's / B's contiguous dimension (else m / n is).  Workgroup
+// tile T x T, four waves of T/2 x T/2 (16x16 tiles of
+// v_mfma_f32_16x16x32_bf16), K staged through LDS kStageK at a time with
+// 16-byte loads, the next stage's loads in flight while the current one is
+// multiplied.  Every output element is one accumulator over the k steps in
+// ascending order whatever T is.  Epilogues:
 //  RELU      out = relu(acc + bias[n]) (f32) and its bf16 copy
 //  LINEAR    out = acc + bias[n]
 //  RELU_BWD  out = acc * (act[m,n] > 0) (f32) and its bf16 copy
 //  STORE     out = acc
-template <int EPI, bool AK, bool BK>
-__global__ __launch_bounds__(256) void gemm_bf16(const uint16_t* __restrict__ A, int64_t sam,
-                                                 int64_t sak, const uint16_t* __restrict__ B,
-                                                 int64_t sbk, int64_t sbn, int M, int N, int K,
-                                                 const float* __restrict__ bias,
-                                                 const float* __restrict__ act,
-                                                 float* __restrict__ out,
-                                                 uint16_t* __restrict__ out16) {
-  __shared__ __attribute__((aligned(16))) uint16_t As[64][40];  // [m][k]
-  __shared__ __attribute__((aligned(16))) uint16_t Bs[64][40];  // [n][k]
+//
+// Bound by the round trips of the stages: a workgroup has little else to run
+// while a stage's loads are on their way.  Hence 128 k per stage (32 before)
+// and, where 64 x 64 tiles would leave CUs without work, 32 x 32 ones.
+template <int EPI, bool AK, bool BK, int T>
+__global__ __launch_bounds__(256) void gemm_bf16(GemmGroup grp) {
+  constexpr int S = T / 32;  // 16 x 16 tiles per wave and dimension
+  __shared__ __attribute__((aligned(16))) uint16_t As[T * kStageK];  // [m][k]
+  __shared__ __attribute__((aligned(16))) uint16_t Bs[T * kStageK];  // [n][k]
+  int p = 0, blk = blockIdx.x;
+  while (p < 2 && blk >= grp.tiles[p]) blk -= grp.tiles[p++];
+  const Gemm g = grp.g[p];
+  const int tn = (g.N + T - 1) / T;
   const int t = threadIdx.x;
   const int lane = t & 63, wave = t >> 6;
-  const int m0 = blockIdx.y * 64, n0 = blockIdx.x * 64;
-  const int wm = (wave >> 1) * 32, wn = (wave & 1) * 32;
+  const int m0 = (blk / tn) * T, n0 = (blk % tn) * T;
+  const int wm = (wave >> 1) * (T / 2), wn = (wave & 1) * (T / 2);
   // 16-byte loads need the assumed contiguous stride and 16-byte alignment
-  const bool va = ((uintptr_t)A & 15) == 0 && (AK ? sak == 1 && (sam & 7) == 0
-                                                  : sam == 1 && (sak & 7) == 0);
-  const bool vb = ((uintptr_t)B & 15) == 0 && (BK ? sbk == 1 && (sbn & 7) == 0
-                                                  : sbn == 1 && (sbk & 7) == 0);
-  floatx4 acc[2][2];
+  const bool va = ((uintptr_t)g.A & 15) == 0 && (AK ? g.sak == 1 && (g.sam & 7) == 0
+                                                    : g.sam == 1 && (g.sak & 7) == 0);
+  const bool vb = ((uintptr_t)g.B & 15) == 0 && (BK ? g.sbk == 1 && (g.sbn & 7) == 0
+                                                    : g.sbn == 1 && (g.sbk & 7) == 0);
+  floatx4 acc[S][S];
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int i = 0; i < S; ++i)
 #pragma unroll
-    for (int j = 0; j < 2; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
-  uint4 ra = tile_load<AK>(A, sam, sak, M, K, m0, 0, t, va);
-  uint4 rb = tile_load<BK>(B, sbn, sbk, N, K, n0, 0, t, vb);
-  tile_store<AK>(As, t, ra);
-  tile_store<BK>(Bs, t, rb);
-  __syncthreads();
+    for (int j = 0; j < S; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+  uint4 ra[T / 16], rb[T / 16];
+  stage_load<AK, T>(g.A, g.sam, g.sak, g.M, g.K, m0, 0, t, va, ra);
+  stage_load<BK, T>(g.B, g.sbn, g.sbk, g.N, g.K, n0, 0, t, vb, rb);
   const int r = lane & 15, kq = 8 * (lane >> 4);
-  for (int k0 = 0; k0 < K; k0 += 32) {
-    const bool more = k0 + 32 < K;
-    if (more) {
-      ra = tile_load<AK>(A, sam, sak, M, K, m0, k0 + 32, t, va);
-      rb = tile_load<BK>(B, sbn, sbk, N, K, n0, k0 + 32, t, vb);
-    }
-    uint4 a[2], b[2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i) a[i] = *reinterpret_cast<const uint4*>(&As[wm + 16 * i + r][kq]);
-#pragma unroll
-    for (int j = 0; j < 2; ++j) b[j] = *reinterpret_cast<const uint4*>(&Bs[wn + 16 * j + r][kq]);
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-      for (int j = 0; j < 2; ++j) acc[i][j] = mfma_k32(a[i], b[j], acc[i][j]);
+  for (int k0 = 0; k0 < g.K; k0 += kStageK) {
+    stage_store<AK, T>(As, t, ra);
+    stage_store<BK, T>(Bs, t, rb);
     __syncthreads();
-    if (more) {
-      tile_store<AK>(As, t, ra);
-      tile_store<BK>(Bs, t, rb);
-      __syncthreads();
+    if (k0 + kStageK < g.K) {
+      stage_load<AK, T>(g.A, g.sam, g.sak, g.M, g.K, m0, k0 + kStageK, t, va, ra);
+      stage_load<BK, T>(g.B, g.sbn, g.sbk, g.N, g.K, n0, k0 + kStageK, t, vb, rb);
     }
+#pragma unroll
+    for (int u = 0; u < kStageK / 32; ++u) {
+      if (k0 + 32 * u >= g.K) break;
+      uint4 a[S], b[S];
+#pragma unroll
+      for (int i = 0; i < S; ++i)
+        a[i] = *reinterpret_cast<const uint4*>(As + stage_at(wm + 16 * i + r, 32 * u + kq));
+#pragma unroll
+      for (int j = 0; j < S; ++j)
+        b[j] = *reinterpret_cast<const uint4*>(Bs + stage_at(wn + 16 * j + r, 32 * u + kq));
+#pragma unroll
+      for (int i = 0; i < S; ++i)
+#pragma unroll
+        for (int j = 0; j < S; ++j) acc[i][j] = mfma_k32(a[i], b[j], acc[i][j]);
+    }
+    __syncthreads();
   }
-  // D layout: lane holds D[4*(lane/16) + v][lane%16]
+  // D layout: lane holds D[4*(lane/16) + v][lane%16].  What the epilogue reads
+  // is loaded before the first store, at clamped addresses: a load between
+  // stores would wait for them all.
+  float bias[S], act[S][S][4];
+  const bool inside = m0 + T <= g.M && n0 + T <= g.N;
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int j = 0; j < S; ++j) {
+    const int n = min(n0 + wn + 16 * j + (lane & 15), g.N - 1);
+    bias[j] = EPI == EPI_RELU || EPI == EPI_LINEAR ? g.bias[n] : 0.f;
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const int n = n0 + wn + 16 * j + (lane & 15);
-      if (n >= N) continue;
+    for (int i = 0; i < S; ++i)
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
-        const int m = m0 + wm + 16 * i + 4 * (lane >> 4) + v;
-        if (m >= M) continue;
-        const int64_t o = (int64_t)m * N + n;
-        float x = acc[i][j][v];
-        if constexpr (EPI == EPI_RELU) {
-          x = fmaxf(x + bias[n], 0.f);
-          out[o] = x;
-          out16[o] = f2bf(x);
-        } else if constexpr (EPI == EPI_LINEAR) {
-          out[o] = x + bias[n];
-        } else if constexpr (EPI == EPI_RELU_BWD) {
-          x = act[o] > 0.f ? x : 0.f;
-          out[o] = x;
-          out16[o] = f2bf(x);
-        } else {
-          out[o] = x;
-        }
+        const int m = min(m0 + wm + 16 * i + 4 * (lane >> 4) + v, g.M - 1);
+        act[i][j][v] = EPI == EPI_RELU_BWD ? g.act[(int64_t)m * g.N + n] : 0.f;
       }
-    }
+  }
+#pragma unroll
+  for (int i = 0; i < S; ++i)
+#pragma unroll
+    for (int j = 0; j < S; ++j)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        float x = acc[i][j][v];
+        if constexpr (EPI == EPI_RELU) x = fmaxf(x + bias[j], 0.f);
+        if constexpr (EPI == EPI_LINEAR) x = x + bias[j];
+        if constexpr (EPI == EPI_RELU_BWD) x = act[i][j][v] > 0.f ? x : 0.f;
+        acc[i][j][v] = x;
+      }
+  auto put = [&](int i, int j, int v) {
+    const int n = n0 + wn + 16 * j + (lane & 15), m = m0 + wm + 16 * i + 4 * (lane >> 4) + v;
+    const int64_t o = (int64_t)m * g.N + n;
+    g.out[o] = acc[i][j][v];
+    if constexpr (EPI == EPI_RELU || EPI == EPI_RELU_BWD) g.out16[o] = f2bf(acc[i][j][v]);
+  };
+  if (inside) {
+#pragma unroll
+    for (int i = 0; i < S; ++i)
+#pragma unroll
+      for (int v = 0; v < 4; ++v)
+#pragma unroll
+        for (int j = 0; j < S; ++j) put(i, j, v);
+  } else {
+#pragma unroll
+    for (int i = 0; i < S; ++i)
+#pragma unroll
+      for (int v = 0; v < 4; ++v)
+#pragma unroll
+        for (int j = 0; j < S; ++j)
+          if (n0 + wn + 16 * j + (lane & 15) < g.N && m0 + wm + 16 * i + 4 * (lane >> 4) + v < g.M)
+            put(i, j, v);
+  }
 }
 
 __device__ __forceinline__ uint32_t pack2(float lo, float hi) {
@@ -817,17 +914,35 @@ __global__ void input_kernel(const float* __restrict__ x, int64_t n, int d,
 }
 
 // Row-wise softmax cross-entropy: dZ = (softmax(z) - onehot(y)) / n and the
-// per-row loss log(sum exp(z - max)) + max - z[y].
+// per-row loss log(sum exp(z - max)) + max - z[y].  Thread t holds columns t +
+// 256 i; with PER > 0 (C <= 256 * PER) its logits and exponentials stay in
+// registers, so Z is read once and each exponential taken once (three reads and
+// two exponentials otherwise).  Bound by the memory traffic (Z in, dZ and its
+// bf16 copy out): 11 us at 1024 x 4096, 18 with the general form, which is left
+// for C > 16384.
+template <int PER>
 __global__ __launch_bounds__(256) void softmax_xent_kernel(const float* __restrict__ Z, int C,
                                                            const int32_t* __restrict__ y, int n,
                                                            float* __restrict__ dZ,
                                                            uint16_t* __restrict__ dZ16,
                                                            float* __restrict__ row_loss) {
   __shared__ float red[256];
+  constexpr int P = PER > 0 ? PER : 1;
   const int row = blockIdx.x;
   const float* z = Z + (int64_t)row * C;
+  float zv[P];
   float mx = -INFINITY;
-  for (int c = threadIdx.x; c < C; c += 256) mx = fmaxf(mx, z[c]);
+  if constexpr (PER > 0) {
+#pragma unroll
+    for (int i = 0; i < P; ++i) {
+      const int c = threadIdx.x + 256 * i;
+      zv[i] = c < C ? z[c] : -INFINITY;
+    }
+#pragma unroll
+    for (int i = 0; i < P; ++i) mx = fmaxf(mx, zv[i]);
+  } else {
+    for (int c = threadIdx.x; c < C; c += 256) mx = fmaxf(mx, z[c]);
+  }
   red[threadIdx.x] = mx;
   __syncthreads();
   for (int s = 128; s > 0; s >>= 1) {
@@ -837,7 +952,16 @@ __global__ __launch_bounds__(256) void softmax_xent_kernel(const float* __restri
   mx = red[0];
   __syncthreads();
   float se = 0.f;
-  for (int c = threadIdx.x; c < C; c += 256) se += expf(z[c] - mx);
+  if constexpr (PER > 0) {
+#pragma unroll
+    for (int i = 0; i < P; ++i) {
+      const int c = threadIdx.x + 256 * i;
+      zv[i] = expf(zv[i] - mx);
+      if (c < C) se += zv[i];
+    }
+  } else {
+    for (int c = threadIdx.x; c < C; c += 256) se += expf(z[c] - mx);
+  }
   red[threadIdx.x] = se;
   __syncthreads();
   for (int s = 128; s > 0; s >>= 1) {
@@ -847,38 +971,98 @@ __global__ __launch_bounds__(256) void softmax_xent_kernel(const float* __restri
   se = red[0];
   const int lab = min(max(y[row], 0), C - 1);  // labels are clamped into [0, C)
   const float inv = 1.f / (float)n;
-  for (int c = threadIdx.x; c < C; c += 256) {
-    const float p = expf(z[c] - mx) / se;
+  auto put = [&](int c, float e) {
+    const float p = e / se;
     const float g = (p - (c == lab ? 1.f : 0.f)) * inv;
     dZ[(int64_t)row * C + c] = g;
     dZ16[(int64_t)row * C + c] = f2bf(g);
+  };
+  if constexpr (PER > 0) {
+#pragma unroll
+    for (int i = 0; i < P; ++i) {
+      const int c = threadIdx.x + 256 * i;
+      if (c < C) put(c, zv[i]);
+    }
+  } else {
+    for (int c = threadIdx.x; c < C; c += 256) put(c, expf(z[c] - mx));
   }
   if (threadIdx.x == 0) row_loss[row] = logf(se) + mx - z[lab];
 }
 
-// column sums of dZ (n x C): bias gradients
-__global__ void colsum_kernel(const float* __restrict__ dZ, int n, int C, float* __restrict__ g) {
-  const int c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= C) return;
+// Column sums of three n x C matrices in one launch (the bias gradients), 64
+// columns per workgroup.  Each column is summed by one thread over the rows
+// in ascending order, so the sums do not depend on the launch; the four waves
+// stage kSumRows rows at a time in LDS, the next rows' loads in flight while
+// the first wave adds.  Bound by that chain of additions (n of them) and the
+// stages' round trips: 12 us at n = 1024 for the three.  One thread per column
+// reading global memory itself, a round trip every few rows, took 225 us for
+// each matrix.
+struct ColSums {
+  const float* x[3];
+  float* out[3];
+  int C[3];
+};
+constexpr int kSumRows = 128;
+__global__ __launch_bounds__(256) void colsum_kernel(ColSums a, int n) {
+  __shared__ float rows[kSumRows][64];
+  constexpr int kPer = kSumRows / 4;
+  int p = 0, blk = blockIdx.x;
+  while (p < 2 && blk >= (a.C[p] + 63) / 64) blk -= (a.C[p++] + 63) / 64;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int C = a.C[p];
+  const int c = blk * 64 + lane;
+  const float* x = a.x[p] + min(c, C - 1);
+  float v[kPer];
+  auto load = [&](int r0) {  // at clamped, valid rows; the sum stops at n
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) v[i] = x[(int64_t)min(r0 + 4 * i + wave, n - 1) * C];
+  };
+  load(0);
   float s = 0.f;
-  for (int r = 0; r < n; ++r) s += dZ[(int64_t)r * C + c];
-  g[c] = s;
+  for (int r0 = 0; r0 < n; r0 += kSumRows) {
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) rows[4 * i + wave][lane] = v[i];
+    __syncthreads();
+    if (r0 + kSumRows < n) load(r0 + kSumRows);
+    if (wave == 0) {
+      const int m = min(kSumRows, n - r0);
+      if (m == kSumRows) {
+#pragma unroll 32
+        for (int r = 0; r < kSumRows; ++r) s += rows[r][lane];
+      } else {
+        for (int r = 0; r < m; ++r) s += rows[r][lane];
+      }
+    }
+    __syncthreads();
+  }
+  if (wave == 0 && c < C) a.out[p][c] = s;
 }
 
-// Adam on FP32 masters; refreshes the bf16 copy
-__global__ void adam_kernel(float* __restrict__ p, const float* __restrict__ g, float* __restrict__ m,
-                            float* __restrict__ v, uint16_t* __restrict__ p16, int64_t n, float lr,
-                            float b1, float b2, float c1, float c2) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const float gi = g[i];
-  const float mi = b1 * m[i] + (1.f - b1) * gi;
-  const float vi = b2 * v[i] + (1.f - b2) * gi * gi;
-  m[i] = mi;
-  v[i] = vi;
-  const float pi = p[i] - lr * (mi / c1) / (sqrtf(vi / c2) + 1e-8f);
-  p[i] = pi;
-  if (p16) p16[i] = f2bf(pi);
+// Adam on FP32 masters; refreshes the bf16 copies.  All six parameter arrays
+// in one launch, each starting at a workgroup of its own.
+struct AdamArgs {
+  float* p[6];
+  const float* g[6];
+  float* m[6];
+  float* v[6];
+  uint16_t* p16[6];  // or null
+  int64_t n[6];
+  int blocks[6];
+};
+__global__ __launch_bounds__(256) void adam_kernel(AdamArgs a, float lr, float b1, float b2,
+                                                   float c1, float c2) {
+  int k = 0, blk = blockIdx.x;
+  while (k < 5 && blk >= a.blocks[k]) blk -= a.blocks[k++];
+  const int64_t i = (int64_t)blk * 256 + threadIdx.x;
+  if (i >= a.n[k]) return;
+  const float gi = a.g[k][i];
+  const float mi = b1 * a.m[k][i] + (1.f - b1) * gi;
+  const float vi = b2 * a.v[k][i] + (1.f - b2) * gi * gi;
+  a.m[k][i] = mi;
+  a.v[k][i] = vi;
+  const float pi = a.p[k][i] - lr * (mi / c1) / (sqrtf(vi / c2) + 1e-8f);
+  a.p[k][i] = pi;
+  if (a.p16[k]) a.p16[k][i] = f2bf(pi);
 }
 
 // argmax leaf and softmax maximum per row; falls back to the kd-tree leaf
@@ -984,77 +1168,90 @@ hipError_t reserve_batch(Mlp* m, int n) {
   return hipSuccess;
 }
 
-dim3 gemm_grid(int M, int N) { return dim3((unsigned)((N + 63) / 64), (unsigned)((M + 63) / 64)); }
-
 // gemm_bf16 with the operand layouts picked from the strides (k contiguous
-// when its stride is 1)
+// when its stride is 1; all products of a group alike) and the tile from the
+// work: 64 x 64 where that gives every CU (256) a workgroup, else 32 x 32.
 template <int EPI>
-void launch_gemm(dim3 grid, hipStream_t st, const uint16_t* A, int64_t sam, int64_t sak,
-                 const uint16_t* B, int64_t sbk, int64_t sbn, int M, int N, int K,
-                 const float* bias, const float* act, float* out, uint16_t* out16) {
-  const bool ak = sak == 1, bk = sbk == 1;
-#define RTE_GEMM(AK, BK)                                                                    \
-  hipLaunchKernelGGL((rte::gemm_bf16<EPI, AK, BK>), grid, dim3(256), 0, st, A, sam, sak, B, \
-                     sbk, sbn, M, N, K, bias, act, out, out16)
+void launch_gemm(hipStream_t st, const rte::Gemm* g, int count) {
+  auto tiles = [&](int i, int T) { return ((g[i].M + T - 1) / T) * ((g[i].N + T - 1) / T); };
+  int n64 = 0;
+  for (int i = 0; i < count; ++i) n64 += tiles(i, 64);
+  const int T = n64 >= 256 ? 64 : 32;
+  rte::GemmGroup grp{};
+  int total = 0;
+  for (int i = 0; i < count; ++i) {
+    grp.g[i] = g[i];
+    grp.tiles[i] = tiles(i, T);
+    total += grp.tiles[i];
+  }
+  const bool ak = g[0].sak == 1, bk = g[0].sbk == 1;
+#define RTE_GEMM(AK, BK)                                                                       \
+  do {                                                                                         \
+    if (T == 64)                                                                               \
+      hipLaunchKernelGGL((rte::gemm_bf16<EPI, AK, BK, 64>), dim3(total), dim3(256), 0, st, grp); \
+    else                                                                                       \
+      hipLaunchKernelGGL((rte::gemm_bf16<EPI, AK, BK, 32>), dim3(total), dim3(256), 0, st, grp); \
+  } while (0)
   if (ak && bk) RTE_GEMM(true, true);
   else if (ak) RTE_GEMM(true, false);
   else if (bk) RTE_GEMM(false, true);
   else RTE_GEMM(false, false);
 #undef RTE_GEMM
 }
+template <int EPI>
+void launch_gemm(hipStream_t st, const rte::Gemm& g) {
+  launch_gemm<EPI>(st, &g, 1);
+}
 
 // forward of n rows already converted to bf16 in X16; logits in Z
 hipError_t forward(Mlp* m, int n, hipStream_t st) {
   const int d0 = m->dims[0], d1 = m->dims[1], d2 = m->dims[2], d3 = m->dims[3];
   // H1 = relu(X W1 + b1): A = X16 (n x d0), B = W1 (d0 x d1, row-major)
-  launch_gemm<rte::EPI_RELU>(gemm_grid(n, d1), st,
-                     m->X16.as<uint16_t>(), (int64_t)d0, (int64_t)1, m->W16[0].as<uint16_t>(),
-                     (int64_t)d1, (int64_t)1, n, d1, d0, m->b[0].as<float>(), nullptr,
-                     m->H1.as<float>(), m->H1b.as<uint16_t>());
-  launch_gemm<rte::EPI_RELU>(gemm_grid(n, d2), st,
-                     m->H1b.as<uint16_t>(), (int64_t)d1, (int64_t)1, m->W16[1].as<uint16_t>(),
-                     (int64_t)d2, (int64_t)1, n, d2, d1, m->b[1].as<float>(), nullptr,
-                     m->H2.as<float>(), m->H2b.as<uint16_t>());
-  launch_gemm<rte::EPI_LINEAR>(gemm_grid(n, d3), st,
-                     m->H2b.as<uint16_t>(), (int64_t)d2, (int64_t)1, m->W16[2].as<uint16_t>(),
-                     (int64_t)d3, (int64_t)1, n, d3, d2, m->b[2].as<float>(), nullptr,
-                     m->Z.as<float>(), nullptr);
+  launch_gemm<rte::EPI_RELU>(st, {m->X16.as<uint16_t>(), d0, 1, m->W16[0].as<uint16_t>(), d1, 1, n,
+                                  d1, d0, m->b[0].as<float>(), nullptr, m->H1.as<float>(),
+                                  m->H1b.as<uint16_t>()});
+  launch_gemm<rte::EPI_RELU>(st, {m->H1b.as<uint16_t>(), d1, 1, m->W16[1].as<uint16_t>(), d2, 1, n,
+                                  d2, d1, m->b[1].as<float>(), nullptr, m->H2.as<float>(),
+                                  m->H2b.as<uint16_t>()});
+  launch_gemm<rte::EPI_LINEAR>(st, {m->H2b.as<uint16_t>(), d2, 1, m->W16[2].as<uint16_t>(), d3, 1,
+                                    n, d3, d2, m->b[2].as<float>(), nullptr, m->Z.as<float>(),
+                                    nullptr});
   return hipGetLastError();
 }
 
 // backward after forward; gradients in gW/gb (mean cross-entropy)
 hipError_t backward(Mlp* m, const int32_t* y, int n, hipStream_t st) {
   const int d0 = m->dims[0], d1 = m->dims[1], d2 = m->dims[2], d3 = m->dims[3];
-  hipLaunchKernelGGL(rte::softmax_xent_kernel, dim3(n), dim3(256), 0, st, m->Z.as<float>(), d3, y,
-                     n, m->dZ.as<float>(), m->dZb.as<uint16_t>(), m->loss.as<float>());
-  // gW3 = H2^T dZ: (d2 x n) . (n x d3); A(m=i,k=r) = H2b[r*d2+i]
-  launch_gemm<rte::EPI_STORE>(gemm_grid(d2, d3), st,
-                     m->H2b.as<uint16_t>(), (int64_t)1, (int64_t)d2, m->dZb.as<uint16_t>(),
-                     (int64_t)d3, (int64_t)1, d2, d3, n, nullptr, nullptr, m->gW[2].as<float>(),
-                     nullptr);
-  hipLaunchKernelGGL(rte::colsum_kernel, dim3((d3 + 255) / 256), dim3(256), 0, st,
-                     m->dZ.as<float>(), n, d3, m->gb[2].as<float>());
+#define RTE_XENT(PER)                                                                           \
+  hipLaunchKernelGGL(rte::softmax_xent_kernel<PER>, dim3(n), dim3(256), 0, st, m->Z.as<float>(), \
+                     d3, y, n, m->dZ.as<float>(), m->dZb.as<uint16_t>(), m->loss.as<float>())
+  if (d3 <= 256 * 4) RTE_XENT(4);
+  else if (d3 <= 256 * 16) RTE_XENT(16);
+  else if (d3 <= 256 * 64) RTE_XENT(64);
+  else RTE_XENT(0);
+#undef RTE_XENT
   // dH2 = (dZ W3^T) * (H2 > 0): B(k=j, n=i) = W3[i*d3 + j]
-  launch_gemm<rte::EPI_RELU_BWD>(gemm_grid(n, d2), st,
-                     m->dZb.as<uint16_t>(), (int64_t)d3, (int64_t)1, m->W16[2].as<uint16_t>(),
-                     (int64_t)1, (int64_t)d3, n, d2, d3, nullptr, m->H2.as<float>(),
-                     m->dH2.as<float>(), m->dH2b.as<uint16_t>());
-  launch_gemm<rte::EPI_STORE>(gemm_grid(d1, d2), st,
-                     m->H1b.as<uint16_t>(), (int64_t)1, (int64_t)d1, m->dH2b.as<uint16_t>(),
-                     (int64_t)d2, (int64_t)1, d1, d2, n, nullptr, nullptr, m->gW[1].as<float>(),
-                     nullptr);
-  hipLaunchKernelGGL(rte::colsum_kernel, dim3((d2 + 255) / 256), dim3(256), 0, st,
-                     m->dH2.as<float>(), n, d2, m->gb[1].as<float>());
-  launch_gemm<rte::EPI_RELU_BWD>(gemm_grid(n, d1), st,
-                     m->dH2b.as<uint16_t>(), (int64_t)d2, (int64_t)1, m->W16[1].as<uint16_t>(),
-                     (int64_t)1, (int64_t)d2, n, d1, d2, nullptr, m->H1.as<float>(),
-                     m->dH1.as<float>(), m->dH1b.as<uint16_t>());
-  launch_gemm<rte::EPI_STORE>(gemm_grid(d0, d1), st,
-                     m->X16.as<uint16_t>(), (int64_t)1, (int64_t)d0, m->dH1b.as<uint16_t>(),
-                     (int64_t)d1, (int64_t)1, d0, d1, n, nullptr, nullptr, m->gW[0].as<float>(),
-                     nullptr);
-  hipLaunchKernelGGL(rte::colsum_kernel, dim3((d1 + 255) / 256), dim3(256), 0, st,
-                     m->dH1.as<float>(), n, d1, m->gb[0].as<float>());
+  launch_gemm<rte::EPI_RELU_BWD>(st, {m->dZb.as<uint16_t>(), d3, 1, m->W16[2].as<uint16_t>(), 1, d3,
+                                      n, d2, d3, nullptr, m->H2.as<float>(), m->dH2.as<float>(),
+                                      m->dH2b.as<uint16_t>()});
+  launch_gemm<rte::EPI_RELU_BWD>(st, {m->dH2b.as<uint16_t>(), d2, 1, m->W16[1].as<uint16_t>(), 1,
+                                      d2, n, d1, d2, nullptr, m->H1.as<float>(),
+                                      m->dH1.as<float>(), m->dH1b.as<uint16_t>()});
+  // the three weight gradients in one launch, e.g. gW3 = H2^T dZ:
+  // (d2 x n) . (n x d3); A(m=i,k=r) = H2b[r*d2+i]
+  const rte::Gemm gw[3] = {
+      {m->H2b.as<uint16_t>(), 1, d2, m->dZb.as<uint16_t>(), d3, 1, d2, d3, n, nullptr, nullptr,
+       m->gW[2].as<float>(), nullptr},
+      {m->H1b.as<uint16_t>(), 1, d1, m->dH2b.as<uint16_t>(), d2, 1, d1, d2, n, nullptr, nullptr,
+       m->gW[1].as<float>(), nullptr},
+      {m->X16.as<uint16_t>(), 1, d0, m->dH1b.as<uint16_t>(), d1, 1, d0, d1, n, nullptr, nullptr,
+       m->gW[0].as<float>(), nullptr}};
+  launch_gemm<rte::EPI_STORE>(st, gw, 3);
+  const rte::ColSums cs{{m->dZ.as<float>(), m->dH2.as<float>(), m->dH1.as<float>()},
+                        {m->gb[2].as<float>(), m->gb[1].as<float>(), m->gb[0].as<float>()},
+                        {d3, d2, d1}};
+  const int blocks = (d3 + 63) / 64 + (d2 + 63) / 64 + (d1 + 63) / 64;
+  hipLaunchKernelGGL(rte::colsum_kernel, dim3(blocks), dim3(256), 0, st, cs, n);
   return hipGetLastError();
 }
 
@@ -1254,15 +1451,22 @@ int rte_mlp_train_step(rte_ctx* c, const float* X, const int32_t* y, int n, floa
   m->wt_dirty = true;
   const float b2 = 0.999f;
   const float c1 = 1.f - powf(beta1, (float)m->step), c2 = 1.f - powf(b2, (float)m->step);
-  for (int l = 0; l < 3; ++l) {
-    const int64_t nw = wsize(m, l), nb = m->dims[l + 1];
-    hipLaunchKernelGGL(rte::adam_kernel, dim3((unsigned)((nw + 255) / 256)), dim3(256), 0,
-                       c->stream, m->W[l].as<float>(), m->gW[l].as<float>(), m->mW[l].as<float>(),
-                       m->vW[l].as<float>(), m->W16[l].as<uint16_t>(), nw, lr, beta1, b2, c1, c2);
-    hipLaunchKernelGGL(rte::adam_kernel, dim3((unsigned)((nb + 255) / 256)), dim3(256), 0,
-                       c->stream, m->b[l].as<float>(), m->gb[l].as<float>(), m->mb[l].as<float>(),
-                       m->vb[l].as<float>(), (uint16_t*)nullptr, nb, lr, beta1, b2, c1, c2);
+  rte::AdamArgs ad{};
+  int blocks = 0;
+  for (int k = 0; k < 6; ++k) {  // W3, W2, W1, b3, b2, b1
+    const int l = 2 - k % 3;
+    const bool w = k < 3;
+    ad.p[k] = (w ? m->W[l] : m->b[l]).as<float>();
+    ad.g[k] = (w ? m->gW[l] : m->gb[l]).as<float>();
+    ad.m[k] = (w ? m->mW[l] : m->mb[l]).as<float>();
+    ad.v[k] = (w ? m->vW[l] : m->vb[l]).as<float>();
+    ad.p16[k] = w ? m->W16[l].as<uint16_t>() : nullptr;
+    ad.n[k] = w ? wsize(m, l) : m->dims[l + 1];
+    ad.blocks[k] = (int)((ad.n[k] + 255) / 256);
+    blocks += ad.blocks[k];
   }
+  hipLaunchKernelGGL(rte::adam_kernel, dim3(blocks), dim3(256), 0, c->stream, ad, lr, beta1, b2, c1,
+                     c2);
   MCHK(c, hipGetLastError(), "adam");
   if (loss) {
     std::vector<float> rl(n);
