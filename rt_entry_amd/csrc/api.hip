@@ -330,16 +330,51 @@ int rte_knn_rows(rte_ctx* c, const float* X, int64_t np, int d, int64_t stride, 
   if (int r = stage_out(c, c->s_out, ids_out, (size_t)nrows * k, where, &di)) return r;
   if (dists_out)
     if (int r = stage_out(c, c->s_aux2, dists_out, (size_t)nrows * k, where, &dd)) return r;
-  DevBuf norms;  // freed on return (hipFree waits for the device)
-  HIPCHK(c, norms.reserve((size_t)np * sizeof(float)), "hipMalloc(norms)");
-  HIPCHK(c, rte::launch_row_norms(dx, np, d, stride, norms.as<float>(), c->stream), "norms");
   // rows in launches of 128k (short kernels)
   const int64_t step = 1 << 17;
+  DevBuf norms, xb, half, flag, lists;  // freed on return (hipFree waits for the device)
+  HIPCHK(c, norms.reserve((size_t)np * sizeof(float)), "hipMalloc(norms)");
+  const int64_t npad = rte::knn_padded(np);
+  // without room for the whole-number kernel's buffers the FP32 kernel runs
+  const bool room = xb.reserve((size_t)npad * d * sizeof(uint16_t)) == hipSuccess &&
+                    half.reserve((size_t)npad * sizeof(float)) == hipSuccess &&
+                    lists.reserve((size_t)std::min(step, nrows) * 64 * sizeof(uint64_t)) ==
+                        hipSuccess &&
+                    flag.reserve(sizeof(uint32_t)) == hipSuccess;
+  if (room) {
+    HIPCHK(c, hipMemsetAsync(flag.p, 0, sizeof(uint32_t), c->stream), "clear flag");
+  } else {
+    (void)hipGetLastError();
+    xb.release();
+    half.release();
+    lists.release();
+    flag.release();
+  }
+  HIPCHK(c, rte::launch_row_norms(dx, np, d, stride, norms.as<float>(), xb.as<uint16_t>(),
+                                  half.as<float>(), flag.as<uint32_t>(), c->stream),
+         "norms");
+  uint32_t bits = rte::kKnnNotWhole;
+  if (room) {
+    HIPCHK(c, hipMemcpyAsync(&bits, flag.p, sizeof bits, hipMemcpyDeviceToHost, c->stream),
+           "read flag");
+    HIPCHK(c, hipStreamSynchronize(c->stream), "sync norms");
+  }
+  // whole numbers up to 256 with small norms: one bf16 product in place of an
+  // FP32 one, exact either way (160k x 128, k = 64: 75.8 ms with the FP32
+  // kernel)
+  const bool whole = rte::knn_whole_numbers(bits);
   for (int64_t r0 = row0; r0 < row0 + nrows; r0 += step) {
     const int64_t n = std::min<int64_t>(step, row0 + nrows - r0);
-    HIPCHK(c, rte::launch_knn(dx, np, d, stride, norms.as<float>(), r0, n, k, di + (r0 - row0) * k,
-                              dd ? dd + (r0 - row0) * k : nullptr, c->stream),
-           "knn launch");
+    int32_t* ids = di + (r0 - row0) * k;
+    float* dists = dd ? dd + (r0 - row0) * k : nullptr;
+    if (whole)
+      HIPCHK(c, rte::launch_knn_whole(xb.as<uint16_t>(), half.as<float>(), np, d, r0, n, k,
+                                      lists.as<uint64_t>(), ids, dists, c->stream),
+             "knn launch");
+    else
+      HIPCHK(c, rte::launch_knn(dx, np, d, stride, norms.as<float>(), r0, n, k, ids, dists,
+                                c->stream),
+             "knn launch");
   }
   if (int r = finish_out(c, ids_out, di, (size_t)nrows * k, where)) return r;
   if (dists_out)

@@ -21,7 +21,21 @@ hipError_t launch_knn(const float* X, int64_t np, int d, int64_t stride, const f
 hipError_t launch_graph_from_knn(const int32_t* knn, int64_t np, int kf, int degree, int rev_rank,
                                  int32_t* graph, void* work, hipStream_t st);
 size_t graph_from_knn_work_bytes(int64_t np, int kf, int rev_rank);
+// Row norms of X and what the whole-number kernel needs: the bf16 rows
+// (knn_padded(np) x d), half = -norm / 2 (-inf past np), and in *flag (zero
+// before the call) the bits that rule it out.
+constexpr uint32_t kKnnNotWhole = 1, kKnnNegative = 2, kKnnLarge = 4, kKnnLargeSigned = 8;
+inline bool knn_whole_numbers(uint32_t flag) {
+  return !(flag & (kKnnNotWhole | kKnnLarge)) &&
+         (flag & (kKnnNegative | kKnnLargeSigned)) != (kKnnNegative | kKnnLargeSigned);
+}
+inline int64_t knn_padded(int64_t np) { return (np + 63) / 64 * 64; }
 hipError_t launch_row_norms(const float* X, int64_t np, int d, int64_t stride, float* norms,
+                            uint16_t* Xb, float* half, uint32_t* flag, hipStream_t st);
+// launch_knn for data of which knn_whole_numbers() holds; same lists.  `lists`
+// is scratch of nq x 64 keys.
+hipError_t launch_knn_whole(const uint16_t* Xb, const float* half, int64_t np, int d, int64_t row0,
+                            int64_t nq, int k, uint64_t* lists, int32_t* ids, float* dists,
                             hipStream_t st);
 
 }  // namespace rte
