@@ -124,6 +124,16 @@ class Context:
     def synchronize(self):
         self._chk(lib().rte_synchronize(self._h))
 
+    def _on_stream(self, dev):
+        """torch allocates and fills on the library's stream inside."""
+        import contextlib
+
+        import torch
+        own = self.stream
+        if own == torch.cuda.current_stream(dev).cuda_stream:
+            return contextlib.nullcontext()
+        return torch.cuda.stream(torch.cuda.ExternalStream(own, device=dev))
+
     # ---- data
     def set_base(self, base, d: int | None = None):
         p, w, keep = _ptr(base, np.float32)
@@ -226,10 +236,22 @@ class Context:
         nq = Q.shape[0]
         dev = Q.device
         k = params.k if params.k > 0 else 1 << (max(params.beam, 1) - 1).bit_length()
-        pq = torch.empty((nq, self.d_out), dtype=torch.float32, device=dev)
-        leaf = torch.zeros(nq, dtype=torch.int32, device=dev)
-        ids = torch.empty((nq, k), dtype=torch.int32, device=dev)
-        dists = torch.empty((nq, k), dtype=torch.float32, device=dev)
+        # The outputs come from the library stream's own pool: their memory is
+        # handed out again only to work behind this call, and the fill of the
+        # leaves runs there too.  Filled on torch's default stream, every call
+        # made that stream and the library's wait for each other: about 45 of a
+        # single query's 125 us, and no two contexts' queries ever overlapped
+        # (three contexts in turn: 126 -> 30 us a query).
+        with self._on_stream(dev):
+            pq = torch.empty((nq, self.d_out), dtype=torch.float32, device=dev)
+            leaf = (torch.empty if params.algo == 1 else torch.zeros)(nq, dtype=torch.int32,
+                                                                      device=dev)
+            ids = torch.empty((nq, k), dtype=torch.int32, device=dev)
+            dists = torch.empty((nq, k), dtype=torch.float32, device=dev)
+        cur = torch.cuda.current_stream(dev)
+        if cur.cuda_stream not in (0, self.stream):  # not ordered with the library's by itself
+            for t in (pq, leaf, ids, dists):
+                t.record_stream(cur)
         qp, _, _ = _ptr(Q, np.float32)
         P = lambda t: C.c_void_p(t.data_ptr())
         self._chk(lib().rte_query(self._h, qp, nq, C.byref(params), P(pq), P(leaf), P(ids),
