@@ -10,9 +10,9 @@
 // per-workgroup partials summed in a fixed order.  Covariance: the d x d
 // result is cut into 128 x 128 tiles; a workgroup accumulates, for one tile
 // on or above the diagonal and one range of rows, sum (x - mu)_i (x - mu)_j
-// with one 8 x 8 sub-tile per thread, the centred rows staged through LDS 16
-// at a time; the per-row-range partials are again summed in a fixed order
-// and the lower triangle is the mirror image (the products are the same
+// in FP64 matrix instructions, the centred rows staged through LDS 32 at a
+// time; the per-row-range partials are again summed in a fixed order and what
+// lies below the diagonal is the mirror image (the products are the same
 // numbers in the same order, so C is exactly symmetric).  Everything is
 // deterministic.
 #include <hip/hip_runtime.h>
@@ -28,39 +28,69 @@
 namespace rte {
 
 constexpr int kPcaTile = 128;
-constexpr int kPcaRowsLds = 16;
 constexpr int kPcaMaxD = 4096;
+
+// Sum of x[0], x[step], ... (n of them) in order: the loads of kSumAhead
+// elements are issued together, so the chain of additions and one memory round
+// trip per kSumAhead elements are what it takes (one round trip per element
+// otherwise: 1M x 128 column sums 808 -> 100 us, the reductions of their and
+// the covariance's partials 118 -> 13 and 123 -> 25 us).
+constexpr int kSumAhead = 32;
+template <typename T>
+__device__ __forceinline__ double ordered_sum(const T* __restrict__ x, int64_t step, int64_t n) {
+  double s = 0.0;
+  int64_t r = 0;
+  for (; r + kSumAhead <= n; r += kSumAhead) {
+    T v[kSumAhead];
+#pragma unroll
+    for (int i = 0; i < kSumAhead; ++i) v[i] = x[(r + i) * step];
+#pragma unroll
+    for (int i = 0; i < kSumAhead; ++i) s += (double)v[i];
+  }
+  for (; r < n; ++r) s += (double)x[r * step];
+  return s;
+}
 
 __global__ __launch_bounds__(256) void col_sum_kernel(const float* __restrict__ X, int64_t n,
                                                       int d, int64_t stride, int64_t rpb,
                                                       double* __restrict__ partial) {
   const int64_t r0 = (int64_t)blockIdx.x * rpb;
   const int64_t r1 = r0 + rpb < n ? r0 + rpb : n;
-  for (int c = threadIdx.x; c < d; c += blockDim.x) {
-    double s = 0.0;
-    for (int64_t r = r0; r < r1; ++r) s += (double)X[r * stride + c];
-    partial[(int64_t)blockIdx.x * d + c] = s;
-  }
+  for (int c = threadIdx.x; c < d; c += blockDim.x)
+    partial[(int64_t)blockIdx.x * d + c] = ordered_sum(X + r0 * stride + c, stride, r1 - r0);
 }
 
 __global__ void col_mean_kernel(const double* __restrict__ partial, int nb, int d, int64_t n,
                                 double* __restrict__ mean) {
   const int c = blockIdx.x * blockDim.x + threadIdx.x;
   if (c >= d) return;
-  double s = 0.0;
-  for (int b = 0; b < nb; ++b) s += partial[(int64_t)b * d + c];
-  mean[c] = s / (double)n;
+  mean[c] = ordered_sum(partial + c, d, nb) / (double)n;
 }
 
 // grid (row ranges, tile pairs); tile pair p -> (bi, bj), bi <= bj, row-major
-// over the upper triangle of the nt x nt tile grid
-__global__ __launch_bounds__(256) void cov_partial_kernel(const float* __restrict__ X, int64_t n,
+// over the upper triangle of the nt x nt tile grid.
+//
+// Products on v_mfma_f64_16x16x4: lane l gives A[l % 16][l / 16] and
+// B[l / 16][l % 16] and holds D[4 r + l / 16][l % 16], and an element is the
+// chain of four FMAs in ascending k, so a sum has the bits of one FMA per row,
+// row after row.  (The FP64 vector unit has the same rate, but an 8 x 8 block a
+// thread reads 128 bytes of LDS per 64 FMAs, which takes LDS as long as the
+// FMAs take.)  Both operands of a block of 16 columns are the same 64 numbers.
+// Off the diagonal a wave has 4 x 4 blocks of 16 x 16.  On it only the 36 blocks
+// with row <= column are computed, nine a wave: block rows w and 7 - w.  A row
+// of LDS is 144 doubles, so the four rows of an operand lie in both halves of
+// the banks.  The next rows' loads are in flight during the products.
+// 1M x 128: 420 us, 1225 us with an 8 x 8 block a thread.
+constexpr int kCovRows = 32;
+constexpr int kCovPitch = kPcaTile + 16;
+typedef double f64x4 __attribute__((ext_vector_type(4)));
+__global__ __launch_bounds__(256, 2) void cov_partial_kernel(const float* __restrict__ X, int64_t n,
                                                           int d, int64_t stride,
                                                           const double* __restrict__ mean,
                                                           int64_t rpb, int nt,
                                                           double* __restrict__ partial) {
-  __shared__ double ra[kPcaRowsLds][kPcaTile];
-  __shared__ double rb[kPcaRowsLds][kPcaTile];
+  __shared__ double ra[kCovRows * kCovPitch];
+  __shared__ double rb[kCovRows * kCovPitch];
   int p = blockIdx.y, bi = 0;
   while (p >= nt - bi) {
     p -= nt - bi;
@@ -68,47 +98,112 @@ __global__ __launch_bounds__(256) void cov_partial_kernel(const float* __restric
   }
   const int bj = bi + p;
   const int c0 = bi * kPcaTile, c1 = bj * kPcaTile;
-  const int t = threadIdx.x;
-  const int ti = t >> 4, tj = t & 15;  // 8 x 8 sub-tile (ti, tj) of the 16 x 16 grid
-  double acc[8][8];
-#pragma unroll
-  for (int i = 0; i < 8; ++i)
-#pragma unroll
-    for (int j = 0; j < 8; ++j) acc[i][j] = 0.0;
+  const int t = threadIdx.x, lane = t & 63;
+  const int w = __builtin_amdgcn_readfirstlane(t >> 6);
   const int64_t r0 = (int64_t)blockIdx.x * rpb;
   const int64_t r1 = r0 + rpb < n ? r0 + rpb : n;
-  for (int64_t rs = r0; rs < r1; rs += kPcaRowsLds) {
-    const int nr = (int)(r1 - rs < kPcaRowsLds ? r1 - rs : kPcaRowsLds);
-    for (int e = t; e < kPcaRowsLds * kPcaTile; e += 256) {
-      const int rr = e / kPcaTile, c = e - rr * kPcaTile;
-      const bool ok = rr < nr;
-      ra[rr][c] = ok && c0 + c < d ? (double)X[(rs + rr) * stride + c0 + c] - mean[c0 + c] : 0.0;
-      rb[rr][c] = ok && c1 + c < d ? (double)X[(rs + rr) * stride + c1 + c] - mean[c1 + c] : 0.0;
+  // thread t stages column t % 128 of rows t / 128 + 2 i; rows past the range
+  // are zeros, columns past d (any valid one) only reach elements past d
+  constexpr int kPer = kCovRows * kPcaTile / 256;
+  const int sc = t & (kPcaTile - 1), sr = t / kPcaTile;
+  const int ca = min(c0 + sc, d - 1), cb = min(c1 + sc, d - 1);
+  const double ma = mean[ca], mb = mean[cb];
+  auto load = [&](int64_t rs, int c, float (&v)[kPer]) {  // at clamped, valid addresses
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) v[i] = X[min(rs + sr + 2 * i, n - 1) * stride + c];
+  };
+  auto stage = [&](int64_t rs, const float (&v)[kPer], double m, double* dst) {
+    dst += sr * kCovPitch + sc;
+    if (rs + kCovRows <= r1) {
+#pragma unroll
+      for (int i = 0; i < kPer; ++i) dst[2 * i * kCovPitch] = (double)v[i] - m;
+    } else {
+#pragma unroll
+      for (int i = 0; i < kPer; ++i)
+        dst[2 * i * kCovPitch] = rs + sr + 2 * i < r1 ? (double)v[i] - m : 0.0;
     }
-    __syncthreads();
-    for (int rr = 0; rr < nr; ++rr) {
-      double a[8], b[8];
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        a[i] = ra[rr][8 * ti + i];
-        b[i] = rb[rr][8 * tj + i];
-      }
-#pragma unroll
-      for (int i = 0; i < 8; ++i)
-#pragma unroll
-        for (int j = 0; j < 8; ++j) acc[i][j] = __builtin_fma(a[i], b[j], acc[i][j]);
-    }
-    __syncthreads();
-  }
+  };
   double* out = partial + (int64_t)blockIdx.x * d * d;
+  const int lo = (lane >> 4) * kCovPitch + (lane & 15);  // the lane's element of an operand
+  auto store = [&](int gi, int gj, const f64x4& v) {     // a 16 x 16 block at (gi, gj)
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const int gi = c0 + 8 * ti + i;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const int gj = c1 + 8 * tj + j;
-      if (gi < d && gj < d) out[(int64_t)gi * d + gj] = acc[i][j];
+    for (int r = 0; r < 4; ++r) {
+      const int i = gi + 4 * r + (lane >> 4), j = gj + (lane & 15);
+      if (i < d && j < d) out[(int64_t)i * d + j] = v[r];
     }
+  };
+  if (bi == bj) {
+    constexpr int kT = 9;
+    f64x4 acc[kT];
+    int br[kT], bc[kT];  // block row and column of the wave's blocks
+#pragma unroll
+    for (int q = 0; q < kT; ++q) {
+      acc[q] = f64x4{0.0, 0.0, 0.0, 0.0};
+      br[q] = q < 8 - w ? w : 7 - w;
+      bc[q] = q < 8 - w ? w + q : q - 1;
+    }
+    float va[kPer];
+    if (r0 < r1) load(r0, ca, va);
+    for (int64_t rs = r0; rs < r1; rs += kCovRows) {
+      stage(rs, va, ma, ra);
+      __syncthreads();
+      if (rs + kCovRows < r1) load(rs + kCovRows, ca, va);
+#pragma unroll 2
+      for (int k = 0; k < kCovRows; k += 4) {
+        double fa[kT], fb[kT];
+#pragma unroll
+        for (int q = 0; q < kT; ++q) {
+          fa[q] = ra[k * kCovPitch + 16 * br[q] + lo];
+          fb[q] = ra[k * kCovPitch + 16 * bc[q] + lo];
+        }
+#pragma unroll
+        for (int q = 0; q < kT; ++q)
+          acc[q] = __builtin_amdgcn_mfma_f64_16x16x4f64(fa[q], fb[q], acc[q], 0, 0, 0);
+      }
+      __syncthreads();
+    }
+#pragma unroll
+    for (int q = 0; q < kT; ++q) store(c0 + 16 * br[q], c1 + 16 * bc[q], acc[q]);
+  } else {
+    const int wi = 4 * (w >> 1), wj = 4 * (w & 1);
+    f64x4 acc[4][4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) acc[i][j] = f64x4{0.0, 0.0, 0.0, 0.0};
+    float va[kPer], vb[kPer];
+    if (r0 < r1) {
+      load(r0, ca, va);
+      load(r0, cb, vb);
+    }
+    for (int64_t rs = r0; rs < r1; rs += kCovRows) {
+      stage(rs, va, ma, ra);
+      stage(rs, vb, mb, rb);
+      __syncthreads();
+      if (rs + kCovRows < r1) {
+        load(rs + kCovRows, ca, va);
+        load(rs + kCovRows, cb, vb);
+      }
+#pragma unroll 2
+      for (int k = 0; k < kCovRows; k += 4) {
+        double fa[4], fb[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          fa[q] = ra[k * kCovPitch + 16 * (wi + q) + lo];
+          fb[q] = rb[k * kCovPitch + 16 * (wj + q) + lo];
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+            acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(fa[i], fb[j], acc[i][j], 0, 0, 0);
+      }
+      __syncthreads();
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) store(c0 + 16 * (wi + i), c1 + 16 * (wj + j), acc[i][j]);
   }
 }
 
@@ -117,53 +212,100 @@ __global__ void cov_reduce_kernel(const double* __restrict__ partial, int nb, in
   const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (e >= (int64_t)d * d) return;
   const int i = (int)(e / d), j = (int)(e - (int64_t)i * d);
-  // tiles below the diagonal were not computed: read the mirror element
-  const int64_t src = i / kPcaTile > j / kPcaTile ? (int64_t)j * d + i : e;
-  double s = 0.0;
-  for (int b = 0; b < nb; ++b) s += partial[(int64_t)b * d * d + src];
-  C[e] = s / (double)(n > 1 ? n - 1 : 1);  // pca.cpp:8-9
+  if (i / 16 > j / 16) return;  // blocks below the diagonal: mirror images
+  const double v =
+      ordered_sum(partial + e, (int64_t)d * d, nb) / (double)(n > 1 ? n - 1 : 1);  // pca.cpp:8-9
+  C[e] = v;
+  if (i / 16 < j / 16) C[(int64_t)j * d + i] = v;
 }
 
 // out[i][c] = sum_j ((double)X[i][j] - (double)mu[j]) * (double)R[j][c],
 // j ascending, multiply then add (the library is built without contraction),
-// stored FP32 -- the FP64 rotation of pca.cpp:122-139.  A workgroup computes
-// 16 rows x 128 columns (8 rows per thread); the centred rows are staged
-// through LDS 128 columns of X at a time.
-__global__ __launch_bounds__(256) void pca_rotate_kernel(const float* __restrict__ X, int64_t n,
+// stored FP32 -- the FP64 rotation of pca.cpp:122-139.
+//
+// Bound by the FP64 multiplies and adds (no FMA, so no matrix instruction: its
+// products are not rounded).  A lane has one row and 16 columns, a wave 64 rows:
+// the centred values, staged through LDS as [j][row] 64 columns of X at a time,
+// cost one 8-byte read per 32 operations, and R, widened to FP64 in rows of a
+// multiple of 16 columns, comes by scalar loads.  A workgroup has up to eight
+// waves, 128 columns.  1M x 128 x 128: 1275 us (834 us at the nominal rate);
+// 1728 us with eight rows and one column a thread, whose reads of the centred
+// values took LDS twice as long as the arithmetic.
+constexpr int kRotRows = 64;
+constexpr int kRotCols = 16;
+constexpr int kRotK = 64;
+__global__ __launch_bounds__(256) void widen_kernel(const float* __restrict__ R, int d, int d_out,
+                                                    int ldr, double* __restrict__ W) {
+  const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (e >= (int64_t)(d + 1) * ldr) return;
+  const int j = (int)(e / ldr), c = (int)(e - (int64_t)j * ldr);
+  W[e] = j < d && c < d_out ? (double)R[(int64_t)j * d_out + c] : 0.0;
+}
+
+__global__ __launch_bounds__(512) void pca_rotate_kernel(const float* __restrict__ X, int64_t n,
                                                          int d, int64_t stride,
-                                                         const float* __restrict__ R,
+                                                         const double* __restrict__ W, int ldr,
                                                          const float* __restrict__ mu, int d_out,
                                                          float* __restrict__ out) {
-  __shared__ double xs[kPcaRowsLds][kPcaTile];
-  const int t = threadIdx.x;
-  const int c = blockIdx.y * kPcaTile + (t & 127);
-  const int half = t >> 7;
-  const int64_t row0 = (int64_t)blockIdx.x * kPcaRowsLds;
-  double acc[8];
+  constexpr int kPitch = kRotRows + 1;
+  __shared__ double xs[(kRotK + 1) * kPitch];
+  const int t = threadIdx.x, lane = t & 63;
+  const int w = __builtin_amdgcn_readfirstlane(t >> 6), nw = blockDim.x >> 6;
+  const int c0 = blockIdx.y * kPcaTile + w * kRotCols;
+  const bool active = c0 < d_out;
+  const int64_t row0 = (int64_t)blockIdx.x * kRotRows;
+  double acc[kRotCols];
 #pragma unroll
-  for (int i = 0; i < 8; ++i) acc[i] = 0.0;
-  for (int j0 = 0; j0 < d; j0 += kPcaTile) {
-    for (int e = t; e < kPcaRowsLds * kPcaTile; e += 256) {
-      const int rr = e / kPcaTile, j = j0 + (e - rr * kPcaTile);
-      xs[rr][e - rr * kPcaTile] =
-          row0 + rr < n && j < d ? (double)X[(row0 + rr) * stride + j] - (double)mu[j] : 0.0;
-    }
+  for (int i = 0; i < kRotCols; ++i) acc[i] = 0.0;
+  typedef const __attribute__((address_space(4))) double* cptr;  // read-only: scalar loads
+  const cptr Wc = (cptr)W + c0;
+  for (int j0 = 0; j0 < d; j0 += kRotK) {
+    const int jn = d - j0 < kRotK ? d - j0 : kRotK;
+    // wave w stages rows w, w + nw, ...; a lane its column (past d: not used)
+    const int j = min(j0 + lane, d - 1);
+    const double m = (double)mu[j];
+#pragma unroll 8
+    for (int r = w; r < kRotRows; r += nw)
+      xs[lane * kPitch + r] = (double)X[min(row0 + r, n - 1) * stride + j] - m;
     __syncthreads();
-    const int jn = d - j0 < kPcaTile ? d - j0 : kPcaTile;
-    if (c < d_out) {
-      for (int j = 0; j < jn; ++j) {
-        const double r = (double)R[(int64_t)(j0 + j) * d_out + c];
+    if (active) {
+      double r[kRotCols], x = xs[lane];
+      cptr wr = Wc + (int64_t)j0 * ldr;
 #pragma unroll
-        for (int i = 0; i < 8; ++i) acc[i] = acc[i] + xs[8 * half + i][j] * r;
+      for (int i = 0; i < kRotCols; ++i) r[i] = wr[i];
+#pragma unroll 2
+      for (int k = 0; k < jn; ++k) {
+        // scalar loads return in any order: wait for this row's, ask for the
+        // next (W and xs have a spare one), then multiply
+        __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
+        __builtin_amdgcn_sched_barrier(0);
+        wr += ldr;
+        double rn[kRotCols];
+        const double xn = xs[(k + 1) * kPitch + lane];
+#pragma unroll
+        for (int i = 0; i < kRotCols; ++i) rn[i] = wr[i];
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < kRotCols; ++i) acc[i] = acc[i] + x * r[i];
+        x = xn;
+#pragma unroll
+        for (int i = 0; i < kRotCols; ++i) r[i] = rn[i];
       }
     }
     __syncthreads();
   }
-  if (c < d_out) {
+  const int64_t row = row0 + lane;
+  if (active && row < n) {
+    float* o = out + row * d_out + c0;
+    if (c0 + kRotCols <= d_out && (d_out & 3) == 0 && ((uintptr_t)out & 15) == 0) {
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int64_t row = row0 + 8 * half + i;
-      if (row < n) out[row * d_out + c] = (float)acc[i];
+      for (int i = 0; i < kRotCols; i += 4)
+        *reinterpret_cast<float4*>(o + i) =
+            make_float4((float)acc[i], (float)acc[i + 1], (float)acc[i + 2], (float)acc[i + 3]);
+    } else {
+#pragma unroll
+      for (int i = 0; i < kRotCols; ++i)
+        if (c0 + i < d_out) o[i] = (float)acc[i];
     }
   }
 }
@@ -182,7 +324,11 @@ __global__ __launch_bounds__(256) void pca_rotate_kernel(const float* __restrict
 // Householder step: A (d x d, row-major, only its lower triangle used) is
 // destroyed; on return A holds Q with A_in = Q T Q^T, diag the diagonal of T
 // and off[i] = T[i][i-1] (off[0] = 0).
-static void householder_tridiag(std::vector<double>& A, int d, std::vector<double>& diag,
+// Page-aligned, so that neither it nor the QL below crosses a page: with an
+// inner loop across a page boundary (wherever the linker happened to put it)
+// the fit at d = 960 took 505 ms instead of 378.
+constexpr int kCodePage = 4096;
+__attribute__((aligned(kCodePage))) static void householder_tridiag(std::vector<double>& A, int d, std::vector<double>& diag,
                                 std::vector<double>& off) {
   diag.assign(d, 0.0);
   off.assign(d, 0.0);
@@ -266,7 +412,7 @@ static void householder_tridiag(std::vector<double>& A, int d, std::vector<doubl
 // of Zt (row i = vector i, Q^T on entry): on return diag holds the
 // eigenvalues and row i of Zt the eigenvector of diag[i].  False if an
 // eigenvalue needed more than 60 iterations.
-static bool tridiag_ql(std::vector<double>& diag, std::vector<double>& off,
+__attribute__((aligned(kCodePage))) static bool tridiag_ql(std::vector<double>& diag, std::vector<double>& off,
                        std::vector<double>& Zt, int d) {
   for (int i = 1; i < d; ++i) off[i - 1] = off[i];
   off[d - 1] = 0.0;
@@ -359,7 +505,9 @@ int rte_pca_fit(rte_ctx* c, const float* X, int64_t n, int d, int64_t stride, fl
     return r;
   if (int r = ck(mean.reserve((size_t)d * sizeof(double)), "hipMalloc")) return r;
   if (int r = ck(cov.reserve(dd * sizeof(double)), "hipMalloc")) return r;
-  hipLaunchKernelGGL(rte::col_sum_kernel, dim3(nb_sum), dim3(256), 0, st, dx, n, d, stride,
+  // whole waves of columns, and no more
+  hipLaunchKernelGGL(rte::col_sum_kernel, dim3(nb_sum), dim3(std::min(256, (d + 63) / 64 * 64)), 0,
+                     st, dx, n, d, stride,
                      rpb_sum, part.as<double>());
   hipLaunchKernelGGL(rte::col_mean_kernel, dim3((d + 127) / 128), dim3(128), 0, st,
                      part.as<double>(), nb_sum, d, n, mean.as<double>());
@@ -409,7 +557,7 @@ int rte_pca_rotate(rte_ctx* c, const float* X, int64_t n, int d, int64_t stride,
   auto ck = [&](hipError_t e, const char* what) {
     return e == hipSuccess ? RTE_OK : rte_fail(c, RTE_EHIP, "%s: %s", what, hipGetErrorString(e));
   };
-  if ((n + rte::kPcaRowsLds - 1) / rte::kPcaRowsLds > 0x7fffffff)
+  if ((n + 15) / 16 > 0x7fffffff)
     return rte_fail(c, RTE_EUNSUP, "pca_rotate: too many rows");
   DevBuf xin, rm, ob;
   const float* dx = X;
@@ -423,18 +571,26 @@ int rte_pca_rotate(rte_ctx* c, const float* X, int64_t n, int d, int64_t stride,
     dx = xin.as<float>();
     dout = ob.as<float>();
   }
-  // R (d x d_out) and mu (d) are host arrays
-  if (int r = ck(rm.reserve(((size_t)d * d_out + d) * sizeof(float)), "hipMalloc")) return r;
-  float* dR = rm.as<float>();
+  // R (d x d_out) and mu (d) are host arrays; R widened comes first
+  const int ldr = (d_out + rte::kRotCols - 1) / rte::kRotCols * rte::kRotCols;
+  const size_t wide = (size_t)(d + 1) * ldr;
+  if (int r = ck(rm.reserve(wide * sizeof(double) + ((size_t)d * d_out + d) * sizeof(float)),
+                 "hipMalloc"))
+    return r;
+  double* dW = rm.as<double>();
+  float* dR = reinterpret_cast<float*>(dW + wide);
   float* dmu = dR + (size_t)d * d_out;
   if (int r = ck(hipMemcpyAsync(dR, R, (size_t)d * d_out * 4, hipMemcpyHostToDevice, st), "copy"))
     return r;
   if (int r = ck(hipMemcpyAsync(dmu, mu, (size_t)d * 4, hipMemcpyHostToDevice, st), "copy"))
     return r;
-  dim3 grid((unsigned)((n + rte::kPcaRowsLds - 1) / rte::kPcaRowsLds),
+  hipLaunchKernelGGL(rte::widen_kernel, dim3((unsigned)((wide + 255) / 256)), dim3(256), 0, st, dR,
+                     d, d_out, ldr, dW);
+  dim3 grid((unsigned)((n + rte::kRotRows - 1) / rte::kRotRows),
             (unsigned)((d_out + rte::kPcaTile - 1) / rte::kPcaTile));
-  hipLaunchKernelGGL(rte::pca_rotate_kernel, grid, dim3(256), 0, st, dx, n, d, stride, dR, dmu,
-                     d_out, dout);
+  const int waves = std::min(ldr, rte::kPcaTile) / rte::kRotCols;
+  hipLaunchKernelGGL(rte::pca_rotate_kernel, grid, dim3(64 * waves), 0, st, dx, n, d, stride, dW,
+                     ldr, dmu, d_out, dout);
   if (int r = ck(hipGetLastError(), "pca_rotate kernel")) return r;
   if (where == RTE_HOST) {
     if (int r = ck(hipMemcpyAsync(out, dout, obytes, hipMemcpyDeviceToHost, st), "copy")) return r;
