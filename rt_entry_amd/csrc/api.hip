@@ -499,10 +499,25 @@ int rte_set_pca(rte_ctx* c, const float* R, const float* mu, int d, int r_cols, 
   HIPCHK(c, c->rot.reserve((size_t)d * d_out * sizeof(float)), "hipMalloc(rot)");
   HIPCHK(c, c->bias.reserve((size_t)d_out * sizeof(float)), "hipMalloc(bias)");
   const hipMemcpyKind kind = where == RTE_HOST ? hipMemcpyHostToDevice : hipMemcpyDeviceToDevice;
-  // keep the first d_out columns (graph.cu:196 CopyHostToDevice(..., DIM))
-  HIPCHK(c, hipMemcpy2DAsync(c->rot.p, d_out * sizeof(float), R, r_cols * sizeof(float),
-                             d_out * sizeof(float), d, kind, c->stream),
-         "copy rotation");
+  // keep the first d_out columns (graph.cu:196 CopyHostToDevice(..., DIM)).  A
+  // host matrix is packed here and copied flat: under a profiler's queue
+  // interception a 2D copy from the host left L2 with what the memory held
+  // before (the covariance of a fit that had just been freed).
+  std::vector<float> packed;
+  if (where == RTE_HOST && r_cols > d_out) {
+    packed.resize((size_t)d * d_out);
+    for (int j = 0; j < d; ++j)
+      std::copy_n(R + (size_t)j * r_cols, d_out, packed.data() + (size_t)j * d_out);
+    R = packed.data();
+    r_cols = d_out;
+  }
+  if (r_cols == d_out)
+    HIPCHK(c, hipMemcpyAsync(c->rot.p, R, (size_t)d * d_out * sizeof(float), kind, c->stream),
+           "copy rotation");
+  else
+    HIPCHK(c, hipMemcpy2DAsync(c->rot.p, d_out * sizeof(float), R, r_cols * sizeof(float),
+                               d_out * sizeof(float), d, kind, c->stream),
+           "copy rotation");
   DevBuf mu_dev;
   HIPCHK(c, mu_dev.reserve(d * sizeof(float)), "hipMalloc(mu)");
   HIPCHK(c, hipMemcpyAsync(mu_dev.p, mu, d * sizeof(float), kind, c->stream), "copy mu");
