@@ -336,10 +336,14 @@ int rte_knn_rows(rte_ctx* c, const float* X, int64_t np, int d, int64_t stride, 
   HIPCHK(c, norms.reserve((size_t)np * sizeof(float)), "hipMalloc(norms)");
   const int64_t npad = rte::knn_padded(np);
   // without room for the whole-number kernel's buffers the FP32 kernel runs
-  const bool room = xb.reserve((size_t)npad * d * sizeof(uint16_t)) == hipSuccess &&
+  int slots = 0;
+  (void)hipDeviceGetAttribute(&slots, hipDeviceAttributeMultiprocessorCount, c->device);
+  slots = std::max(slots, 1);
+  const bool room = np <= rte::kKnnWholeMax &&
+                    xb.reserve((size_t)npad * d * sizeof(uint16_t)) == hipSuccess &&
                     half.reserve((size_t)npad * sizeof(float)) == hipSuccess &&
-                    lists.reserve((size_t)std::min(step, nrows) * 64 * sizeof(uint64_t)) ==
-                        hipSuccess &&
+                    lists.reserve(rte::knn_whole_keys(std::min(step, nrows), slots) *
+                                  sizeof(uint64_t)) == hipSuccess &&
                     flag.reserve(sizeof(uint32_t)) == hipSuccess;
   if (room) {
     HIPCHK(c, hipMemsetAsync(flag.p, 0, sizeof(uint32_t), c->stream), "clear flag");
@@ -368,7 +372,7 @@ int rte_knn_rows(rte_ctx* c, const float* X, int64_t np, int d, int64_t stride, 
     int32_t* ids = di + (r0 - row0) * k;
     float* dists = dd ? dd + (r0 - row0) * k : nullptr;
     if (whole)
-      HIPCHK(c, rte::launch_knn_whole(xb.as<uint16_t>(), half.as<float>(), np, d, r0, n, k,
+      HIPCHK(c, rte::launch_knn_whole(xb.as<uint16_t>(), half.as<float>(), np, d, r0, n, k, slots,
                                       lists.as<uint64_t>(), ids, dists, c->stream),
              "knn launch");
     else
