@@ -332,18 +332,17 @@ int rte_knn_rows(rte_ctx* c, const float* X, int64_t np, int d, int64_t stride, 
     if (int r = stage_out(c, c->s_aux2, dists_out, (size_t)nrows * k, where, &dd)) return r;
   // rows in launches of 128k (short kernels)
   const int64_t step = 1 << 17;
-  DevBuf norms, xb, half, flag, lists;  // freed on return (hipFree waits for the device)
+  DevBuf norms, xb, half, flag, work;  // freed on return (hipFree waits for the device)
   HIPCHK(c, norms.reserve((size_t)np * sizeof(float)), "hipMalloc(norms)");
   const int64_t npad = rte::knn_padded(np);
   // without room for the whole-number kernel's buffers the FP32 kernel runs
-  int slots = 0;
-  (void)hipDeviceGetAttribute(&slots, hipDeviceAttributeMultiprocessorCount, c->device);
-  slots = std::max(slots, 1);
+  int cus = 0;
+  (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device);
+  cus = std::max(cus, 1);
   const bool room = np <= rte::kKnnWholeMax &&
                     xb.reserve((size_t)npad * d * sizeof(uint16_t)) == hipSuccess &&
                     half.reserve((size_t)npad * sizeof(float)) == hipSuccess &&
-                    lists.reserve(rte::knn_whole_keys(std::min(step, nrows), slots) *
-                                  sizeof(uint64_t)) == hipSuccess &&
+                    work.reserve(rte::knn_whole_bytes(np, d, nrows, cus)) == hipSuccess &&
                     flag.reserve(sizeof(uint32_t)) == hipSuccess;
   if (room) {
     HIPCHK(c, hipMemsetAsync(flag.p, 0, sizeof(uint32_t), c->stream), "clear flag");
@@ -351,7 +350,7 @@ int rte_knn_rows(rte_ctx* c, const float* X, int64_t np, int d, int64_t stride, 
     (void)hipGetLastError();
     xb.release();
     half.release();
-    lists.release();
+    work.release();
     flag.release();
   }
   HIPCHK(c, rte::launch_row_norms(dx, np, d, stride, norms.as<float>(), xb.as<uint16_t>(),
@@ -367,18 +366,15 @@ int rte_knn_rows(rte_ctx* c, const float* X, int64_t np, int d, int64_t stride, 
   // FP32 one, exact either way (160k x 128, k = 64: 75.8 ms with the FP32
   // kernel)
   const bool whole = rte::knn_whole_numbers(bits);
-  for (int64_t r0 = row0; r0 < row0 + nrows; r0 += step) {
+  if (whole)
+    HIPCHK(c, rte::launch_knn_whole(xb.as<uint16_t>(), half.as<float>(), np, d, row0, nrows, k, cus,
+                                    work.p, di, dd, c->stream),
+           "knn launch");
+  for (int64_t r0 = row0; !whole && r0 < row0 + nrows; r0 += step) {
     const int64_t n = std::min<int64_t>(step, row0 + nrows - r0);
-    int32_t* ids = di + (r0 - row0) * k;
-    float* dists = dd ? dd + (r0 - row0) * k : nullptr;
-    if (whole)
-      HIPCHK(c, rte::launch_knn_whole(xb.as<uint16_t>(), half.as<float>(), np, d, r0, n, k, slots,
-                                      lists.as<uint64_t>(), ids, dists, c->stream),
-             "knn launch");
-    else
-      HIPCHK(c, rte::launch_knn(dx, np, d, stride, norms.as<float>(), r0, n, k, ids, dists,
-                                c->stream),
-             "knn launch");
+    HIPCHK(c, rte::launch_knn(dx, np, d, stride, norms.as<float>(), r0, n, k, di + (r0 - row0) * k,
+                              dd ? dd + (r0 - row0) * k : nullptr, c->stream),
+           "knn launch");
   }
   if (int r = finish_out(c, ids_out, di, (size_t)nrows * k, where)) return r;
   if (dists_out)

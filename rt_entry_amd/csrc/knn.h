@@ -33,15 +33,12 @@ inline int64_t knn_padded(int64_t np) { return (np + 63) / 64 * 64; }
 hipError_t launch_row_norms(const float* X, int64_t np, int d, int64_t stride, float* norms,
                             uint16_t* Xb, float* half, uint32_t* flag, hipStream_t st);
 // launch_knn for data of which knn_whole_numbers() holds and np <= kKnnWholeMax;
-// same lists.  At most `slots` workgroups (the card's compute units) run, and
-// `keys` is their scratch: knn_whole_keys(nq, slots) keys.
+// same lists, for rows [row0, row0 + nrows).  cus: the card's compute units;
+// `work` has knn_whole_bytes() bytes.
 constexpr int64_t kKnnWholeMax = 1 << 27;
-inline size_t knn_whole_keys(int64_t nq, int slots) {
-  const int64_t blocks = (nq + 255) / 256;
-  return (size_t)(blocks < slots ? blocks : slots) * 256 * 128;
-}
+size_t knn_whole_bytes(int64_t np, int d, int64_t nrows, int cus);
 hipError_t launch_knn_whole(const uint16_t* Xb, const float* half, int64_t np, int d, int64_t row0,
-                            int64_t nq, int k, int slots, uint64_t* keys, int32_t* ids,
-                            float* dists, hipStream_t st);
+                            int64_t nrows, int k, int cus, void* work, int32_t* ids, float* dists,
+                            hipStream_t st);
 
 }  // namespace rte

@@ -230,388 +230,6 @@ __global__ __launch_bounds__(512) void knn_kernel(const float* __restrict__ X, i
   }
 }
 
-// ---- whole-number data ----------------------------------------------------
-// kNN lists of data whose values are whole numbers of magnitude <= 256 (image
-// descriptors are bytes): they are bf16 values, so one bf16 MFMA product of 16
-// times the FP32 rate gives the same numbers.  The accumulator starts at
-// -(|q|^2 + |x|^2) / 2 and ends at -dist / 2.  With norms below 2^23 and no
-// negative value (below 2^22 with negative ones) every partial sum is a
-// multiple of 1/2 below 2^23 in magnitude: exact in FP32 in any order, and
-// equal to what the FP32 kernel computes.
-//
-// A workgroup of 8 waves owns 256 rows, 32 per wave (their operands in
-// registers), so that a 16-byte operand read of the tile feeds two MFMAs: with
-// 16 rows the LDS reads take twice the MFMAs' time.  Tiles of 64 points come
-// straight into an LDS ring of two groups of four (16-byte units XOR-swizzled
-// per point), one barrier a group: a wave's points to pick differ from tile to
-// tile, and with a barrier every tile each tile took as long as its slowest wave
-// and the waves of a SIMD were all at the matrix unit or all away from it.  A
-// point nearer than its row's threshold (the k-th best of the row's list) goes
-// to the wave's queue -- writes only, no round trip through LDS -- and 64 at a
-// time to the rows' buffers.  A buffer is sorted across the wave and merged
-// with its row's sorted list when it is full, and in all rows at tiles 0, 1, 3,
-// 6, ... times 1.7: a point enters the k best of n seen with probability k / n,
-// so that a buffer of 64 lasts while n grows by a factor.  Lists and buffers lie
-// in global memory, 1 KiB a row, touched by the row's wave only; the workgroups
-// are as many as the card holds at once and take block after block of rows, so
-// they stay in L2.
-//
-// 160k x 128, k = 64: 13.8 ms, 16.5 with two tiles in LDS and a barrier a tile.
-// 5 ms of it are products and operand reads, the rest points that pass.
-constexpr int kWnQueue = 416;  // queued points per wave: a block's 256 and some
-constexpr int kWnGroup = 4;    // tiles between barriers
-constexpr int kWnKeys = 128;   // of a row: 64 list, 64 buffer
-
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef __attribute__((address_space(3))) void lds_void_t;
-typedef __attribute__((address_space(1))) const void global_void_t;
-
-// compare-exchange of 64-bit keys at lane distance SUB: ascending, or
-// descending where DESC(lane) holds
-template <int SUB>
-__device__ __forceinline__ uint64_t cas_key(uint64_t k, int lane, bool want_larger) {
-  const uint32_t lo = (uint32_t)xor_lane<SUB>((int)(uint32_t)k, lane);
-  const uint32_t hi = (uint32_t)xor_lane<SUB>((int)(uint32_t)(k >> 32), lane);
-  const uint64_t p = ((uint64_t)hi << 32) | lo;
-  return (p > k) == want_larger ? p : k;
-}
-template <int STEP, int SUB>
-__device__ __forceinline__ uint64_t sort_keys_step(uint64_t k, int lane) {
-  // pairs of a step are descending where (lane & 2 * STEP) == 0
-  k = cas_key<SUB>(k, lane, ((lane & SUB) == 0) == ((lane & (2 * STEP)) == 0));
-  if constexpr (SUB > 1) return sort_keys_step<STEP, SUB / 2>(k, lane);
-  return k;
-}
-template <int STEP = 1>
-__device__ __forceinline__ uint64_t sort_keys_desc(uint64_t k, int lane) {
-  k = sort_keys_step<STEP, STEP>(k, lane);
-  if constexpr (STEP < 32) return sort_keys_desc<STEP * 2>(k, lane);
-  return k;
-}
-template <int SUB = 32>
-__device__ __forceinline__ uint64_t merge_keys_asc(uint64_t k, int lane) {
-  k = cas_key<SUB>(k, lane, (lane & SUB) != 0);
-  if constexpr (SUB > 1) return merge_keys_asc<SUB / 2>(k, lane);
-  return k;
-}
-
-template <int KS>  // d / 32
-struct WnTile {
-  static constexpr int CPR = 4 * KS;            // 16-byte units per point
-  static constexpr int SWM = (CPR & -CPR) - 1;  // 3, 7, 3, 15
-  static constexpr int UNITS = kKnnCols * CPR;  // per tile
-  static constexpr int SLOT = UNITS + 16;       // and 64 floats: -|x|^2 / 2
-};
-
-// 64 lanes x 16 (or 4) bytes from global memory to LDS at `dst` + 16 (4) * lane.
-// As asm, so that the compiler does not wait for it before every LDS read that
-// might alias; the kernel waits once, before the group's barrier.
-__device__ __forceinline__ void wn_copy16(const void* src, uint32_t dst) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(dst), "v"(src)
-               : "memory", "m0");
-}
-__device__ __forceinline__ void wn_copy4(const void* src, uint32_t dst) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off" ::"s"(dst), "v"(src)
-               : "memory", "m0");
-}
-
-// the kWnGroup tiles from `tile` (past the last: the last again, never read)
-template <int KS, int NW>
-__device__ __forceinline__ void wn_copy_group(const uint16_t* Xb, const float* half, int64_t tile,
-                                              int64_t ntile, uint32_t dst, int wave, int lane) {
-  using W = WnTile<KS>;
-#pragma unroll 1
-  for (int j = 0; j < kWnGroup; ++j) {
-    const int64_t n0 = min(tile + j, ntile - 1) * kKnnCols;
-    const uint32_t at = dst + 16u * (uint32_t)(j * W::SLOT);
-#pragma unroll
-    for (int i = 0; i < (W::UNITS / 64 + NW - 1) / NW; ++i) {
-      const int u0 = 64 * (NW * i + wave);
-      if (u0 < W::UNITS) {
-        const int u = u0 + lane, c = u / W::CPR, q = (u % W::CPR) ^ (c & W::SWM);
-        wn_copy16(Xb + (n0 + c) * (32 * KS) + 8 * q, at + 16u * (uint32_t)u0);
-      }
-    }
-    if (wave == j % NW) wn_copy4(half + n0 + lane, at + 16u * W::UNITS);
-  }
-}
-
-struct WnArgs {
-  const uint16_t* Xb;  // npad x d
-  const float* half;   // npad
-  int64_t np, npad;    // npad: a multiple of 64
-  int64_t row0, nq;
-  int k;
-  uint64_t* keys;  // gridDim x 32 NW rows x kWnKeys (distance bits << 32 | id), lists ascending
-  int32_t* ids_out;
-  float* dists_out;
-};
-
-template <int KS, int NW>
-__global__ __launch_bounds__(64 * NW, 1) void knn_whole_kernel(WnArgs a) {
-  using W = WnTile<KS>;
-  constexpr int D = 32 * KS;
-  constexpr int ROWS = 32 * NW;
-  constexpr uint64_t kNone = ~0ull;
-  __shared__ __attribute__((aligned(16))) uint4 ring[2 * kWnGroup * W::SLOT];
-  __shared__ uint2 qe[NW][kWnQueue];  // a wave's queue: product, row << 27 | id
-  __shared__ int cnt[ROWS];
-  __shared__ float thr[ROWS];  // -(k-th best distance) / 2 + |q|^2 / 2
-  __shared__ float hrow[ROWS];
-  const int t = threadIdx.x;
-  const int lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
-  const int r = lane & 15, g = lane >> 4;
-  const int lrow0 = 32 * wave;  // the wave's rows in the workgroup
-  const uint32_t ring0 = (uint32_t)(uintptr_t)(lds_void_t*)ring;
-  constexpr uint32_t kHalf = 16u * kWnGroup * W::SLOT;
-  const int64_t rend = a.row0 + a.nq;
-  const int64_t ntile = a.npad / kKnnCols;
-  uint64_t* const keys = a.keys + ((int64_t)blockIdx.x * ROWS + lrow0) * kWnKeys + lane;
-  for (int64_t blk = blockIdx.x; blk * ROWS < a.nq; blk += gridDim.x) {
-    const int64_t mrow0 = a.row0 + blk * ROWS + lrow0;
-    __syncthreads();  // every wave is done with the ring
-    wn_copy_group<KS, NW>(a.Xb, a.half, 0, ntile, ring0, wave, lane);
-    uint4 A[2][KS];
-#pragma unroll
-    for (int rb = 0; rb < 2; ++rb) {
-      const int64_t row = min(mrow0 + 16 * rb + r, a.np - 1);
-#pragma unroll
-      for (int s = 0; s < KS; ++s)
-        A[rb][s] = *reinterpret_cast<const uint4*>(a.Xb + row * D + 32 * s + 8 * g);
-    }
-    if (lane < 32) {  // nothing passes in a row past the end
-      cnt[lrow0 + lane] = 0;
-      thr[lrow0 + lane] = mrow0 + lane < rend ? -INFINITY : INFINITY;
-      hrow[lrow0 + lane] = a.half[min(mrow0 + lane, a.np - 1)];
-    }
-#pragma unroll 4
-    for (int i = 0; i < 32; ++i) keys[i * kWnKeys] = kNone;
-    wave_sync();
-    float th[2][4];
-    auto load_thr = [&]() {
-#pragma unroll
-      for (int rb = 0; rb < 2; ++rb)
-#pragma unroll
-        for (int v = 0; v < 4; ++v) th[rb][v] = thr[lrow0 + 16 * rb + 4 * g + v];
-    };
-    load_thr();
-    // rows' list and buffer (c entries) of row i of the wave, and their merge
-    auto take = [&](int i, int c, uint64_t& fresh, uint64_t& old) {
-      fresh = lane < c ? keys[i * kWnKeys + 64] : kNone;
-      old = keys[i * kWnKeys];
-    };
-    auto merge = [&](int i, uint64_t fresh, uint64_t old) {
-      fresh = sort_keys_desc(fresh, lane);
-      const uint64_t key = merge_keys_asc(fresh < old ? fresh : old, lane);
-      keys[i * kWnKeys] = key;
-      const uint32_t kth = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(key >> 32), a.k - 1);
-      if (lane == 0) {
-        cnt[lrow0 + i] = 0;
-        thr[lrow0 + i] = kth == 0xffffffffu
-                             ? -INFINITY
-                             : -0.5f * __uint_as_float(kth) - hrow[lrow0 + i];
-      }
-    };
-    // the lanes of mask m queue point col of row i with their product x
-    int queued = 0;
-    auto push = [&](uint64_t m, float x, int i, int col) {
-      if (__builtin_expect(m == 0, 1)) return;
-      const int at = queued + (int)__builtin_amdgcn_mbcnt_hi(
-                                  (uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
-      if (__builtin_amdgcn_inverse_ballot_w64(m))
-        qe[wave][at] = make_uint2(__float_as_uint(x), (uint32_t)i << 27 | (uint32_t)col);
-      queued += __popcll(m);
-    };
-    // the queued points (but a row itself) into their rows' buffers, 64 at a time
-    auto drain = [&]() {
-      wave_sync();
-      while (queued > 0) {
-        const int n = min(queued, 64);
-        queued -= n;
-        bool left = lane < n;
-        uint64_t key = kNone;
-        int i = -1;
-        if (left) {
-          const uint2 e = qe[wave][queued + lane];
-          i = (int)(e.y >> 27);
-          const uint32_t id = e.y & 0x7ffffffu;
-          // + 0: a distance of zero is +0, as a key too
-          const float dist =
-              __builtin_fmaf(-2.f, __uint_as_float(e.x) + hrow[lrow0 + i], 0.f);
-          key = (uint64_t)__float_as_uint(dist) << 32 | id;
-          left = (int64_t)id != mrow0 + i;
-        }
-        while (true) {
-          if (left) {
-            const int at = atomicAdd(&cnt[lrow0 + i], 1);
-            if (at < 64) {
-              (keys - lane)[i * kWnKeys + 64 + at] = key;
-              left = false;
-            }
-          }
-          wave_sync();
-          uint64_t full = __builtin_amdgcn_ballot_w64(left);
-          if (!full) break;
-          __builtin_amdgcn_s_waitcnt(0x0f70);  // the buffers' entries are written
-          while (full) {
-            const int f = __builtin_amdgcn_readlane(i, __builtin_ctzll(full));
-            uint64_t fresh, old;
-            take(f, 64, fresh, old);
-            merge(f, fresh, old);
-            full &= ~__builtin_amdgcn_ballot_w64(i == f);
-          }
-          wave_sync();
-        }
-      }
-    };
-    // every row's buffer into its list, the next row's keys in flight
-    auto flush_all = [&]() {
-      drain();
-      __builtin_amdgcn_s_waitcnt(0x0f70);
-      wave_sync();
-      const int c = lane < 32 ? min(cnt[lrow0 + lane], 64) : 0;
-      uint64_t todo = __builtin_amdgcn_ballot_w64(c > 0);
-      int i = 0;
-      uint64_t fresh = 0, old = 0;
-      if (todo) {
-        i = __builtin_ctzll(todo);
-        take(i, __builtin_amdgcn_readlane(c, i), fresh, old);
-      }
-      while (todo) {
-        todo &= todo - 1;
-        const int i1 = todo ? __builtin_ctzll(todo) : i;
-        uint64_t fresh1, old1;
-        take(i1, __builtin_amdgcn_readlane(c, i1), fresh1, old1);
-        merge(i, fresh, old);
-        i = i1;
-        fresh = fresh1;
-        old = old1;
-      }
-      wave_sync();
-      load_thr();
-    };
-    // a tile's operands in registers: a step's are read again, for the next
-    // tile, as soon as its products are under way, so that LDS and the matrix
-    // unit work at the same time and the picking waits for neither
-    uint4 b[KS][4];
-    float hx[4];
-    auto fetch_half = [&](const uint4* Bt, float (&h)[4]) {
-      const float* ht = reinterpret_cast<const float*>(Bt + W::UNITS);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) h[j] = ht[16 * j + r];
-    };
-    auto fetch_step = [&](const uint4* Bt, int s) {
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-        b[s][j] = Bt[(16 * j + r) * W::CPR + ((4 * s + g) ^ (r & W::SWM))];
-    };
-    // one tile: products, then the points that pass
-    auto tile = [&](int64_t n0, const uint4* following) {
-      floatx4 acc[2][4];
-      float hn[4] = {0.f, 0.f, 0.f, 0.f};
-      fetch_half(following, hn);
-#pragma unroll
-      for (int s = 0; s < KS; ++s) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-#pragma unroll
-          for (int rb = 0; rb < 2; ++rb)
-            acc[rb][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                __builtin_bit_cast(bf16x8, A[rb][s]), __builtin_bit_cast(bf16x8, b[s][j]),
-                s ? acc[rb][j] : floatx4{hx[j], hx[j], hx[j], hx[j]}, 0, 0, 0);
-        __builtin_amdgcn_sched_barrier(0);
-        fetch_step(following, s);
-        __builtin_amdgcn_sched_barrier(0);
-      }
-      asm volatile("" ::: "memory");  // the reads stay here
-#pragma unroll
-      for (int j = 0; j < 4; ++j) hx[j] = hn[j];
-      // points that pass, block (rb, v) by block; a block that the queue may
-      // have no room for (the first tiles) is left for the loop below.  What
-      // is done with them lies out of line: a tile's branches fall through
-      // unless a point passes (a taken branch costs a wave as much as ten
-      // instructions, and there were eight a tile)
-      uint32_t left = 0;
-      const int col0 = (int)n0 + r;
-#pragma unroll
-      for (int rb = 0; rb < 2; ++rb)
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          uint64_t m[4];
-#pragma unroll
-          for (int j = 0; j < 4; ++j) m[j] = __builtin_amdgcn_ballot_w64(acc[rb][j][v] > th[rb][v]);
-          if (__builtin_expect(((m[0] | m[1]) | (m[2] | m[3])) != 0, 0)) {
-            if (queued > kWnQueue - 256) {
-              left |= 1u << (4 * rb + v);
-            } else {
-              const int i = 16 * rb + 4 * g + v;
-#pragma unroll
-              for (int j = 0; j < 4; ++j) push(m[j], acc[rb][j][v], i, col0 + 16 * j);
-            }
-          }
-        }
-      if (__builtin_expect(queued >= 64, 0)) drain();
-      // a rolled loop, draining as it goes; the block's values are picked by a
-      // scalar branch
-      while (__builtin_expect(left != 0, 0)) {
-        const int q = __builtin_ctz(left);
-        left &= left - 1;
-        float x[4], tb = 0.f;
-#pragma unroll
-        for (int e = 0; e < 8; ++e)
-          if (e == q) {
-            tb = th[e >> 2][e & 3];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) x[j] = acc[e >> 2][j][e & 3];
-          }
-        const int i = 16 * (q >> 2) + 4 * g + (q & 3);
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-          push(__builtin_amdgcn_ballot_w64(x[j] > tb), x[j], i, col0 + 16 * j);
-        drain();
-      }
-    };
-    int64_t next = 0;
-    uint32_t here = 0;  // the ring's half that holds the group
-    for (int64_t t0 = 0; t0 < ntile; t0 += kWnGroup) {
-      // the group's copies have landed (each wave waits for its own) and every
-      // wave is done with the other half
-      __builtin_amdgcn_s_waitcnt(0x0f70);
-      __syncthreads();
-      if (t0 + kWnGroup < ntile)
-        wn_copy_group<KS, NW>(a.Xb, a.half, t0 + kWnGroup, ntile, ring0 + (kHalf - here), wave, lane);
-      const int n = (int)min<int64_t>(kWnGroup, ntile - t0);
-      const uint4* Bt = ring + here / 16;
-      fetch_half(Bt, hx);
-#pragma unroll
-      for (int s = 0; s < KS; ++s) fetch_step(Bt, s);
-#pragma unroll 1
-      for (int j = 0; j < n; ++j) {
-        const int64_t tl = t0 + j;
-        Bt += W::SLOT;
-        tile(tl * kKnnCols, j + 1 < n ? Bt : Bt - W::SLOT);  // past the group's last: not used
-        if (tl >= next) {
-          flush_all();
-          next = tl + 1 + 7 * tl / 10;
-        }
-      }
-      here = kHalf - here;
-    }
-    flush_all();
-    __builtin_amdgcn_s_waitcnt(0x0f70);
-#pragma unroll 4
-    for (int i = 0; i < 32; ++i) {
-      const int64_t row = mrow0 + i;
-      const uint64_t key = keys[i * kWnKeys];
-      if (row < rend && lane < a.k) {
-        a.ids_out[(row - a.row0) * a.k + lane] = (int32_t)(uint32_t)key;
-        if (a.dists_out)
-          a.dists_out[(row - a.row0) * a.k + lane] = __uint_as_float((uint32_t)(key >> 32));
-      }
-    }
-  }
-}
-
 // ---- search graph from kNN lists -----------------------------------------
 // Candidate edges of u: forward u -> knn[u][j] (rank j, type 0) and reverse
 // u -> v for every v with knn[v][j] == u, j < rev_rank (rank j, type 1); a
@@ -809,43 +427,6 @@ hipError_t launch_row_norms(const float* X, int64_t np, int d, int64_t stride, f
   const int64_t npad = knn_padded(np);
   hipLaunchKernelGGL(row_norms_kernel, dim3((unsigned)(npad / 64)), dim3(256), 0, st, X, np, d,
                      stride, npad, norms, Xb, half, flag);
-  return hipGetLastError();
-}
-
-hipError_t launch_knn_whole(const uint16_t* Xb, const float* half, int64_t np, int d, int64_t row0,
-                            int64_t nq, int k, int slots, uint64_t* keys, int32_t* ids,
-                            float* dists, hipStream_t st) {
-  WnArgs a{Xb, half, np, knn_padded(np), row0, nq, k, keys, ids, dists};
-  // whole rounds of 256-row blocks first; what is left over in blocks of 128
-  // rows where they still run all at once (a round of them takes 0.6 of one of
-  // 256-row blocks)
-  const int64_t blocks = (nq + 255) / 256, rest = blocks % slots;
-  const bool split = 2 * rest <= slots;
-  const int64_t n8 = split ? std::min(nq, (blocks - rest) * 256) : nq;
-#define KNNW(KS)                                                                                 \
-  {                                                                                              \
-    a.nq = n8;                                                                                   \
-    if (a.nq > 0)                                                                                \
-      hipLaunchKernelGGL((knn_whole_kernel<KS, 8>),                                              \
-                         dim3((unsigned)std::min<int64_t>((a.nq + 255) / 256, slots)), dim3(512), \
-                         0, st, a);                                                              \
-    a.row0 = row0 + n8;                                                                          \
-    a.nq = nq - n8;                                                                              \
-    a.ids_out = ids + n8 * k;                                                                    \
-    a.dists_out = dists ? dists + n8 * k : nullptr;                                              \
-    if (a.nq > 0)                                                                                \
-      hipLaunchKernelGGL((knn_whole_kernel<KS, 4>), dim3((unsigned)((a.nq + 127) / 128)),        \
-                         dim3(256), 0, st, a);                                                   \
-    break;                                                                                       \
-  }
-  switch (d / 32) {
-    case 1: KNNW(1)
-    case 2: KNNW(2)
-    case 3: KNNW(3)
-    case 4: KNNW(4)
-    default: return hipErrorInvalidValue;
-  }
-#undef KNNW
   return hipGetLastError();
 }
 
