@@ -54,6 +54,15 @@ int hip_fail(rte_ctx* c, hipError_t e, const char* what) {
     if (e_ != hipSuccess) return hip_fail(ctx, e_, what); \
   } while (0)
 
+// s_work is kept for the next call up to 1 GiB (allocating and freeing it took 1 ms
+// of the 4 ms that lists and graph of 160k points take)
+struct WorkGuard {
+  rte_ctx* c;
+  ~WorkGuard() {
+    if (c->s_work.bytes > (size_t)1 << 30) c->s_work.release();  // hipFree waits for the device
+  }
+};
+
 bool is_pow2(int x) { return x > 0 && (x & (x - 1)) == 0; }
 int pow2_ceil(int x) {
   int p = 1;
@@ -332,54 +341,55 @@ int rte_knn_rows(rte_ctx* c, const float* X, int64_t np, int d, int64_t stride, 
     if (int r = stage_out(c, c->s_aux2, dists_out, (size_t)nrows * k, where, &dd)) return r;
   // rows in launches of 128k (short kernels)
   const int64_t step = 1 << 17;
-  DevBuf norms, xb, half, flag, work;  // freed on return (hipFree waits for the device)
-  HIPCHK(c, norms.reserve((size_t)np * sizeof(float)), "hipMalloc(norms)");
   const int64_t npad = rte::knn_padded(np);
-  // without room for the whole-number kernel's buffers the FP32 kernel runs
   int cus = 0;
   (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device);
   cus = std::max(cus, 1);
+  // norms | half | flag | bf16 rows | the whole-number kernel's scratch; without
+  // room for the last four (and half) the FP32 kernel runs
+  auto up = [](size_t n) { return (n + 255) & ~(size_t)255; };
+  const size_t norm_bytes = up((size_t)npad * sizeof(float)),
+               xb_bytes = up((size_t)npad * d * sizeof(uint16_t));
   const bool room = np <= rte::kKnnWholeMax &&
-                    xb.reserve((size_t)npad * d * sizeof(uint16_t)) == hipSuccess &&
-                    half.reserve((size_t)npad * sizeof(float)) == hipSuccess &&
-                    work.reserve(rte::knn_whole_bytes(np, d, nrows, cus)) == hipSuccess &&
-                    flag.reserve(sizeof(uint32_t)) == hipSuccess;
-  if (room) {
-    HIPCHK(c, hipMemsetAsync(flag.p, 0, sizeof(uint32_t), c->stream), "clear flag");
-  } else {
+                    c->s_work.reserve(2 * norm_bytes + 256 + xb_bytes +
+                                      rte::knn_whole_bytes(np, d, nrows, cus)) == hipSuccess;
+  WorkGuard guard{c};
+  if (!room) {
     (void)hipGetLastError();
-    xb.release();
-    half.release();
-    work.release();
-    flag.release();
+    HIPCHK(c, c->s_work.reserve(norm_bytes), "hipMalloc(norms)");
   }
-  HIPCHK(c, rte::launch_row_norms(dx, np, d, stride, norms.as<float>(), xb.as<uint16_t>(),
-                                  half.as<float>(), flag.as<uint32_t>(), c->stream),
+  char* w = c->s_work.as<char>();
+  float* norms = reinterpret_cast<float*>(w);
+  float* half = room ? reinterpret_cast<float*>(w + norm_bytes) : nullptr;
+  uint32_t* flag = room ? reinterpret_cast<uint32_t*>(w + 2 * norm_bytes) : nullptr;
+  uint16_t* xb = room ? reinterpret_cast<uint16_t*>(w + 2 * norm_bytes + 256) : nullptr;
+  void* work = room ? w + 2 * norm_bytes + 256 + xb_bytes : nullptr;
+  if (room) HIPCHK(c, hipMemsetAsync(flag, 0, sizeof(uint32_t), c->stream), "clear flag");
+  HIPCHK(c, rte::launch_row_norms(dx, np, d, stride, norms, xb, half, flag, c->stream),
          "norms");
   uint32_t bits = rte::kKnnNotWhole;
   if (room) {
-    HIPCHK(c, hipMemcpyAsync(&bits, flag.p, sizeof bits, hipMemcpyDeviceToHost, c->stream),
+    HIPCHK(c, hipMemcpyAsync(&bits, flag, sizeof bits, hipMemcpyDeviceToHost, c->stream),
            "read flag");
     HIPCHK(c, hipStreamSynchronize(c->stream), "sync norms");
   }
   // whole numbers up to 256 with small norms: one bf16 product in place of an
-  // FP32 one, exact either way (160k x 128, k = 64: 75.8 ms with the FP32
-  // kernel)
+  // FP32 one, exact either way (160k x 128, k = 64: 2.3 ms in clusters, 18 for
+  // uniform values, 75.8 with the FP32 kernel)
   const bool whole = rte::knn_whole_numbers(bits);
   if (whole)
-    HIPCHK(c, rte::launch_knn_whole(xb.as<uint16_t>(), half.as<float>(), np, d, row0, nrows, k, cus,
-                                    work.p, di, dd, c->stream),
+    HIPCHK(c, rte::launch_knn_whole(xb, half, np, d, row0, nrows, k, cus, work, di, dd, c->stream),
            "knn launch");
   for (int64_t r0 = row0; !whole && r0 < row0 + nrows; r0 += step) {
     const int64_t n = std::min<int64_t>(step, row0 + nrows - r0);
-    HIPCHK(c, rte::launch_knn(dx, np, d, stride, norms.as<float>(), r0, n, k, di + (r0 - row0) * k,
+    HIPCHK(c, rte::launch_knn(dx, np, d, stride, norms, r0, n, k, di + (r0 - row0) * k,
                               dd ? dd + (r0 - row0) * k : nullptr, c->stream),
            "knn launch");
   }
   if (int r = finish_out(c, ids_out, di, (size_t)nrows * k, where)) return r;
   if (dists_out)
     if (int r = finish_out(c, dists_out, dd, (size_t)nrows * k, where)) return r;
-  HIPCHK(c, hipStreamSynchronize(c->stream), "sync knn");  // norms is freed on return
+  HIPCHK(c, hipStreamSynchronize(c->stream), "sync knn");  // s_work is idle on return
   return RTE_OK;
 }
 
@@ -399,9 +409,10 @@ int rte_graph_from_knn(rte_ctx* c, const int32_t* knn, int64_t np, int kf, int d
   int32_t* dg;
   if (int r = stage_in(c, c->s_aux, knn, (size_t)np * kf, where, &dk)) return r;
   if (int r = stage_out(c, c->s_out, graph_out, (size_t)np * degree, where, &dg)) return r;
-  DevBuf work;  // freed on return (hipFree waits for the device)
-  HIPCHK(c, work.reserve(rte::graph_from_knn_work_bytes(np, kf, rev_rank)), "hipMalloc(graph work)");
-  HIPCHK(c, rte::launch_graph_from_knn(dk, np, kf, degree, rev_rank, dg, work.p, c->stream),
+  HIPCHK(c, c->s_work.reserve(rte::graph_from_knn_work_bytes(np, kf, rev_rank)),
+         "hipMalloc(graph work)");
+  WorkGuard guard{c};
+  HIPCHK(c, rte::launch_graph_from_knn(dk, np, kf, degree, rev_rank, dg, c->s_work.p, c->stream),
          "graph launch");
   if (int r = finish_out(c, graph_out, dg, (size_t)np * degree, where)) return r;
   HIPCHK(c, hipStreamSynchronize(c->stream), "sync graph");

@@ -81,6 +81,9 @@ struct rte_ctx {
   // staging for host-pointer calls
   DevBuf s_in, s_out, s_aux, s_aux2, s_aux3;
 
+  // scratch of the graph-building calls, which end with the stream idle
+  DevBuf s_work;
+
   // batched search: per-query shapes, query order, work counter, and the
   // captured launch (reused while its key is unchanged)
   DevBuf b_k, b_beam, b_order, b_counter, b_kin, b_bin;

@@ -17,8 +17,10 @@
 // nearly all neighbours and tight thresholds, and then every tile that could hold
 // a nearer point than some row's k-th best: by the triangle inequality none of its
 // points is nearer than max(D - b, a - D) for a row at distance D from the pivot.
-// Data without clusters lose the sort and the padding to it, 0.1 of the time, and
-// gain that few points pass a threshold of the start.
+//
+// 160k x 128, k = 64: 2.3 ms in 160 clusters, of which 1.9 go to picking points in
+// about 30 tiles a block; 18 ms for uniform values, where every tile is visited
+// (products and operand reads 5, picking the rest); 73 ms with the FP32 kernel.
 #include <hip/hip_runtime.h>
 #include <float.h>
 #include <limits.h>
@@ -27,8 +29,8 @@
 
 #include <algorithm>
 
+#include "key_sort.h"
 #include "knn.h"
-#include "search_impl.h"
 
 namespace rte {
 
@@ -38,42 +40,16 @@ typedef __attribute__((address_space(3))) void lds_void_t;
 
 constexpr int kWnCols = 64;    // points per tile
 constexpr int kWnQueue = 416;  // queued points per wave: a block's 256 and some
-constexpr int kWnGroup = 3;    // tiles between barriers
+constexpr int kWnWaves = 4;    // of a workgroup
+constexpr int kWnRows = 32 * kWnWaves;
+constexpr int kWnPerCu = 2;    // workgroups
+constexpr int kWnGroup = 1;    // tiles between barriers
 constexpr int kWnKeys = 128;   // of a row: 64 list, 64 buffer
 constexpr int kWnPivots = 1024;
 constexpr int kWnBuckets = 32;  // of a cell, by distance from its pivot
 constexpr int kWnFarBins = 2048;
+constexpr int64_t kWnStep = 1 << 19;  // rows per launch
 constexpr int kWnList = 2048;  // tiles looked at together
-constexpr int kWnSteps = 6;    // of the bisection
-
-// compare-exchange of 64-bit keys at lane distance SUB: ascending, or
-// descending where DESC(lane) holds
-template <int SUB>
-__device__ __forceinline__ uint64_t cas_key(uint64_t k, int lane, bool want_larger) {
-  const uint32_t lo = (uint32_t)xor_lane<SUB>((int)(uint32_t)k, lane);
-  const uint32_t hi = (uint32_t)xor_lane<SUB>((int)(uint32_t)(k >> 32), lane);
-  const uint64_t p = ((uint64_t)hi << 32) | lo;
-  return (p > k) == want_larger ? p : k;
-}
-template <int STEP, int SUB>
-__device__ __forceinline__ uint64_t sort_keys_step(uint64_t k, int lane) {
-  // pairs of a step are descending where (lane & 2 * STEP) == 0
-  k = cas_key<SUB>(k, lane, ((lane & SUB) == 0) == ((lane & (2 * STEP)) == 0));
-  if constexpr (SUB > 1) return sort_keys_step<STEP, SUB / 2>(k, lane);
-  return k;
-}
-template <int STEP = 1>
-__device__ __forceinline__ uint64_t sort_keys_desc(uint64_t k, int lane) {
-  k = sort_keys_step<STEP, STEP>(k, lane);
-  if constexpr (STEP < 32) return sort_keys_desc<STEP * 2>(k, lane);
-  return k;
-}
-template <int SUB = 32>
-__device__ __forceinline__ uint64_t merge_keys_asc(uint64_t k, int lane) {
-  k = cas_key<SUB>(k, lane, (lane & SUB) != 0);
-  if constexpr (SUB > 1) return merge_keys_asc<SUB / 2>(k, lane);
-  return k;
-}
 
 template <int KS>  // d / 32
 struct WnTile {
@@ -94,6 +70,7 @@ struct WnLayout {
   int64_t np, slots;  // slots: of the sorted points, pads included, at most
   int d, pivots, ppad;
   int pivots1;  // those evenly spaced
+  int launches;
   uint16_t* Xs;   // slots x d: the points by cell
   float* hs;      // slots: -|x|^2 / 2 (-inf: no point)
   int32_t* sid;   // slots: row of X (-1: no point)
@@ -109,6 +86,7 @@ struct WnLayout {
   uint16_t* Pb;     // ppad x d
   float* ph;        // ppad
   int32_t* far;     // kWnFarBins counts of points by distance, and a counter
+  int32_t* next;    // of a launch: next block of rows
   int32_t* rows;    // rows asked for, by cell
   uint64_t* keys;   // of every row in flight: kWnKeys
 };
@@ -121,7 +99,8 @@ static size_t wn_layout(int64_t np, int d, int64_t nrows, int cus, char* w, WnLa
   l.ppad = (l.pivots + kWnCols - 1) / kWnCols * kWnCols;
   l.slots = (np + kWnCols - 1) / kWnCols * kWnCols + (int64_t)kWnCols * l.pivots;
   const int64_t nk = (int64_t)l.pivots * kWnBuckets;
-  const int64_t blocks = std::min<int64_t>((nrows + 255) / 256, cus);
+  const int64_t blocks = std::min<int64_t>((nrows + kWnRows - 1) / kWnRows, kWnPerCu * cus);
+  l.launches = (int)((nrows + kWnStep - 1) / kWnStep);
   size_t at = 0;
   auto take = [&](auto*& p, size_t n) {
     p = reinterpret_cast<std::remove_reference_t<decltype(p)>>(w + at);
@@ -142,8 +121,9 @@ static size_t wn_layout(int64_t np, int d, int64_t nrows, int cus, char* w, WnLa
   take(l.Pb, (size_t)l.ppad * d);
   take(l.ph, l.ppad);
   take(l.far, kWnFarBins + 1);
+  take(l.next, l.launches);
   take(l.rows, nrows);
-  take(l.keys, (size_t)blocks * 256 * kWnKeys);
+  take(l.keys, (size_t)blocks * kWnRows * kWnKeys);
   return at;
 }
 
@@ -162,6 +142,7 @@ __global__ __launch_bounds__(256) void wn_init_kernel(WnLayout l, const uint16_t
   }
   for (int64_t e = i; e < (int64_t)l.pivots * kWnBuckets; e += step) l.hist[e] = l.rhist[e] = 0;
   for (int64_t e = i; e < kWnFarBins + 1; e += step) l.far[e] = 0;
+  for (int64_t e = i; e < l.launches; e += step) l.next[e] = 0;
   const int units = l.d / 8;
   for (int64_t e = i; e < (int64_t)l.ppad * units; e += step) {
     const int p = (int)(e / units), u = (int)(e - (int64_t)p * units);
@@ -415,15 +396,15 @@ __device__ __forceinline__ void wn_copy4(const void* src, uint32_t dst) {
                : "memory", "m0");
 }
 
-// the tile of points from n0 to LDS at `dst`, by NW waves
-template <int KS, int NW>
+// the tile of points from n0 to LDS at `dst`, by the workgroup
+template <int KS>
 __device__ __forceinline__ void wn_copy_tile(const uint16_t* X, const float* half,
                                              const int32_t* ids, int64_t n0, uint32_t dst, int wave,
                                              int lane) {
   using W = WnTile<KS>;
 #pragma unroll
-  for (int i = 0; i < (W::UNITS / 64 + NW - 1) / NW; ++i) {
-    const int u0 = 64 * (NW * i + wave);
+  for (int i = 0; i < (W::UNITS / 64 + kWnWaves - 1) / kWnWaves; ++i) {
+    const int u0 = 64 * (kWnWaves * i + wave);
     if (u0 < W::UNITS) {
       const int u = u0 + lane, c = u / W::CPR, q = (u % W::CPR) ^ (c & W::SWM);
       wn_copy16(X + (n0 + c) * (32 * KS) + 8 * q, dst + 16u * (uint32_t)u0);
@@ -439,47 +420,46 @@ struct WnArgs {
   const float* half;   // np
   int64_t row0;        // of the outputs
   int64_t first, nq;   // of l.rows
+  int launch;
   int k;
   int32_t* ids_out;
   float* dists_out;
 };
 
-// A workgroup of NW waves owns 32 rows a wave (their operands in registers, so
+// A workgroup of four waves owns 32 rows a wave (their operands in registers, so
 // that a 16-byte operand read of a tile feeds two MFMAs: with 16 rows the LDS
 // reads take twice the MFMAs' time).  Tiles come straight into an LDS ring of two
-// groups of three (16-byte units XOR-swizzled per point), one barrier a group: a
-// wave's points to pick differ from tile to tile, and with a barrier every tile
-// each tile took as long as its slowest wave.  A point nearer than its row's
-// threshold (the k-th best of the row's list) goes to the wave's queue -- writes
+// tiles (16-byte units XOR-swizzled per point), one barrier a tile; two
+// workgroups a compute unit, since a wave's points to pick differ from tile to tile
+// and a workgroup waits for its slowest wave (one of eight waves, three tiles to a
+// barrier: 4.0 ms at 160k x 128, two: 2.6).  A point nearer than its row's threshold (the k-th best of the row's list) goes to the wave's queue -- writes
 // only, no round trip through LDS -- and 64 at a time to the rows' buffers.  A
 // buffer is sorted across the wave and merged with its row's sorted list when it
 // is full, in all rows at tiles 0, 1, 2, 4, ... times 1.8 (a point enters the k
 // best of n seen with probability k / n, so that a buffer of 64 lasts while n
-// grows by a factor), and after each of its lists of
-// tiles.  Lists and buffers lie in
-// global memory, 1 KiB a row, touched by the row's wave only; the workgroups are
-// as many as the card holds at once and take block after block of rows, so they
-// stay in L2.  Points come in any order of ids, so one at the k-th best distance
+// grows by a factor), and after each list of tiles.  Lists and buffers lie in global
+// memory, 1 KiB a row, touched by the row's wave only; the workgroups are as many as
+// the card holds at once and take block after block of rows, so they stay in L2.
+// Points come in any order of ids, so one at the k-th best distance
 // passes if its id is lower.
-template <int KS, int NW>
-__global__ __launch_bounds__(64 * NW, 1) void knn_whole_kernel(WnArgs a) {
+template <int KS>
+__global__ __launch_bounds__(64 * kWnWaves, 2) void knn_whole_kernel(WnArgs a) {
   using W = WnTile<KS>;
   constexpr int D = 32 * KS;
-  constexpr int ROWS = 32 * NW;
+  constexpr int ROWS = kWnRows;
   constexpr uint64_t kNone = ~0ull;
   __shared__ __attribute__((aligned(16))) uint4 ring[2 * kWnGroup * W::SLOT];
-  __shared__ uint2 qe[NW][kWnQueue];  // a wave's queue: product, row << 27 | id
+  __shared__ uint2 qe[kWnWaves][kWnQueue];  // a wave's queue: product, row << 27 | id
   __shared__ int cnt[ROWS];
   __shared__ float thr[ROWS];  // -(k-th best distance) / 2 + |q|^2 / 2
   __shared__ float kth[ROWS];  // k-th best distance
   __shared__ int kid[ROWS];    // its id
   __shared__ float hrow[ROWS];
   __shared__ int rid[ROWS];
-  __shared__ float blo[ROWS], bhi[ROWS], bmid[ROWS];  // bounds of the k-th best distance
   __shared__ float dmin[kWnPivots], dmax[kWnPivots];  // of the block's rows from a pivot
   __shared__ int list[kWnList];                       // tiles to visit
-  __shared__ int listed;
-  __shared__ float wk[NW];
+  __shared__ int listed;  // their number; before that, the block
+  __shared__ float wk[kWnWaves];
   const int t = threadIdx.x;
   const int lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
   const int r = lane & 15, g = lane >> 4;
@@ -488,11 +468,14 @@ __global__ __launch_bounds__(64 * NW, 1) void knn_whole_kernel(WnArgs a) {
   constexpr uint32_t kHalf = 16u * kWnGroup * W::SLOT;
   const int ntile = a.l.cstart[a.l.pivots] / kWnCols;
   uint64_t* const keys = a.l.keys + ((int64_t)blockIdx.x * ROWS + lrow0) * kWnKeys + lane;
-  for (int64_t blk = blockIdx.x; blk * ROWS < a.nq; blk += gridDim.x) {
-    const int64_t j0 = blk * ROWS;
-    const int last = (int)min<int64_t>(ROWS, a.nq - j0) - 1;  // the block's last row
+  while (true) {
     __syncthreads();  // every wave is done with the block before
-    for (int i = t; i < ROWS; i += 64 * NW) {
+    if (t == 0) listed = atomicAdd(&a.l.next[a.launch], 1);
+    __syncthreads();
+    const int64_t j0 = (int64_t)listed * ROWS;
+    if (j0 >= a.nq) break;
+    const int last = (int)min<int64_t>(ROWS, a.nq - j0) - 1;  // the block's last row
+    for (int i = t; i < ROWS; i += 64 * kWnWaves) {
       const int id = a.l.rows[a.first + j0 + min(i, last)];
       rid[i] = id;
       hrow[i] = a.half[id];
@@ -501,11 +484,8 @@ __global__ __launch_bounds__(64 * NW, 1) void knn_whole_kernel(WnArgs a) {
       thr[i] = i <= last ? -FLT_MAX : INFINITY;
       kth[i] = i <= last ? INFINITY : 0.f;
       kid[i] = INT_MAX;
-      blo[i] = 0.f;
-      bhi[i] = INFINITY;
-      bmid[i] = 4.f * fmaxf(a.l.d2[id], 16.f);
     }
-    for (int i = t; i < a.l.pivots; i += 64 * NW) {
+    for (int i = t; i < a.l.pivots; i += 64 * kWnWaves) {
       reinterpret_cast<uint32_t*>(dmin)[i] = 0x7f800000u;
       reinterpret_cast<uint32_t*>(dmax)[i] = 0u;
     }
@@ -523,7 +503,7 @@ __global__ __launch_bounds__(64 * NW, 1) void knn_whole_kernel(WnArgs a) {
     // the rows' distances from the pivots
     for (int p0 = 0; p0 < a.l.ppad; p0 += kWnCols) {
       __syncthreads();
-      wn_copy_tile<KS, NW>(a.l.Pb, a.l.ph, nullptr, p0, ring0, wave, lane);
+      wn_copy_tile<KS>(a.l.Pb, a.l.ph, nullptr, p0, ring0, wave, lane);
       __builtin_amdgcn_s_waitcnt(0x0f70);
       __syncthreads();
       const float* ht = reinterpret_cast<const float*>(ring + W::UNITS);
@@ -564,7 +544,7 @@ __global__ __launch_bounds__(64 * NW, 1) void knn_whole_kernel(WnArgs a) {
       }
     }
     __syncthreads();
-    for (int i = t; i < a.l.pivots; i += 64 * NW) {
+    for (int i = t; i < a.l.pivots; i += 64 * kWnWaves) {
       dmin[i] = sqrtf(dmin[i]);
       dmax[i] = sqrtf(dmax[i]);
     }
@@ -689,9 +669,8 @@ __global__ __launch_bounds__(64 * NW, 1) void knn_whole_kernel(WnArgs a) {
       for (int j = 0; j < 4; ++j)
         b[s][j] = Bt[(16 * j + r) * W::CPR + ((4 * s + g) ^ (r & W::SWM))];
     };
-    // one tile: products, then the points that pass (COUNT: their number)
-    int passing[2][4];
-    auto tile = [&](const uint4* Bt, const uint4* following, bool count) {
+    // one tile: products, then the points that pass
+    auto tile = [&](const uint4* Bt, const uint4* following) {
       floatx4 acc[2][4];
       float hn[4] = {0.f, 0.f, 0.f, 0.f};
       fetch_half(following, hn);
@@ -715,15 +694,6 @@ __global__ __launch_bounds__(64 * NW, 1) void knn_whole_kernel(WnArgs a) {
       asm volatile("" ::: "memory");  // the reads stay here
 #pragma unroll
       for (int j = 0; j < 4; ++j) hx[j] = hn[j];
-      if (count) {
-#pragma unroll
-        for (int rb = 0; rb < 2; ++rb)
-#pragma unroll
-          for (int v = 0; v < 4; ++v)
-#pragma unroll
-            for (int j = 0; j < 4; ++j) passing[rb][v] += acc[rb][j][v] >= th[rb][v] ? 1 : 0;
-        return;
-      }
       // points that pass, block (rb, v) by block; a block that the queue may
       // have no room for (the first tiles) is left for the loop below.  What
       // is done with them lies out of line: a tile's branches fall through
@@ -805,12 +775,12 @@ __global__ __launch_bounds__(64 * NW, 1) void knn_whole_kernel(WnArgs a) {
         if (phase == 3 || (phase == 2 && c0 == 0)) {
           float d = wk[0];
 #pragma unroll
-          for (int w = 1; w < NW; ++w) d = phase == 2 ? fminf(d, wk[w]) : fmaxf(d, wk[w]);
+          for (int w = 1; w < kWnWaves; ++w) d = phase == 2 ? fminf(d, wk[w]) : fmaxf(d, wk[w]);
           // distances as rounded: a margin of a ten-thousandth and 0.01
           bound = sqrtf(d) * 1.0002f + 0.01f;
           if (phase == 3 && bound <= above) break;
         }
-        for (int c = t; c < kWnList; c += 64 * NW) {
+        for (int c = t; c < kWnList; c += 64 * kWnWaves) {
           const int tl = c0 + c;
           bool keep = tl < hi;
           if (phase && keep) {
@@ -833,75 +803,34 @@ __global__ __launch_bounds__(64 * NW, 1) void knn_whole_kernel(WnArgs a) {
         auto copy_group = [&](int g0, uint32_t dst) {
 #pragma unroll 1
           for (int j = 0; j < kWnGroup && g0 + j < n; ++j)
-            wn_copy_tile<KS, NW>(a.l.Xs, a.l.hs, a.l.sid,
+            wn_copy_tile<KS>(a.l.Xs, a.l.hs, a.l.sid,
                                  (int64_t)__builtin_amdgcn_readfirstlane(list[g0 + j]) * kWnCols,
                                  dst + 16u * (uint32_t)(j * W::SLOT), wave, lane);
         };
-        // The first list: thresholds by bisection, each step a count of the points
-        // that would pass.  A count costs a tenth of what picking a cell's points
-        // with thresholds that only tighten as they come does.
-        const int steps = phase == 0 && c0 == own0 && n > 2 ? kWnSteps : 0;
-        for (int step = 0; step <= steps; ++step) {
-          const bool count = step < steps;
-          if (steps) {
-            if (step) __syncthreads();  // every wave is done with the ring
+        copy_group(0, ring0);
+        uint32_t here = 0;  // the ring's half that holds the group
+        for (int g0 = 0; g0 < n; g0 += kWnGroup) {
+          // the group's copies have landed (each wave waits for its own) and
+          // every wave is done with the other half
+          __builtin_amdgcn_s_waitcnt(0x0f70);
+          __syncthreads();
+          if (g0 + kWnGroup < n) copy_group(g0 + kWnGroup, ring0 + (kHalf - here));
+          const int m = min(kWnGroup, n - g0);
+          const uint4* Bt = ring + here / 16;
+          fetch_half(Bt, hx);
 #pragma unroll
-            for (int rb = 0; rb < 2; ++rb)
-#pragma unroll
-              for (int v = 0; v < 4; ++v) {
-                const int i = lrow0 + 16 * rb + 4 * g + v;
-                if (r == 0 && i <= last) {
-                  const float d = count ? bmid[i] : bhi[i];
-                  thr[i] = d < INFINITY ? -0.5f * d - hrow[i] : -FLT_MAX;
-                }
-                passing[rb][v] = 0;
-              }
-            wave_sync();
-            load_thr();
-            if (!count) next = seen + n;
-          }
-          copy_group(0, ring0);
-          uint32_t here = 0;  // the ring's half that holds the group
-          for (int g0 = 0; g0 < n; g0 += kWnGroup) {
-            // the group's copies have landed (each wave waits for its own) and
-            // every wave is done with the other half
-            __builtin_amdgcn_s_waitcnt(0x0f70);
-            __syncthreads();
-            if (g0 + kWnGroup < n) copy_group(g0 + kWnGroup, ring0 + (kHalf - here));
-            const int m = min(kWnGroup, n - g0);
-            const uint4* Bt = ring + here / 16;
-            fetch_half(Bt, hx);
-#pragma unroll
-            for (int s = 0; s < KS; ++s) fetch_step(Bt, s);
+          for (int s = 0; s < KS; ++s) fetch_step(Bt, s);
 #pragma unroll 1
-            for (int j = 0; j < m; ++j) {
-              tile(Bt, j + 1 < m ? Bt + W::SLOT : Bt, count);  // past the group's last: not used
-              Bt += W::SLOT;
-              if (count) continue;
-              if (seen >= next) {
-                flush_all();
-                next = seen + 1 + 8 * seen / 10;
-              }
-              ++seen;
+          for (int j = 0; j < m; ++j) {
+            tile(Bt, j + 1 < m ? Bt + W::SLOT : Bt);  // past the group's last: not used
+            Bt += W::SLOT;
+            if (seen >= next) {
+              flush_all();
+              next = seen + 1 + 8 * seen / 10;
             }
-            here = kHalf - here;
+            ++seen;
           }
-          if (!count) break;
-#pragma unroll
-          for (int rb = 0; rb < 2; ++rb)
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-              int c = passing[rb][v];
-#pragma unroll
-              for (int o = 1; o < 16; o <<= 1) c += __shfl_xor(c, o, 64);
-              const int i = lrow0 + 16 * rb + 4 * g + v;
-              if (r == 0) {  // the row itself is one of them
-                const float mid = bmid[i];
-                (c > a.k ? bhi[i] : blo[i]) = mid;
-                bmid[i] = bhi[i] < INFINITY ? 0.5f * (blo[i] + bhi[i]) : 4.f * mid;
-              }
-            }
-          wave_sync();
+          here = kHalf - here;
         }
         flush_all();
       }
@@ -942,25 +871,14 @@ static void launch_wn(WnArgs a, int64_t nrows, int cus, int32_t* ids, float* dis
                      l);
   a.ids_out = ids;
   a.dists_out = dists;
-  // rows in launches of 128k (short kernels); of a launch, whole rounds of
-  // 256-row blocks first, and what is left over in blocks of 128 rows where they
-  // still run all at once (a round of them takes 0.6 of one of 256-row blocks)
-  const int64_t step = 1 << 17;
-  for (int64_t f = 0; f < nrows; f += step) {
-    const int64_t nq = std::min(step, nrows - f);
-    const int64_t blocks = (nq + 255) / 256, rest = blocks % cus;
-    const int64_t n8 = 2 * rest <= cus ? std::min(nq, (blocks - rest) * 256) : nq;
-    a.first = f;
-    a.nq = n8;
-    if (n8 > 0)
-      hipLaunchKernelGGL((knn_whole_kernel<KS, 8>),
-                         dim3((unsigned)std::min<int64_t>((n8 + 255) / 256, cus)), dim3(512), 0, st,
-                         a);
-    a.first = f + n8;
-    a.nq = nq - n8;
-    if (a.nq > 0)
-      hipLaunchKernelGGL((knn_whole_kernel<KS, 4>), dim3((unsigned)((a.nq + 127) / 128)), dim3(256),
-                         0, st, a);
+  for (int i = 0; i < l.launches; ++i) {
+    a.launch = i;
+    a.first = i * kWnStep;
+    a.nq = std::min(kWnStep, nrows - a.first);
+    hipLaunchKernelGGL(
+        knn_whole_kernel<KS>,
+        dim3((unsigned)std::min<int64_t>((a.nq + kWnRows - 1) / kWnRows, kWnPerCu * cus)),
+        dim3(64 * kWnWaves), 0, st, a);
   }
 }
 
