@@ -54,15 +54,6 @@ int hip_fail(rte_ctx* c, hipError_t e, const char* what) {
     if (e_ != hipSuccess) return hip_fail(ctx, e_, what); \
   } while (0)
 
-// s_work is kept for the next call up to 1 GiB (allocating and freeing it took 1 ms
-// of the 4 ms that lists and graph of 160k points take)
-struct WorkGuard {
-  rte_ctx* c;
-  ~WorkGuard() {
-    if (c->s_work.bytes > (size_t)1 << 30) c->s_work.release();  // hipFree waits for the device
-  }
-};
-
 bool is_pow2(int x) { return x > 0 && (x & (x - 1)) == 0; }
 int pow2_ceil(int x) {
   int p = 1;

@@ -12,23 +12,27 @@
 // below the split go left.  Every output depends only on the set of points
 // in a node, never on their order, which the parallel partitions below use.
 //
-// Large nodes (more than kKdSmall points) are split a level at a time:
-//   box       one workgroup per 4096-point chunk of a node, min/max of
-//             order-preserving integer keys of the coordinates, atomics per node
-//   bisection the split-axis coordinates of the level are gathered once into
-//             a contiguous array; every node of the level runs findxM's loop
-//             in lockstep: one counting kernel (chunks, one atomic per
-//             workgroup) and one per-node update kernel per step; the host
-//             stops the steps when no node is left (read back every fourth
-//             step)
-//   partition slots from both ends of the node's segment, one atomic per
-//             side and workgroup
+// Points travel as 16-byte records (three coordinates, id) between two buffers,
+// and the device plans its own work: large nodes (more than kKdSmall points) are
+// split in rounds of five launches on grids of the largest possible size, which
+// the host queues for the expected depth at once and checks afterwards.
+//   count x 3  findxM's loop, four steps a launch: a workgroup per 2048-point
+//              chunk counts its points at or below the 15 midpoints that four
+//              steps can meet; who needs a node's state walks its counts
+//   partition  slots from both ends of the node's segment, one atomic per side
+//              and workgroup; the children's boxes on the way, as order-preserving
+//              integer keys; a node whose search has not ended is carried over
+//   plan       one workgroup makes the next round's nodes of the children, the map
+//              from chunks to nodes and the list of small nodes
+// A round of 1M points takes 30 us; a launch per step, boxes and split-axis values
+// gathered from the rows by id, and a read-back every four steps took 270.
 // Small nodes (at most kKdSmall points) are finished by one workgroup each:
 // ids, coordinates and a local permutation in LDS, an explicit stack of
 // segments, block-wide counts for the bisection.  Left children always come
 // before right children in the index array, so the left-first DFS order of
-// the leaves is the order of their segment starts.  Each leaf's ids are
-// sorted by a bitonic network in LDS to form its pid row.
+// the leaves is the order of their segment starts: starts are marked and counted
+// in order.  Each leaf's ids are sorted by a bitonic network in LDS to form its
+// pid row.
 #include <hip/hip_runtime.h>
 #include <limits.h>
 #include <stdint.h>
@@ -43,16 +47,43 @@ namespace rte {
 namespace {
 
 constexpr int kKdSmall = 2048;   // nodes up to this size: one workgroup in LDS
-constexpr int kKdChunk = 4096;   // points per workgroup in the level kernels
+constexpr int kKdChunk = 2048;   // points per workgroup in the rounds' kernels
 constexpr int kKdMaxIter = 64;   // findxM ends within about 11 steps
+constexpr int kKdSteps = 4;      // of findxM in a launch
+constexpr int kKdPasses = 3;     // launches in a round
+constexpr int kKdMids = (1 << kKdSteps) - 1;
 
 struct LevelNode {
-  int64_t l, r;       // segment [l, r) of the index array
-  int64_t blk0;       // first workgroup of this node in the level grids
-  unsigned key[6];    // ordered keys: min x, y, z, max x, y, z
-  int axis, done;
+  int l, r;               // segment [l, r)
+  int blk0;               // first workgroup of this node in the round's grids
+  int axis, done, steps;  // done: the search has ended, xm is the split
   float bl, br, xm, eps;
-  unsigned cnt, nl, nr, pad;
+  unsigned nl, nr;                         // points left and right of the split
+  unsigned cnt[kKdPasses][kKdMids + 1];    // points at or below midpoint i of a pass
+  unsigned key[2][6];  // children's ordered keys: min x, y, z, max x, y, z
+};
+
+struct Seg {
+  int l, r, buf, pad;  // a small node, in record buffer `buf`
+};
+
+struct Header {
+  int m[2], blocks[2];  // nodes and workgroups, by parity of the round
+  int ns;               // small nodes
+  unsigned err, leaves;
+};
+
+struct KdWork {
+  float4* rec[2];
+  int* idx;    // np: ids in leaf order
+  int* mark;   // np: leaf record + 1 at a leaf's start, 0 elsewhere
+  int* marks;  // marks per chunk
+  LevelNode* nodes[2];
+  int* map[2];  // node of a workgroup
+  Seg* segs;
+  Header* h;
+  int64_t np;
+  int cap;  // of segs and leaves
 };
 
 struct LeafRec {
@@ -73,16 +104,6 @@ __device__ __forceinline__ float funkey(unsigned k) {
 // findxM's midpoint (kdtree.cpp:103-125): the float sum, halved in double
 __device__ __forceinline__ float kd_mid(float l, float r) {
   return (float)((double)(r + l) / 2.0);
-}
-
-__device__ __forceinline__ int node_of_block(const LevelNode* nodes, int m, int64_t b) {
-  int lo = 0, hi = m - 1;
-  while (lo < hi) {
-    const int mid = (lo + hi + 1) >> 1;
-    if (nodes[mid].blk0 <= b) lo = mid;
-    else hi = mid - 1;
-  }
-  return lo;
 }
 
 __device__ __forceinline__ unsigned lanes_below(unsigned long long mask) {
@@ -139,37 +160,52 @@ __device__ __forceinline__ void split_setup(const float lo[3], const float hi[3]
   eps = fmaxf((br - bl) / 1000.0f, 0.00001f);
 }
 
-__global__ void kd_iota_kernel(int* idx, int64_t np) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < np) idx[i] = (int)i;
-}
-
-__global__ void kd_level_init_kernel(LevelNode* nodes, int m, unsigned* act) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < kKdMaxIter) act[i] = 0;
-  if (i >= m) return;
-  LevelNode& n = nodes[i];
-  for (int k = 0; k < 3; ++k) {
-    n.key[k] = 0xffffffffu;
-    n.key[3 + k] = 0u;
+// findxM's state after the steps that the counts of the first `passes` launches
+// decide (kdtree.cpp:111-124)
+struct KdState {
+  float bl, br, xm;
+  int done, steps;
+};
+__device__ __forceinline__ KdState kd_walk(const LevelNode& n, int passes) {
+  KdState s{n.bl, n.br, n.xm, n.done, n.steps};
+  const unsigned half = (unsigned)(n.r - n.l) / 2;
+  for (int p = 0; p < passes; ++p) {
+    int q = 1;  // midpoints as a heap: 2q where the upper half goes, 2q + 1 the lower
+    for (int i = 0; i < kKdSteps && !s.done && s.steps < kKdMaxIter; ++i) {
+      const float mid = kd_mid(s.bl, s.br);
+      const unsigned c = n.cnt[p][q];
+      ++s.steps;
+      if (c <= half) {
+        s.bl = mid;
+        s.xm = mid;
+        if (c == half) s.done = 1;
+        q = 2 * q + 1;
+      } else {
+        s.br = mid;
+        q = 2 * q;
+      }
+      if (!(s.br - s.bl > n.eps)) s.done = 1;
+    }
   }
-  n.cnt = n.nl = n.nr = 0;
-  n.done = 0;
+  return s;
 }
 
-__global__ __launch_bounds__(256) void kd_box_kernel(const float* __restrict__ pts, int64_t stride,
-                                                     const int* __restrict__ idx,
-                                                     LevelNode* nodes, int m) {
+// records of the points; the root's box goes to `root` as a left child's
+__global__ __launch_bounds__(256) void kd_root_kernel(const float* __restrict__ pts, int64_t stride,
+                                                      KdWork w, LevelNode* root) {
   __shared__ unsigned red[6][4];
-  const int nd = node_of_block(nodes, m, blockIdx.x);
-  const int64_t s0 = nodes[nd].l + ((int64_t)blockIdx.x - nodes[nd].blk0) * kKdChunk;
-  const int64_t s1 = min(nodes[nd].r, s0 + kKdChunk);
+  const int64_t s0 = (int64_t)blockIdx.x * kKdChunk, s1 = min(w.np, s0 + kKdChunk);
   unsigned v[6] = {0xffffffffu, 0xffffffffu, 0xffffffffu, 0u, 0u, 0u};
+#pragma unroll 4
   for (int64_t i = s0 + threadIdx.x; i < s1; i += 256) {
-    const float* p = pts + (int64_t)idx[i] * stride;
+    const float* p = pts + i * stride;
+    const float4 c = make_float4(p[0], p[1], p[2], __int_as_float((int)i));
+    w.rec[0][i] = c;
+    w.mark[i] = 0;
+    const float x[3] = {c.x, c.y, c.z};
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
-      const unsigned k = fkey(p[a]);
+      const unsigned k = fkey(x[a]);
       v[a] = min(v[a], k);
       v[3 + a] = max(v[3 + a], k);
     }
@@ -178,112 +214,126 @@ __global__ __launch_bounds__(256) void kd_box_kernel(const float* __restrict__ p
   if (threadIdx.x == 0) {
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
-      atomicMin(&nodes[nd].key[a], v[a]);
-      atomicMax(&nodes[nd].key[3 + a], v[3 + a]);
+      atomicMin(&root->key[0][a], v[a]);
+      atomicMax(&root->key[0][3 + a], v[3 + a]);
     }
   }
 }
 
-__global__ void kd_split_init_kernel(LevelNode* nodes, int m) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= m) return;
-  LevelNode& n = nodes[i];
-  float lo[3], hi[3];
-  for (int a = 0; a < 3; ++a) {
-    lo[a] = funkey(n.key[a]);
-    hi[a] = funkey(n.key[3 + a]);
+// the root as the left child of a node that is done, nothing to its right
+__global__ void kd_start_kernel(KdWork w) {
+  if (threadIdx.x) return;
+  *w.h = Header{};
+  w.h->m[1] = 1;
+  LevelNode& n = w.nodes[1][0];
+  n = LevelNode{};
+  n.r = (int)w.np;
+  n.done = 1;
+  n.nl = (unsigned)w.np;
+  for (int c = 0; c < 2; ++c)
+    for (int k = 0; k < 3; ++k) n.key[c][k] = 0xffffffffu;
+}
+
+// Pass `pass` of a round: points of a chunk at or below each midpoint of the next
+// four steps.  Bound by the launch and three dependent loads.
+__global__ __launch_bounds__(256) void kd_count_kernel(KdWork w, int par, int pass) {
+  if ((int)blockIdx.x >= w.h->blocks[par]) return;
+  LevelNode& n = w.nodes[par][w.map[par][blockIdx.x]];
+  __shared__ unsigned tot[kKdMids + 1];
+  const int t = threadIdx.x;
+  if (t <= kKdMids) tot[t] = 0;
+  const KdState s = kd_walk(n, pass);
+  if (s.done || s.steps >= kKdMaxIter) return;  // all threads
+  float bl[kKdMids + 1], br[kKdMids + 1], mid[kKdMids + 1];
+  bl[1] = s.bl;
+  br[1] = s.br;
+#pragma unroll
+  for (int q = 1; q <= kKdMids; ++q) {
+    mid[q] = kd_mid(bl[q], br[q]);
+    if (2 * q + 1 <= kKdMids) {
+      bl[2 * q] = bl[q];
+      br[2 * q] = mid[q];
+      bl[2 * q + 1] = mid[q];
+      br[2 * q + 1] = br[q];
+    }
   }
-  int axis;
-  float bl, br, xm, eps;
-  split_setup(lo, hi, axis, bl, br, xm, eps);
-  n.axis = axis;
-  n.bl = bl;
-  n.br = br;
-  n.xm = xm;
-  n.eps = eps;
-  n.done = !(br - bl > eps);
-}
-
-// vals[i] = the split-axis coordinate of point idx[i], once per level, so
-// the bisection steps and the partition read it contiguously
-__global__ __launch_bounds__(256) void kd_gather_kernel(const float* __restrict__ pts,
-                                                        int64_t stride,
-                                                        const int* __restrict__ idx,
-                                                        const LevelNode* nodes, int m,
-                                                        float* __restrict__ vals) {
-  const int nd = node_of_block(nodes, m, blockIdx.x);
-  const int axis = nodes[nd].axis;
-  const int64_t s0 = nodes[nd].l + ((int64_t)blockIdx.x - nodes[nd].blk0) * kKdChunk;
-  const int64_t s1 = min(nodes[nd].r, s0 + kKdChunk);
-  for (int64_t i = s0 + threadIdx.x; i < s1; i += 256)
-    vals[i] = pts[(int64_t)idx[i] * stride + axis];
-}
-
-__global__ __launch_bounds__(256) void kd_count_kernel(const float* __restrict__ vals,
-                                                       LevelNode* nodes, int m) {
-  __shared__ unsigned red[4];
-  const int nd = node_of_block(nodes, m, blockIdx.x);
-  if (nodes[nd].done) return;
-  const float mid = kd_mid(nodes[nd].bl, nodes[nd].br);
-  const int64_t s0 = nodes[nd].l + ((int64_t)blockIdx.x - nodes[nd].blk0) * kKdChunk;
-  const int64_t s1 = min(nodes[nd].r, s0 + kKdChunk);
-  unsigned c = 0;
-  for (int64_t i = s0 + threadIdx.x; i < s1; i += 256) c += vals[i] <= mid;
-  c = block_sum(c, red);
-  if (threadIdx.x == 0 && c) atomicAdd(&nodes[nd].cnt, c);
-}
-
-// one findxM step per node (kdtree.cpp:111-124); act counts nodes still going
-__global__ void kd_update_kernel(LevelNode* nodes, int m, unsigned* act) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= m) return;
-  LevelNode& n = nodes[i];
-  if (n.done) return;
-  const float mid = kd_mid(n.bl, n.br);
-  const int64_t half = (n.r - n.l) / 2;
-  const int64_t cnt = n.cnt;
-  n.cnt = 0;
-  if (cnt <= half) {
-    n.bl = mid;
-    n.xm = mid;
-    if (cnt == half) n.done = 1;
-  } else {
-    n.br = mid;
+  const int s0 = n.l + ((int)blockIdx.x - n.blk0) * kKdChunk, s1 = min(n.r, s0 + kKdChunk);
+  const float* x = reinterpret_cast<const float*>(w.rec[par]) + n.axis;
+  constexpr int PER = kKdChunk / 256;
+  float v[PER];
+#pragma unroll
+  for (int k = 0; k < PER; ++k)  // past the end: above every midpoint, or NaN
+    v[k] = s0 + 256 * k + t < s1 ? x[4 * (int64_t)(s0 + 256 * k + t)] : INFINITY;
+  __syncthreads();
+#pragma unroll
+  for (int q = 1; q <= kKdMids; ++q) {
+    unsigned c = 0;
+#pragma unroll
+    for (int k = 0; k < PER; ++k)
+      c += (unsigned)__popcll(__ballot(s0 + 256 * k + t < s1 && v[k] <= mid[q]));
+    if ((t & 63) == 0 && c) atomicAdd(&tot[q], c);
   }
-  if (!n.done && !(n.br - n.bl > n.eps)) n.done = 1;
-  if (!n.done) atomicAdd(act, 1u);
+  __syncthreads();
+  if (t >= 1 && t <= kKdMids && tot[t]) atomicAdd(&n.cnt[pass][t], tot[t]);
 }
 
-// Points of a chunk below the split go to the front of the node's segment,
-// the rest to the back.  Each thread holds its 16 points of the chunk; the
-// workgroup counts both sides, takes its slots with one atomic per side and
-// node, and the waves place their points from per-wave bases.
-__global__ __launch_bounds__(256) void kd_partition_kernel(const float* __restrict__ vals,
-                                                           const int* __restrict__ idx,
-                                                           int* __restrict__ idx2,
-                                                           LevelNode* nodes, int m) {
+// Points of a chunk below the split go to the front of the node's segment in the
+// other buffer, the rest to the back, with their boxes.  The workgroup counts both
+// sides, takes its slots with one atomic per side and node, and the waves place
+// their points from per-wave bases.  Where the search has not ended the points
+// keep their places.
+__global__ __launch_bounds__(256) void kd_partition_kernel(KdWork w, int par) {
+  if ((int)blockIdx.x >= w.h->blocks[par]) return;
   constexpr int PER = kKdChunk / 256;
   __shared__ unsigned cnt_w[2][4];
   __shared__ unsigned base_w[2][4];
+  __shared__ unsigned red[6][4];
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-  const int nd = node_of_block(nodes, m, blockIdx.x);
-  const int64_t l = nodes[nd].l, r = nodes[nd].r;
-  const float xm = nodes[nd].xm;
-  const int64_t s0 = l + ((int64_t)blockIdx.x - nodes[nd].blk0) * kKdChunk;
-  const int64_t s1 = min(r, s0 + kKdChunk);
-  int id[PER];
+  LevelNode& n = w.nodes[par][w.map[par][blockIdx.x]];
+  const int l = n.l, r = n.r;
+  const int s0 = l + ((int)blockIdx.x - n.blk0) * kKdChunk, s1 = min(r, s0 + kKdChunk);
+  const float4* in = w.rec[par];
+  float4* out = w.rec[par ^ 1];
+  const KdState s = kd_walk(n, kKdPasses);
+  float4 p[PER];
+#pragma unroll
+  for (int k = 0; k < PER; ++k) {
+    const int i = s0 + 256 * k + t;
+    p[k] = i < s1 ? in[i] : make_float4(0.f, 0.f, 0.f, 0.f);
+  }
+  if (!s.done) {
+#pragma unroll
+    for (int k = 0; k < PER; ++k)
+      if (s0 + 256 * k + t < s1) out[s0 + 256 * k + t] = p[k];
+    return;  // all threads
+  }
+  const int axis = n.axis;
+  unsigned v[2][6];
+  for (int c = 0; c < 2; ++c)
+    for (int k = 0; k < 6; ++k) v[c][k] = k < 3 ? 0xffffffffu : 0u;
   unsigned lmask = 0, vmask = 0;  // bit k: element k is valid / goes left
   unsigned nl = 0, nr = 0;        // this wave's counts (uniform)
 #pragma unroll
   for (int k = 0; k < PER; ++k) {
-    const int64_t i = s0 + 256 * k + t;
-    const bool valid = i < s1;
-    id[k] = valid ? idx[i] : 0;
-    const bool left = valid && vals[i] < xm;
+    const bool valid = s0 + 256 * k + t < s1;
+    const float x[3] = {p[k].x, p[k].y, p[k].z};
+    const float xa = axis == 0 ? x[0] : axis == 1 ? x[1] : x[2];
+    const bool left = valid && xa < s.xm;
     vmask |= (unsigned)valid << k;
     lmask |= (unsigned)left << k;
     nl += (unsigned)__popcll(__ballot(left));
     nr += (unsigned)__popcll(__ballot(valid && !left));
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+      const unsigned key = fkey(x[a]);
+      if (left) {
+        v[0][a] = min(v[0][a], key);
+        v[0][3 + a] = max(v[0][3 + a], key);
+      } else if (valid) {
+        v[1][a] = min(v[1][a], key);
+        v[1][3 + a] = max(v[1][3 + a], key);
+      }
+    }
   }
   if (lane == 0) {
     cnt_w[0][wave] = nl;
@@ -293,44 +343,172 @@ __global__ __launch_bounds__(256) void kd_partition_kernel(const float* __restri
   if (t == 0) {
     const unsigned tl = cnt_w[0][0] + cnt_w[0][1] + cnt_w[0][2] + cnt_w[0][3];
     const unsigned tr = cnt_w[1][0] + cnt_w[1][1] + cnt_w[1][2] + cnt_w[1][3];
-    unsigned bl = tl ? atomicAdd(&nodes[nd].nl, tl) : 0u;
-    unsigned br = tr ? atomicAdd(&nodes[nd].nr, tr) : 0u;
-    for (int w = 0; w < 4; ++w) {
-      base_w[0][w] = bl;
-      base_w[1][w] = br;
-      bl += cnt_w[0][w];
-      br += cnt_w[1][w];
+    unsigned bl = tl ? atomicAdd(&n.nl, tl) : 0u;
+    unsigned br = tr ? atomicAdd(&n.nr, tr) : 0u;
+    for (int i = 0; i < 4; ++i) {
+      base_w[0][i] = bl;
+      base_w[1][i] = br;
+      bl += cnt_w[0][i];
+      br += cnt_w[1][i];
     }
   }
-  __syncthreads();
+#pragma unroll
+  for (int c = 0; c < 2; ++c) {
+    block_minmax6(v[c], red);
+    if (t < 6) {  // v is the same in all threads
+      unsigned x = v[c][0];
+#pragma unroll
+      for (int k = 1; k < 6; ++k) x = t == k ? v[c][k] : x;
+      if (t < 3) atomicMin(&n.key[c][t], x);
+      else atomicMax(&n.key[c][t], x);
+    }
+  }
   unsigned ol = base_w[0][wave], orr = base_w[1][wave];
 #pragma unroll
   for (int k = 0; k < PER; ++k) {
     const bool valid = (vmask >> k) & 1u, left = (lmask >> k) & 1u;
     const unsigned long long ml = __ballot(left), mr = __ballot(valid && !left);
-    if (left) idx2[l + ol + lanes_below(ml)] = id[k];
-    if (valid && !left) idx2[r - 1 - (int64_t)(orr + lanes_below(mr))] = id[k];
+    if (left) out[l + ol + lanes_below(ml)] = p[k];
+    if (valid && !left) out[r - 1 - (int)(orr + lanes_below(mr))] = p[k];
     ol += (unsigned)__popcll(ml);
     orr += (unsigned)__popcll(mr);
   }
 }
 
-__global__ __launch_bounds__(256) void kd_copy_kernel(const int* __restrict__ idx2,
-                                                      int* __restrict__ idx,
-                                                      const LevelNode* nodes, int m) {
-  const int nd = node_of_block(nodes, m, blockIdx.x);
-  const int64_t s0 = nodes[nd].l + ((int64_t)blockIdx.x - nodes[nd].blk0) * kKdChunk;
-  const int64_t s1 = min(nodes[nd].r, s0 + kKdChunk);
-  for (int64_t i = s0 + threadIdx.x; i < s1; i += 256) idx[i] = idx2[i];
+// The next round's nodes: children of nodes that are done, and those that are not.
+// One workgroup; nodes of the round `par` to the other parity.
+__global__ __launch_bounds__(1024) void kd_plan_kernel(KdWork w, int par) {
+  __shared__ int sn[1024], sb[1024];
+  __shared__ int nseg;
+  const int t = threadIdx.x, m = w.h->m[par];
+  int base_n = 0, base_b = 0;
+  if (t == 0) nseg = w.h->ns;
+  for (int i0 = 0; i0 < m; i0 += 1024) {
+    LevelNode c[2];
+    int large = 0, blocks = 0;
+    if (i0 + t < m) {
+      const LevelNode& n = w.nodes[par][i0 + t];
+      const KdState s = kd_walk(n, kKdPasses);
+      if (!s.done) {
+        if (s.steps >= kKdMaxIter) {
+          atomicOr(&w.h->err, 2u);
+        } else {
+          c[0] = n;
+          c[0].bl = s.bl;
+          c[0].br = s.br;
+          c[0].xm = s.xm;
+          c[0].steps = s.steps;
+          large = 1;
+        }
+      } else {
+        const int mid = n.l + (int)n.nl;
+        if ((mid == n.l || mid == n.r) && n.axis >= 0 && n.eps > 0.f) atomicOr(&w.h->err, 1u);
+        else
+          for (int k = 0; k < 2; ++k) {
+            const int l = k ? mid : n.l, r = k ? n.r : mid;
+            if (r - l > kKdSmall) {
+              LevelNode& d = c[large++];
+              d.l = l;
+              d.r = r;
+              float lo[3], hi[3];
+              for (int a = 0; a < 3; ++a) {
+                lo[a] = funkey(n.key[k][a]);
+                hi[a] = funkey(n.key[k][3 + a]);
+              }
+              split_setup(lo, hi, d.axis, d.bl, d.br, d.xm, d.eps);
+              d.done = !(d.br - d.bl > d.eps);
+              d.steps = 0;
+            } else if (r > l) {
+              const int at = atomicAdd(&nseg, 1);
+              if (at < w.cap) w.segs[at] = Seg{l, r, par ^ 1, 0};
+            }
+          }
+      }
+      for (int k = 0; k < large; ++k) blocks += (c[k].r - c[k].l + kKdChunk - 1) / kKdChunk;
+    }
+    __syncthreads();
+    sn[t] = large;
+    sb[t] = blocks;
+    __syncthreads();
+    for (int o = 1; o < 1024; o <<= 1) {
+      const int x = t >= o ? sn[t - o] : 0, y = t >= o ? sb[t - o] : 0;
+      __syncthreads();
+      sn[t] += x;
+      sb[t] += y;
+      __syncthreads();
+    }
+    int at = base_n + sn[t] - large, b = base_b + sb[t] - blocks;
+    for (int k = 0; k < large; ++k) {
+      LevelNode& d = c[k];
+      d.blk0 = b;
+      d.nl = d.nr = 0;
+      for (int p = 0; p < kKdPasses; ++p)
+        for (int q = 0; q <= kKdMids; ++q) d.cnt[p][q] = 0;
+      for (int e = 0; e < 2; ++e)
+        for (int a = 0; a < 6; ++a) d.key[e][a] = a < 3 ? 0xffffffffu : 0u;
+      w.nodes[par ^ 1][at] = d;
+      for (int j = (d.r - d.l + kKdChunk - 1) / kKdChunk; j > 0; --j) w.map[par ^ 1][b++] = at;
+      ++at;
+    }
+    base_n += sn[1023];
+    base_b += sb[1023];
+  }
+  __syncthreads();
+  if (t == 0) {
+    w.h->m[par ^ 1] = base_n;
+    w.h->blocks[par ^ 1] = base_b;
+    w.h->ns = nseg;
+    if (nseg > w.cap) atomicOr(&w.h->err, 4u);
+  }
+}
+
+// marks of a chunk
+__global__ __launch_bounds__(256) void kd_mark_kernel(KdWork w) {
+  __shared__ unsigned red[4];
+  const int64_t s0 = (int64_t)blockIdx.x * kKdChunk, s1 = min(w.np, s0 + kKdChunk);
+  unsigned c = 0;
+  for (int64_t i = s0 + threadIdx.x; i < s1; i += 256) c += w.mark[i] != 0;
+  c = block_sum(c, red);
+  if (threadIdx.x == 0) w.marks[blockIdx.x] = (int)c;
+}
+
+// leaves in the order of their starts
+__global__ __launch_bounds__(256) void kd_order_kernel(KdWork w, const LeafRec* __restrict__ leaves,
+                                                       int* __restrict__ start,
+                                                       int* __restrict__ count,
+                                                       float* __restrict__ boxes) {
+  __shared__ unsigned red[4];
+  __shared__ unsigned wsum[4];
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  unsigned before = 0;
+  for (int i = t; i < (int)blockIdx.x; i += 256) before += (unsigned)w.marks[i];
+  before = block_sum(before, red);
+  const int64_t s0 = (int64_t)blockIdx.x * kKdChunk, s1 = min(w.np, s0 + kKdChunk);
+  for (int64_t i0 = s0; i0 < s1; i0 += 256) {  // 256 in a row at a time
+    const int64_t i = i0 + t;
+    const int k = i < s1 ? w.mark[i] : 0;
+    const unsigned long long mk = __ballot(k != 0);
+    if (lane == 0) wsum[wave] = (unsigned)__popcll(mk);
+    __syncthreads();
+    unsigned at = before + lanes_below(mk);
+    for (int x = 0; x < 4; ++x) {
+      if (x < wave) at += wsum[x];
+      before += wsum[x];
+    }
+    if (k) {
+      const LeafRec& rec = leaves[k - 1];
+      start[at] = (int)i;
+      count[at] = rec.cnt;
+      for (int b = 0; b < 6; ++b) boxes[(int64_t)at * 6 + b] = rec.box[b];
+    }
+    __syncthreads();
+  }
 }
 
 // err bits: 1 = split failed, 2 = findxM did not end, 4 = leaf capacity
-__global__ __launch_bounds__(256) void kd_small_kernel(const float* __restrict__ pts,
-                                                       int64_t stride, int* __restrict__ idx,
-                                                       const int64_t* __restrict__ segs,
-                                                       int max_node, LeafRec* __restrict__ leaves,
-                                                       unsigned* leaf_ctr, int max_leaves,
-                                                       unsigned* err) {
+__global__ __launch_bounds__(256) void kd_small_kernel(KdWork w, int max_node,
+                                                       LeafRec* __restrict__ leaves,
+                                                       int max_leaves) {
   __shared__ int ids[kKdSmall];
   __shared__ float cs[3][kKdSmall];
   __shared__ uint16_t perm[2][kKdSmall];
@@ -338,15 +516,16 @@ __global__ __launch_bounds__(256) void kd_small_kernel(const float* __restrict__
   __shared__ unsigned red[6][4];
   __shared__ unsigned cnts[2];
   const int t = threadIdx.x;
-  const int64_t l = segs[2 * blockIdx.x];
-  const int n = (int)(segs[2 * blockIdx.x + 1] - l);
+  const Seg sg = w.segs[blockIdx.x];
+  const int l = sg.l, n = sg.r - sg.l;
+  int* const idx = w.idx;
+  unsigned* const err = &w.h->err;
   for (int j = t; j < n; j += 256) {
-    const int id = idx[l + j];
-    ids[j] = id;
-    const float* p = pts + (int64_t)id * stride;
-    cs[0][j] = p[0];
-    cs[1][j] = p[1];
-    cs[2][j] = p[2];
+    const float4 p = w.rec[sg.buf][l + j];
+    ids[j] = __float_as_int(p.w);
+    cs[0][j] = p.x;
+    cs[1][j] = p.y;
+    cs[2][j] = p.z;
     perm[0][j] = (uint16_t)j;
   }
   if (t == 0) stack[0] = (unsigned)n;
@@ -374,9 +553,10 @@ __global__ __launch_bounds__(256) void kd_small_kernel(const float* __restrict__
     }
     if (cnt <= max_node) {  // leaf (kdtree.cpp:171-174)
       if (t == 0) {
-        const unsigned s = atomicAdd(leaf_ctr, 1u);
+        const unsigned s = atomicAdd(&w.h->leaves, 1u);
         if (s < (unsigned)max_leaves) {
           LeafRec& rec = leaves[s];
+          w.mark[l + a] = (int)s + 1;
           rec.start = l + a;
           rec.cnt = cnt;
           rec.pad = 0;
@@ -452,7 +632,7 @@ __global__ __launch_bounds__(256) void kd_small_kernel(const float* __restrict__
 
 // pid row of leaf i: its ids ascending, padded with np (kdtree.cpp:91-101)
 __global__ __launch_bounds__(256) void kd_pids_kernel(const int* __restrict__ idx,
-                                                      const int64_t* __restrict__ start,
+                                                      const int* __restrict__ start,
                                                       const int* __restrict__ count, int max_node,
                                                       int P, int64_t np,
                                                       int32_t* __restrict__ pids) {
@@ -480,8 +660,6 @@ __global__ __launch_bounds__(256) void kd_pids_kernel(const int* __restrict__ id
   for (int j = threadIdx.x; j < max_node; j += 256)
     pids[(int64_t)leaf * max_node + j] = j < cnt ? s[j] : (int32_t)np;
 }
-
-unsigned blocks_1d(int64_t n, int b) { return (unsigned)((n + b - 1) / b); }
 
 }  // namespace
 
@@ -511,7 +689,7 @@ int rte_build_kdtree_gpu(rte_ctx* c, const float* pts, int64_t np, int64_t strid
   do {                                  \
     if (int r_ = ck((expr), what)) return r_; \
   } while (0)
-  DevBuf pin, idxb, idx2b, valsb, nodesb, actb, segb, leafb, ctrb, ordb, pidb;
+  DevBuf pin, outb;
   const float* dp = pts;
   int64_t ds = stride;
   if (where == RTE_HOST) {  // only the three coordinates travel
@@ -525,143 +703,100 @@ int rte_build_kdtree_gpu(rte_ctx* c, const float* pts, int64_t np, int64_t strid
     dp = pin.as<float>();
     ds = 3;
   }
-  KCK(idxb.reserve((size_t)np * 4), "hipMalloc");
-  KCK(idx2b.reserve((size_t)np * 4), "hipMalloc");
-  KCK(valsb.reserve((size_t)np * 4), "hipMalloc");
-  float* vals = valsb.as<float>();
-  KCK(actb.reserve(kKdMaxIter * sizeof(unsigned)), "hipMalloc");
-  KCK(ctrb.reserve(2 * sizeof(unsigned)), "hipMalloc");
-  int* idx = idxb.as<int>();
-  int* idx2 = idx2b.as<int>();
-  unsigned* act = actb.as<unsigned>();
-  hipLaunchKernelGGL(kd_iota_kernel, dim3(blocks_1d(np, 256)), dim3(256), 0, st, idx, np);
-
-  std::vector<std::pair<int64_t, int64_t>> level, small;
-  (np <= kKdSmall ? small : level).push_back({0, np});
-  std::vector<LevelNode> hn;
-  while (!level.empty()) {
-    const int m = (int)level.size();
-    hn.assign(m, LevelNode{});
-    int64_t blocks = 0;
-    for (int i = 0; i < m; ++i) {
-      hn[i].l = level[i].first;
-      hn[i].r = level[i].second;
-      hn[i].blk0 = blocks;
-      blocks += (hn[i].r - hn[i].l + kKdChunk - 1) / kKdChunk;
+  // leaves and small nodes: no more than points
+  const int cap = (int)std::min<int64_t>(max_leaves, np);
+  const int64_t chunks = (np + kKdChunk - 1) / kKdChunk;
+  const int64_t max_nodes = np / (kKdSmall + 1) + 1, max_blocks = np / kKdChunk + max_nodes;
+  KdWork w{};
+  LeafRec* leaves = nullptr;
+  int *dstart = nullptr, *dcount = nullptr;
+  auto lay = [&](char* base) {
+    size_t at = 0;
+    auto take = [&](auto*& p, size_t n) {
+      p = reinterpret_cast<std::remove_reference_t<decltype(p)>>(base + at);
+      at = (at + n * sizeof(*p) + 255) & ~(size_t)255;
+    };
+    for (int i = 0; i < 2; ++i) {
+      take(w.rec[i], np);
+      take(w.nodes[i], max_nodes);
+      take(w.map[i], max_blocks);
     }
-    if (blocks > INT_MAX) return rte_fail(c, RTE_EINVAL, "kd-tree level too large");
-    KCK(nodesb.reserve((size_t)m * sizeof(LevelNode)), "hipMalloc");
-    LevelNode* nodes = nodesb.as<LevelNode>();
-    KCK(hipMemcpyAsync(nodes, hn.data(), (size_t)m * sizeof(LevelNode), hipMemcpyHostToDevice, st),
-        "copy");
-    const unsigned gm = blocks_1d(std::max(m, kKdMaxIter), 256);
-    hipLaunchKernelGGL(kd_level_init_kernel, dim3(gm), dim3(256), 0, st, nodes, m, act);
-    hipLaunchKernelGGL(kd_box_kernel, dim3((unsigned)blocks), dim3(256), 0, st, dp, ds, idx, nodes,
-                       m);
-    hipLaunchKernelGGL(kd_split_init_kernel, dim3(gm), dim3(256), 0, st, nodes, m);
-    hipLaunchKernelGGL(kd_gather_kernel, dim3((unsigned)blocks), dim3(256), 0, st, dp, ds, idx,
-                       nodes, m, vals);
-    bool converged = false;
-    for (int it = 0; it < kKdMaxIter; ++it) {
-      hipLaunchKernelGGL(kd_count_kernel, dim3((unsigned)blocks), dim3(256), 0, st, vals, nodes,
-                         m);
-      hipLaunchKernelGGL(kd_update_kernel, dim3(gm), dim3(256), 0, st, nodes, m, act + it);
-      if ((it & 3) == 3 || it == kKdMaxIter - 1) {
-        unsigned left = 0;
-        KCK(hipMemcpyAsync(&left, act + it, sizeof(unsigned), hipMemcpyDeviceToHost, st), "copy");
-        KCK(hipStreamSynchronize(st), "sync");
-        if (left == 0) {
-          converged = true;
-          break;
-        }
-      }
+    take(w.idx, np);
+    take(w.mark, np);
+    take(w.marks, chunks);
+    take(w.segs, cap);
+    take(w.h, 1);
+    take(leaves, cap);
+    take(dstart, cap);
+    take(dcount, cap);
+    return at;
+  };
+  KCK(c->s_work.reserve(lay(nullptr)), "hipMalloc(kd-tree work)");
+  WorkGuard guard{c};
+  lay(c->s_work.as<char>());
+  w.np = np;
+  w.cap = cap;
+  hipLaunchKernelGGL(kd_start_kernel, dim3(1), dim3(64), 0, st, w);
+  hipLaunchKernelGGL(kd_root_kernel, dim3((unsigned)chunks), dim3(256), 0, st, dp, ds, w,
+                     w.nodes[1]);
+  // the root's plan, then rounds: two more than halving takes, one of them empty
+  // as a rule, and then two at a time while nodes are left
+  hipLaunchKernelGGL(kd_plan_kernel, dim3(1), dim3(1024), 0, st, w, 1);
+  int rounds = 0;
+  for (int64_t n = np; n > kKdSmall; n = (n + 1) / 2) ++rounds;
+  if (rounds) ++rounds;
+  Header hh{};
+  for (int r = 0;; ++r) {
+    const int par = r & 1;
+    if (r >= rounds) {
+      KCK(hipGetLastError(), "kd-tree kernels");
+      KCK(hipMemcpyAsync(&hh, w.h, sizeof hh, hipMemcpyDeviceToHost, st), "copy");
+      KCK(hipStreamSynchronize(st), "sync");
+      if (hh.err & 1u) return rte_fail(c, RTE_EBUILD, "kd-tree split failed");
+      if (hh.err & 2u) return rte_fail(c, RTE_EBUILD, "kd-tree split search did not end");
+      if (hh.err & 4u) break;
+      if (hh.m[par] == 0) break;
+      rounds = r + 2;
     }
-    if (!converged) return rte_fail(c, RTE_EBUILD, "kd-tree split search did not end");
-    hipLaunchKernelGGL(kd_partition_kernel, dim3((unsigned)blocks), dim3(256), 0, st, vals, idx,
-                       idx2, nodes, m);
-    hipLaunchKernelGGL(kd_copy_kernel, dim3((unsigned)blocks), dim3(256), 0, st, idx2, idx, nodes,
-                       m);
-    KCK(hipGetLastError(), "kd-tree level kernels");
-    KCK(hipMemcpyAsync(hn.data(), nodes, (size_t)m * sizeof(LevelNode), hipMemcpyDeviceToHost, st),
-        "copy");
+    for (int p = 0; p < kKdPasses; ++p)
+      hipLaunchKernelGGL(kd_count_kernel, dim3((unsigned)max_blocks), dim3(256), 0, st, w, par, p);
+    hipLaunchKernelGGL(kd_partition_kernel, dim3((unsigned)max_blocks), dim3(256), 0, st, w, par);
+    hipLaunchKernelGGL(kd_plan_kernel, dim3(1), dim3(1024), 0, st, w, par);
+  }
+  if (!(hh.err & 4u)) {
+    // boxes straight to the caller where it can hold all there may be
+    KCK(outb.reserve(where == RTE_HOST ? (size_t)cap * 24 : 1), "hipMalloc");
+    float* boxes = where == RTE_HOST ? outb.as<float>() : aabbs_out;
+    hipLaunchKernelGGL(kd_small_kernel, dim3((unsigned)hh.ns), dim3(256), 0, st, w, max_node,
+                       leaves, max_leaves);
+    hipLaunchKernelGGL(kd_mark_kernel, dim3((unsigned)chunks), dim3(256), 0, st, w);
+    hipLaunchKernelGGL(kd_order_kernel, dim3((unsigned)chunks), dim3(256), 0, st, w, leaves, dstart,
+                       dcount, boxes);
+    KCK(hipGetLastError(), "kd_small_kernel");
+    KCK(hipMemcpyAsync(&hh, w.h, sizeof hh, hipMemcpyDeviceToHost, st), "copy");
     KCK(hipStreamSynchronize(st), "sync");
-    std::vector<std::pair<int64_t, int64_t>> next;
-    for (int i = 0; i < m; ++i) {
-      const int64_t l = hn[i].l, r = hn[i].r, mid = l + hn[i].nl;
-      if (mid == l || mid == r) return rte_fail(c, RTE_EBUILD, "kd-tree split failed");
-      for (auto ch : {std::make_pair(l, mid), std::make_pair(mid, r)})
-        (ch.second - ch.first <= kKdSmall ? small : next).push_back(ch);
-    }
-    level.swap(next);
   }
-
-  // small nodes and leaves
-  const int ns = (int)small.size();
-  KCK(segb.reserve((size_t)ns * 2 * sizeof(int64_t)), "hipMalloc");
-  KCK(leafb.reserve((size_t)max_leaves * sizeof(LeafRec)), "hipMalloc");
-  std::vector<int64_t> segs((size_t)ns * 2);
-  for (int i = 0; i < ns; ++i) {
-    segs[2 * i] = small[i].first;
-    segs[2 * i + 1] = small[i].second;
-  }
-  KCK(hipMemcpyAsync(segb.p, segs.data(), segs.size() * sizeof(int64_t), hipMemcpyHostToDevice, st),
-      "copy");
-  KCK(hipMemsetAsync(ctrb.p, 0, 2 * sizeof(unsigned), st), "memset");
-  unsigned* leaf_ctr = ctrb.as<unsigned>();
-  hipLaunchKernelGGL(kd_small_kernel, dim3(ns), dim3(256), 0, st, dp, ds, idx,
-                     segb.as<int64_t>(), max_node, leafb.as<LeafRec>(), leaf_ctr, max_leaves,
-                     leaf_ctr + 1);
-  KCK(hipGetLastError(), "kd_small_kernel");
-  unsigned hc[2];
-  KCK(hipMemcpyAsync(hc, ctrb.p, sizeof(hc), hipMemcpyDeviceToHost, st), "copy");
-  KCK(hipStreamSynchronize(st), "sync");
-  if (hc[1] & 1u) return rte_fail(c, RTE_EBUILD, "kd-tree split failed");
-  if (hc[1] & 2u) return rte_fail(c, RTE_EBUILD, "kd-tree split search did not end");
-  if ((hc[1] & 4u) || hc[0] > (unsigned)max_leaves)
+  if (hh.err & 1u) return rte_fail(c, RTE_EBUILD, "kd-tree split failed");
+  if (hh.err & 2u) return rte_fail(c, RTE_EBUILD, "kd-tree split search did not end");
+  if ((hh.err & 4u) || hh.leaves > (unsigned)max_leaves)
     return rte_fail(c, RTE_EINVAL, "kd-tree: more than max_leaves=%d leaves", max_leaves);
-  const int nl = (int)hc[0];
-  std::vector<LeafRec> recs(nl);
-  KCK(hipMemcpyAsync(recs.data(), leafb.p, (size_t)nl * sizeof(LeafRec), hipMemcpyDeviceToHost,
-                     st),
-      "copy");
-  KCK(hipStreamSynchronize(st), "sync");
-  std::sort(recs.begin(), recs.end(),
-            [](const LeafRec& x, const LeafRec& y) { return x.start < y.start; });
-  std::vector<float> boxes((size_t)nl * 6);
-  std::vector<int64_t> starts(nl);
-  std::vector<int> counts(nl);
-  for (int i = 0; i < nl; ++i) {
-    std::copy(recs[i].box, recs[i].box + 6, boxes.begin() + (size_t)i * 6);
-    starts[i] = recs[i].start;
-    counts[i] = recs[i].cnt;
-  }
-  KCK(ordb.reserve((size_t)nl * (sizeof(int64_t) + sizeof(int))), "hipMalloc");
-  int64_t* dstart = ordb.as<int64_t>();
-  int* dcount = reinterpret_cast<int*>(dstart + nl);
-  KCK(hipMemcpyAsync(dstart, starts.data(), (size_t)nl * sizeof(int64_t), hipMemcpyHostToDevice,
-                     st),
-      "copy");
-  KCK(hipMemcpyAsync(dcount, counts.data(), (size_t)nl * sizeof(int), hipMemcpyHostToDevice, st),
-      "copy");
+  const int nl = (int)hh.leaves;
   int P = 1;
   while (P < max_node) P <<= 1;
   int32_t* dpids = pids_out;
+  DevBuf pidb;
   if (where == RTE_HOST) {
     KCK(pidb.reserve((size_t)nl * max_node * sizeof(int32_t)), "hipMalloc");
     dpids = pidb.as<int32_t>();
   }
-  hipLaunchKernelGGL(kd_pids_kernel, dim3(nl), dim3(256), 0, st, idx, dstart, dcount, max_node, P,
+  hipLaunchKernelGGL(kd_pids_kernel, dim3(nl), dim3(256), 0, st, w.idx, dstart, dcount, max_node, P,
                      np, dpids);
   KCK(hipGetLastError(), "kd_pids_kernel");
   if (where == RTE_HOST) {
     KCK(hipMemcpyAsync(pids_out, dpids, (size_t)nl * max_node * sizeof(int32_t),
                        hipMemcpyDeviceToHost, st),
         "copy");
-    std::copy(boxes.begin(), boxes.end(), aabbs_out);
-  } else {
-    KCK(hipMemcpyAsync(aabbs_out, boxes.data(), boxes.size() * sizeof(float),
-                       hipMemcpyHostToDevice, st),
-        "copy");
+    KCK(hipMemcpyAsync(aabbs_out, outb.p, (size_t)nl * 24, hipMemcpyDeviceToHost, st), "copy");
   }
   KCK(hipStreamSynchronize(st), "sync");
 #undef KCK

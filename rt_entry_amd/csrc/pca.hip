@@ -481,7 +481,7 @@ int rte_pca_fit(rte_ctx* c, const float* X, int64_t n, int d, int64_t stride, fl
   auto ck = [&](hipError_t e, const char* what) {
     return e == hipSuccess ? RTE_OK : rte_fail(c, RTE_EHIP, "%s: %s", what, hipGetErrorString(e));
   };
-  DevBuf xin, part, mean, cov;
+  DevBuf xin;
   const float* dx = X;
   if (where == RTE_HOST) {
     const size_t bytes = ((size_t)(n - 1) * stride + d) * sizeof(float);
@@ -500,26 +500,29 @@ int rte_pca_fit(rte_ctx* c, const float* X, int64_t n, int d, int64_t stride, fl
   const int nb = (int)std::min<int64_t>(std::max(1, (2 * cus + ntp - 1) / ntp), by_rows);
   const int64_t rpb_sum = (n + nb_sum - 1) / nb_sum, rpb = (n + nb - 1) / nb;
   const size_t dd = (size_t)d * d;
-  if (int r = ck(part.reserve(std::max((size_t)nb * dd, (size_t)nb_sum * d) * sizeof(double)),
-                 "hipMalloc(pca partials)"))
+  // covariance | mean | partials
+  const size_t part_n = std::max((size_t)nb * dd, (size_t)nb_sum * d);
+  if (int r = ck(c->s_work.reserve((dd + d + part_n) * sizeof(double)), "hipMalloc(pca work)"))
     return r;
-  if (int r = ck(mean.reserve((size_t)d * sizeof(double)), "hipMalloc")) return r;
-  if (int r = ck(cov.reserve(dd * sizeof(double)), "hipMalloc")) return r;
+  WorkGuard guard{c};
+  double* cov = c->s_work.as<double>();
+  double* mean = cov + dd;
+  double* part = mean + d;
   // whole waves of columns, and no more
   hipLaunchKernelGGL(rte::col_sum_kernel, dim3(nb_sum), dim3(std::min(256, (d + 63) / 64 * 64)), 0,
                      st, dx, n, d, stride,
-                     rpb_sum, part.as<double>());
+                     rpb_sum, part);
   hipLaunchKernelGGL(rte::col_mean_kernel, dim3((d + 127) / 128), dim3(128), 0, st,
-                     part.as<double>(), nb_sum, d, n, mean.as<double>());
+                     part, nb_sum, d, n, mean);
   hipLaunchKernelGGL(rte::cov_partial_kernel, dim3(nb, ntp), dim3(256), 0, st, dx, n, d, stride,
-                     mean.as<double>(), rpb, nt, part.as<double>());
+                     mean, rpb, nt, part);
   hipLaunchKernelGGL(rte::cov_reduce_kernel, dim3((unsigned)((dd + 255) / 256)), dim3(256), 0, st,
-                     part.as<double>(), nb, d, n, cov.as<double>());
+                     part, nb, d, n, cov);
   if (int r = ck(hipGetLastError(), "pca kernels")) return r;
   std::vector<double> C(dd), mu(d);
-  if (int r = ck(hipMemcpyAsync(C.data(), cov.p, dd * 8, hipMemcpyDeviceToHost, st), "copy"))
+  if (int r = ck(hipMemcpyAsync(C.data(), cov, dd * 8, hipMemcpyDeviceToHost, st), "copy"))
     return r;
-  if (int r = ck(hipMemcpyAsync(mu.data(), mean.p, (size_t)d * 8, hipMemcpyDeviceToHost, st),
+  if (int r = ck(hipMemcpyAsync(mu.data(), mean, (size_t)d * 8, hipMemcpyDeviceToHost, st),
                  "copy"))
     return r;
   if (int r = ck(hipStreamSynchronize(st), "sync")) return r;
@@ -559,7 +562,7 @@ int rte_pca_rotate(rte_ctx* c, const float* X, int64_t n, int d, int64_t stride,
   };
   if ((n + 15) / 16 > 0x7fffffff)
     return rte_fail(c, RTE_EUNSUP, "pca_rotate: too many rows");
-  DevBuf xin, rm, ob;
+  DevBuf xin, ob;
   const float* dx = X;
   float* dout = out;
   const size_t xbytes = ((size_t)(n - 1) * stride + d) * sizeof(float);
@@ -574,10 +577,12 @@ int rte_pca_rotate(rte_ctx* c, const float* X, int64_t n, int d, int64_t stride,
   // R (d x d_out) and mu (d) are host arrays; R widened comes first
   const int ldr = (d_out + rte::kRotCols - 1) / rte::kRotCols * rte::kRotCols;
   const size_t wide = (size_t)(d + 1) * ldr;
-  if (int r = ck(rm.reserve(wide * sizeof(double) + ((size_t)d * d_out + d) * sizeof(float)),
+  if (int r = ck(c->s_work.reserve(wide * sizeof(double) +
+                                   ((size_t)d * d_out + d) * sizeof(float)),
                  "hipMalloc"))
     return r;
-  double* dW = rm.as<double>();
+  WorkGuard guard{c};
+  double* dW = c->s_work.as<double>();
   float* dR = reinterpret_cast<float*>(dW + wide);
   float* dmu = dR + (size_t)d * d_out;
   if (int r = ck(hipMemcpyAsync(dR, R, (size_t)d * d_out * 4, hipMemcpyHostToDevice, st), "copy"))
