@@ -151,17 +151,67 @@ struct Gemm {
   float* out;
   uint16_t* out16;
 };
+// Column sums of three n x C matrices (the bias gradients), 64 columns per
+// workgroup, in the first workgroups of the weight gradients' launch.  Each column
+// is summed by one thread over the rows in ascending order, so the sums do not
+// depend on the launch; the four waves stage ROWS rows at a time in LDS, the next
+// rows' loads in flight while the first wave adds.  Bound by that chain of
+// additions (n of them) and the stages' round trips: 12 us at n = 1024 in a launch
+// of their own, hidden beside the products' 15.
+struct ColSums {
+  const float* x[3];
+  float* out[3];
+  int C[3];
+  int n;
+  int blocks;  // workgroups; 0: none
+};
+template <int ROWS>
+__device__ __forceinline__ void colsum_block(const ColSums& a, int blk, float (*rows)[64]) {
+  constexpr int kPer = ROWS / 4;
+  int p = 0;
+  while (p < 2 && blk >= (a.C[p] + 63) / 64) blk -= (a.C[p++] + 63) / 64;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int C = a.C[p], n = a.n;
+  const int c = blk * 64 + lane;
+  const float* x = a.x[p] + min(c, C - 1);
+  float v[kPer];
+  auto load = [&](int r0) {  // at clamped, valid rows; the sum stops at n
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) v[i] = x[(int64_t)min(r0 + 4 * i + wave, n - 1) * C];
+  };
+  load(0);
+  float s = 0.f;
+  for (int r0 = 0; r0 < n; r0 += ROWS) {
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) rows[4 * i + wave][lane] = v[i];
+    __syncthreads();
+    if (r0 + ROWS < n) load(r0 + ROWS);
+    if (wave == 0) {
+      const int m = min(ROWS, n - r0);
+      if (m == ROWS) {
+#pragma unroll 32
+        for (int r = 0; r < ROWS; ++r) s += rows[r][lane];
+      } else {
+        for (int r = 0; r < m; ++r) s += rows[r][lane];
+      }
+    }
+    __syncthreads();
+  }
+  if (wave == 0 && c < C) a.out[p][c] = s;
+}
+
 // Up to three products of one kind in one launch (workgroups in their order).
 struct GemmGroup {
   Gemm g[3];
   int tiles[3];  // workgroups of each product (0: none)
+  ColSums sums;  // before the products (EPI_STORE)
 };
 
 // AK / BK: k is A's / B's contiguous dimension (else m / n is).  Workgroup
 // tile T x T, four waves of T/2 x T/2 (16x16 tiles of
 // v_mfma_f32_16x16x32_bf16), K staged through LDS kStageK at a time with
-// 16-byte loads, the next stage's loads in flight while the current one is
-// multiplied.  Every output element is one accumulator over the k steps in
+// 16-byte loads, the loads of the next two stages (three at T = 32) in flight
+// while the current one is multiplied.  Every output element is one accumulator over the k steps in
 // ascending order whatever T is.  Epilogues:
 //  RELU      out = relu(acc + bias[n]) (f32) and its bf16 copy
 //  LINEAR    out = acc + bias[n]
@@ -169,14 +219,25 @@ struct GemmGroup {
 //  STORE     out = acc
 //
 // Bound by the round trips of the stages: a workgroup has little else to run
-// while a stage's loads are on their way.  Hence 128 k per stage (32 before)
-// and, where 64 x 64 tiles would leave CUs without work, 32 x 32 ones.
+// while a stage's loads are on their way.  Hence 128 k per stage (32 before),
+// loads two and three stages ahead (one ahead: 19 -> 13 us for 1024 x 4096 x 256,
+// 23 -> 15 the weight gradients of a step with its column sums, 15 -> 13 the input
+// gradients) and, where 64 x 64 tiles would leave CUs without work, 32 x 32 ones.
 template <int EPI, bool AK, bool BK, int T>
 __global__ __launch_bounds__(256) void gemm_bf16(GemmGroup grp) {
   constexpr int S = T / 32;  // 16 x 16 tiles per wave and dimension
-  __shared__ __attribute__((aligned(16))) uint16_t As[T * kStageK];  // [m][k]
-  __shared__ __attribute__((aligned(16))) uint16_t Bs[T * kStageK];  // [n][k]
+  constexpr int kAhead = T == 32 ? 3 : 2;
+  __shared__ __attribute__((aligned(16))) uint16_t lds[2 * T * kStageK];
+  uint16_t* const As = lds;                // [m][k]
+  uint16_t* const Bs = lds + T * kStageK;  // [n][k]
   int p = 0, blk = blockIdx.x;
+  if constexpr (EPI == EPI_STORE) {
+    if (blk < grp.sums.blocks) {  // whole workgroups
+      colsum_block<2 * T>(grp.sums, blk, reinterpret_cast<float (*)[64]>(lds));
+      return;
+    }
+    blk -= grp.sums.blocks;
+  }
   while (p < 2 && blk >= grp.tiles[p]) blk -= grp.tiles[p++];
   const Gemm g = grp.g[p];
   const int tn = (g.N + T - 1) / T;
@@ -194,34 +255,41 @@ __global__ __launch_bounds__(256) void gemm_bf16(GemmGroup grp) {
   for (int i = 0; i < S; ++i)
 #pragma unroll
     for (int j = 0; j < S; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
-  uint4 ra[T / 16], rb[T / 16];
-  stage_load<AK, T>(g.A, g.sam, g.sak, g.M, g.K, m0, 0, t, va, ra);
-  stage_load<BK, T>(g.B, g.sbn, g.sbk, g.N, g.K, n0, 0, t, vb, rb);
+  uint4 ra[kAhead][T / 16], rb[kAhead][T / 16];
+  auto load = [&](int s, int k0) {
+    if (k0 >= g.K) return;
+    stage_load<AK, T>(g.A, g.sam, g.sak, g.M, g.K, m0, k0, t, va, ra[s]);
+    stage_load<BK, T>(g.B, g.sbn, g.sbk, g.N, g.K, n0, k0, t, vb, rb[s]);
+  };
+#pragma unroll
+  for (int s = 0; s < kAhead; ++s) load(s, s * kStageK);
   const int r = lane & 15, kq = 8 * (lane >> 4);
-  for (int k0 = 0; k0 < g.K; k0 += kStageK) {
-    stage_store<AK, T>(As, t, ra);
-    stage_store<BK, T>(Bs, t, rb);
-    __syncthreads();
-    if (k0 + kStageK < g.K) {
-      stage_load<AK, T>(g.A, g.sam, g.sak, g.M, g.K, m0, k0 + kStageK, t, va, ra);
-      stage_load<BK, T>(g.B, g.sbn, g.sbk, g.N, g.K, n0, k0 + kStageK, t, vb, rb);
+  for (int kb = 0; kb < g.K; kb += kAhead * kStageK) {
+#pragma unroll
+    for (int s = 0; s < kAhead; ++s) {
+      const int k0 = kb + s * kStageK;
+      if (k0 >= g.K) break;
+      stage_store<AK, T>(As, t, ra[s]);
+      stage_store<BK, T>(Bs, t, rb[s]);
+      __syncthreads();
+      load(s, k0 + kAhead * kStageK);
+#pragma unroll
+      for (int u = 0; u < kStageK / 32; ++u) {
+        if (k0 + 32 * u >= g.K) break;
+        uint4 a[S], b[S];
+#pragma unroll
+        for (int i = 0; i < S; ++i)
+          a[i] = *reinterpret_cast<const uint4*>(As + stage_at(wm + 16 * i + r, 32 * u + kq));
+#pragma unroll
+        for (int j = 0; j < S; ++j)
+          b[j] = *reinterpret_cast<const uint4*>(Bs + stage_at(wn + 16 * j + r, 32 * u + kq));
+#pragma unroll
+        for (int i = 0; i < S; ++i)
+#pragma unroll
+          for (int j = 0; j < S; ++j) acc[i][j] = mfma_k32(a[i], b[j], acc[i][j]);
+      }
+      __syncthreads();
     }
-#pragma unroll
-    for (int u = 0; u < kStageK / 32; ++u) {
-      if (k0 + 32 * u >= g.K) break;
-      uint4 a[S], b[S];
-#pragma unroll
-      for (int i = 0; i < S; ++i)
-        a[i] = *reinterpret_cast<const uint4*>(As + stage_at(wm + 16 * i + r, 32 * u + kq));
-#pragma unroll
-      for (int j = 0; j < S; ++j)
-        b[j] = *reinterpret_cast<const uint4*>(Bs + stage_at(wn + 16 * j + r, 32 * u + kq));
-#pragma unroll
-      for (int i = 0; i < S; ++i)
-#pragma unroll
-        for (int j = 0; j < S; ++j) acc[i][j] = mfma_k32(a[i], b[j], acc[i][j]);
-    }
-    __syncthreads();
   }
   // D layout: lane holds D[4*(lane/16) + v][lane%16].  What the epilogue reads
   // is loaded before the first store, at clamped addresses: a load between
@@ -989,55 +1057,6 @@ __global__ __launch_bounds__(256) void softmax_xent_kernel(const float* __restri
   if (threadIdx.x == 0) row_loss[row] = logf(se) + mx - z[lab];
 }
 
-// Column sums of three n x C matrices in one launch (the bias gradients), 64
-// columns per workgroup.  Each column is summed by one thread over the rows
-// in ascending order, so the sums do not depend on the launch; the four waves
-// stage kSumRows rows at a time in LDS, the next rows' loads in flight while
-// the first wave adds.  Bound by that chain of additions (n of them) and the
-// stages' round trips: 12 us at n = 1024 for the three.  One thread per column
-// reading global memory itself, a round trip every few rows, took 225 us for
-// each matrix.
-struct ColSums {
-  const float* x[3];
-  float* out[3];
-  int C[3];
-};
-constexpr int kSumRows = 128;
-__global__ __launch_bounds__(256) void colsum_kernel(ColSums a, int n) {
-  __shared__ float rows[kSumRows][64];
-  constexpr int kPer = kSumRows / 4;
-  int p = 0, blk = blockIdx.x;
-  while (p < 2 && blk >= (a.C[p] + 63) / 64) blk -= (a.C[p++] + 63) / 64;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int C = a.C[p];
-  const int c = blk * 64 + lane;
-  const float* x = a.x[p] + min(c, C - 1);
-  float v[kPer];
-  auto load = [&](int r0) {  // at clamped, valid rows; the sum stops at n
-#pragma unroll
-    for (int i = 0; i < kPer; ++i) v[i] = x[(int64_t)min(r0 + 4 * i + wave, n - 1) * C];
-  };
-  load(0);
-  float s = 0.f;
-  for (int r0 = 0; r0 < n; r0 += kSumRows) {
-#pragma unroll
-    for (int i = 0; i < kPer; ++i) rows[4 * i + wave][lane] = v[i];
-    __syncthreads();
-    if (r0 + kSumRows < n) load(r0 + kSumRows);
-    if (wave == 0) {
-      const int m = min(kSumRows, n - r0);
-      if (m == kSumRows) {
-#pragma unroll 32
-        for (int r = 0; r < kSumRows; ++r) s += rows[r][lane];
-      } else {
-        for (int r = 0; r < m; ++r) s += rows[r][lane];
-      }
-    }
-    __syncthreads();
-  }
-  if (wave == 0 && c < C) a.out[p][c] = s;
-}
-
 // Adam on FP32 masters; refreshes the bf16 copies.  All six parameter arrays
 // in one launch, each starting at a workgroup of its own.
 struct AdamArgs {
@@ -1172,13 +1191,15 @@ hipError_t reserve_batch(Mlp* m, int n) {
 // when its stride is 1; all products of a group alike) and the tile from the
 // work: 64 x 64 where that gives every CU (256) a workgroup, else 32 x 32.
 template <int EPI>
-void launch_gemm(hipStream_t st, const rte::Gemm* g, int count) {
+void launch_gemm(hipStream_t st, const rte::Gemm* g, int count,
+                 const rte::ColSums& sums = rte::ColSums{}) {
   auto tiles = [&](int i, int T) { return ((g[i].M + T - 1) / T) * ((g[i].N + T - 1) / T); };
   int n64 = 0;
   for (int i = 0; i < count; ++i) n64 += tiles(i, 64);
   const int T = n64 >= 256 ? 64 : 32;
   rte::GemmGroup grp{};
-  int total = 0;
+  grp.sums = sums;
+  int total = sums.blocks;
   for (int i = 0; i < count; ++i) {
     grp.g[i] = g[i];
     grp.tiles[i] = tiles(i, T);
@@ -1246,12 +1267,13 @@ hipError_t backward(Mlp* m, const int32_t* y, int n, hipStream_t st) {
        m->gW[1].as<float>(), nullptr},
       {m->X16.as<uint16_t>(), 1, d0, m->dH1b.as<uint16_t>(), d1, 1, d0, d1, n, nullptr, nullptr,
        m->gW[0].as<float>(), nullptr}};
-  launch_gemm<rte::EPI_STORE>(st, gw, 3);
+  // and the bias gradients
   const rte::ColSums cs{{m->dZ.as<float>(), m->dH2.as<float>(), m->dH1.as<float>()},
                         {m->gb[2].as<float>(), m->gb[1].as<float>(), m->gb[0].as<float>()},
-                        {d3, d2, d1}};
-  const int blocks = (d3 + 63) / 64 + (d2 + 63) / 64 + (d1 + 63) / 64;
-  hipLaunchKernelGGL(rte::colsum_kernel, dim3(blocks), dim3(256), 0, st, cs, n);
+                        {d3, d2, d1},
+                        n,
+                        (d3 + 63) / 64 + (d2 + 63) / 64 + (d1 + 63) / 64};
+  launch_gemm<rte::EPI_STORE>(st, gw, 3, cs);
   return hipGetLastError();
 }
 
