@@ -100,12 +100,14 @@ struct rte_ctx {
   ~rte_ctx();
 };
 
-// s_work is kept for the next call up to 1 GiB (allocating and freeing it took 1 ms
-// of the 4 ms that lists and graph of 160k points take)
+// s_work is kept for the next call up to 256 MiB: allocating and freeing it took
+// 1 ms of the 4 ms that lists and graph of 160k points take.  (The set-up calls
+// allocate for themselves: with their scratch kept a fit took 0.4 ms less, but the
+// first allocations of the queries after it 0.3 ms more.)
 struct WorkGuard {
   rte_ctx* c;
   ~WorkGuard() {
-    if (c->s_work.bytes > (size_t)1 << 30) c->s_work.release();  // hipFree waits for the device
+    if (c->s_work.bytes > (size_t)256 << 20) c->s_work.release();  // hipFree waits for the device
   }
 };
 

@@ -689,7 +689,7 @@ int rte_build_kdtree_gpu(rte_ctx* c, const float* pts, int64_t np, int64_t strid
   do {                                  \
     if (int r_ = ck((expr), what)) return r_; \
   } while (0)
-  DevBuf pin, outb;
+  DevBuf pin, work, outb;  // freed on return (hipFree waits for the device)
   const float* dp = pts;
   int64_t ds = stride;
   if (where == RTE_HOST) {  // only the three coordinates travel
@@ -731,9 +731,8 @@ int rte_build_kdtree_gpu(rte_ctx* c, const float* pts, int64_t np, int64_t strid
     take(dcount, cap);
     return at;
   };
-  KCK(c->s_work.reserve(lay(nullptr)), "hipMalloc(kd-tree work)");
-  WorkGuard guard{c};
-  lay(c->s_work.as<char>());
+  KCK(work.reserve(lay(nullptr)), "hipMalloc(kd-tree work)");
+  lay(work.as<char>());
   w.np = np;
   w.cap = cap;
   hipLaunchKernelGGL(kd_start_kernel, dim3(1), dim3(64), 0, st, w);

@@ -502,10 +502,9 @@ int rte_pca_fit(rte_ctx* c, const float* X, int64_t n, int d, int64_t stride, fl
   const size_t dd = (size_t)d * d;
   // covariance | mean | partials
   const size_t part_n = std::max((size_t)nb * dd, (size_t)nb_sum * d);
-  if (int r = ck(c->s_work.reserve((dd + d + part_n) * sizeof(double)), "hipMalloc(pca work)"))
-    return r;
-  WorkGuard guard{c};
-  double* cov = c->s_work.as<double>();
+  DevBuf work;  // freed on return (hipFree waits for the device)
+  if (int r = ck(work.reserve((dd + d + part_n) * sizeof(double)), "hipMalloc(pca work)")) return r;
+  double* cov = work.as<double>();
   double* mean = cov + dd;
   double* part = mean + d;
   // whole waves of columns, and no more
@@ -562,7 +561,7 @@ int rte_pca_rotate(rte_ctx* c, const float* X, int64_t n, int d, int64_t stride,
   };
   if ((n + 15) / 16 > 0x7fffffff)
     return rte_fail(c, RTE_EUNSUP, "pca_rotate: too many rows");
-  DevBuf xin, ob;
+  DevBuf xin, rm, ob;
   const float* dx = X;
   float* dout = out;
   const size_t xbytes = ((size_t)(n - 1) * stride + d) * sizeof(float);
@@ -577,12 +576,10 @@ int rte_pca_rotate(rte_ctx* c, const float* X, int64_t n, int d, int64_t stride,
   // R (d x d_out) and mu (d) are host arrays; R widened comes first
   const int ldr = (d_out + rte::kRotCols - 1) / rte::kRotCols * rte::kRotCols;
   const size_t wide = (size_t)(d + 1) * ldr;
-  if (int r = ck(c->s_work.reserve(wide * sizeof(double) +
-                                   ((size_t)d * d_out + d) * sizeof(float)),
+  if (int r = ck(rm.reserve(wide * sizeof(double) + ((size_t)d * d_out + d) * sizeof(float)),
                  "hipMalloc"))
     return r;
-  WorkGuard guard{c};
-  double* dW = c->s_work.as<double>();
+  double* dW = rm.as<double>();
   float* dR = reinterpret_cast<float*>(dW + wide);
   float* dmu = dR + (size_t)d * d_out;
   if (int r = ck(hipMemcpyAsync(dR, R, (size_t)d * d_out * 4, hipMemcpyHostToDevice, st), "copy"))
