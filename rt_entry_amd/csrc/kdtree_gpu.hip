@@ -24,8 +24,9 @@
 //              integer keys; a node whose search has not ended is carried over
 //   plan       one workgroup makes the next round's nodes of the children, the map
 //              from chunks to nodes and the list of small nodes
-// A round of 1M points takes 30 us; a launch per step, boxes and split-axis values
-// gathered from the rows by id, and a read-back every four steps took 270.
+// 1M points, cap 256: ten rounds of 58 us, 0.9 ms in all; 3.4 with a launch per
+// step, boxes and split-axis values gathered from the rows by id, and a read-back
+// every four steps.
 // Small nodes (at most kKdSmall points) are finished by one workgroup each:
 // ids, coordinates and a local permutation in LDS, an explicit stack of
 // segments, block-wide counts for the bisection.  Left children always come
