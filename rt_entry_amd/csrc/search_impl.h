@@ -633,8 +633,9 @@ struct SearchCore {
   // no branch.  J = 2 and 8 also serve smaller d (1..32, 129..224): every
   // dim group is masked there.
   //
-  // FAST (d == 32 * J, every row offset below 2^32 bytes, ids below 2^24): a
-  // row's byte offset is one full-rate 24-bit multiply-add into one VGPR,
+  // FAST (d == 32 * J, every row offset below 2^32 bytes, ids and row sizes in
+  // bytes below 2^24, the two factors of the product): a row's byte offset is
+  // one full-rate 24-bit multiply-add into one VGPR,
   // added to the scalar base by the load itself, and no dim is masked.  The
   // 64-bit form needs a quarter-rate multiply-add and two VGPRs per point,
   // and an addition for the last dim group.
@@ -1393,12 +1394,13 @@ hipError_t launch_f(const SearchArgs& a, int grid, int wpb, hipStream_t st, int*
 }
 
 // The FAST kernels: one row per iteration, whole 32-dim groups, 32-bit row
-// offsets from 24-bit ids.  The rest (wider search, other dims, bases of 4
-// GiB or 16.7M rows and more, several waves per query) takes the general form.
+// offsets from 24-bit ids and 24-bit row sizes.  The rest (wider search, other
+// dims, bases of 4 GiB, 16.7M rows or 16 MiB a row and more, several waves per
+// query) takes the general form.
 template <bool TUNED, int NR, int MR, int J, int WPQ, bool LQ>
 hipError_t launch_t(const SearchArgs& a, int grid, int wpb, hipStream_t st, int* occ) {
   if constexpr (MR == 1 && WPQ == 1) {
-    if (a.width == 1 && a.d == 32 * J && a.np < (1 << 24) &&
+    if (a.width == 1 && a.d == 32 * J && a.np < (1 << 24) && a.stride < (1 << 22) &&
         (uint64_t)a.np * (uint64_t)a.stride <= (1ull << 30))
       return launch_f<TUNED, NR, MR, J, WPQ, LQ, true>(a, grid, wpb, st, occ);
   }
