@@ -88,6 +88,7 @@ class Context:
         rc = lib().rte_create(C.byref(self._h), int(device))
         if rc != 0:
             raise RteError(rc, f"rte_create(device={device}) failed")
+        self._own_stream = self.stream
         self._keep = {}
         self.d = 0
         self.d_out = 0
@@ -239,17 +240,22 @@ class Context:
         # The outputs come from the library stream's own pool: their memory is
         # handed out again only to work behind this call, and the fill of the
         # leaves runs there too.  Filled on torch's default stream, every call
-        # made that stream and the library's wait for each other: about 45 of a
-        # single query's 125 us, and no two contexts' queries ever overlapped
-        # (three contexts in turn: 126 -> 30 us a query).
+        # made that stream and the library's wait for each other, and no two
+        # contexts' queries ever overlapped (three contexts in turn: 126 -> 30
+        # us for a single query; one context alone: 139 -> 110).
         with self._on_stream(dev):
             pq = torch.empty((nq, self.d_out), dtype=torch.float32, device=dev)
             leaf = (torch.empty if params.algo == 1 else torch.zeros)(nq, dtype=torch.int32,
                                                                       device=dev)
             ids = torch.empty((nq, k), dtype=torch.int32, device=dev)
             dists = torch.empty((nq, k), dtype=torch.float32, device=dev)
+        # Work behind this call is behind the current stream's readers of outputs
+        # that were dropped only where the two streams are one, or the default
+        # stream and the context's own, which is ordered with it.
         cur = torch.cuda.current_stream(dev)
-        if cur.cuda_stream not in (0, self.stream):  # not ordered with the library's by itself
+        lib_stream = self.stream
+        if cur.cuda_stream != lib_stream and (cur.cuda_stream != 0
+                                              or lib_stream != self._own_stream):
             for t in (pq, leaf, ids, dists):
                 t.record_stream(cur)
         qp, _, _ = _ptr(Q, np.float32)
