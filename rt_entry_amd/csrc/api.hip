@@ -10,6 +10,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -172,6 +173,51 @@ int set_device(rte_ctx* c) {
 
 static hipError_t set_sort_kernel_attributes();
 
+namespace {
+
+// Streams of destroyed contexts, idle, for the next contexts on their device.  A
+// caller's allocator may keep memory under a stream's handle (torch does): were the
+// stream destroyed, the runtime could give its handle to a stream of another kind,
+// which is not ordered with the null stream, and with it that memory.  At most
+// kIdleStreams are kept.
+constexpr size_t kIdleStreams = 64;
+struct IdleStreams {
+  std::mutex mu;
+  std::vector<std::pair<int, hipStream_t>> list;
+};
+IdleStreams& idle_streams() {
+  static IdleStreams* s = new IdleStreams();  // contexts may be destroyed at exit
+  return *s;
+}
+
+hipError_t take_stream(int device, hipStream_t* out) {
+  {
+    IdleStreams& s = idle_streams();
+    std::lock_guard<std::mutex> lock(s.mu);
+    for (size_t i = s.list.size(); i-- > 0;)
+      if (s.list[i].first == device) {
+        *out = s.list[i].second;
+        s.list.erase(s.list.begin() + i);
+        return hipSuccess;
+      }
+  }
+  return hipStreamCreate(out);
+}
+
+void give_stream(int device, hipStream_t st) {
+  if (hipStreamSynchronize(st) == hipSuccess) {  // fails on a stream that is being captured
+    IdleStreams& s = idle_streams();
+    std::lock_guard<std::mutex> lock(s.mu);
+    if (s.list.size() < kIdleStreams) {
+      s.list.emplace_back(device, st);
+      return;
+    }
+  }
+  (void)hipStreamDestroy(st);
+}
+
+}  // namespace
+
 extern "C" {
 
 int rte_create(rte_ctx** out, int device) {
@@ -185,12 +231,12 @@ int rte_create(rte_ctx** out, int device) {
   // a blocking stream: ordered with the null stream, so work the caller
   // queues there (torch's default stream) and the context's kernels see each
   // other's results without explicit events
-  if (hipSetDevice(device) != hipSuccess || hipStreamCreate(&c->own) != hipSuccess) {
+  if (hipSetDevice(device) != hipSuccess || take_stream(device, &c->own) != hipSuccess) {
     delete c;
     return RTE_EHIP;
   }
   if (set_sort_kernel_attributes() != hipSuccess) {
-    (void)hipStreamDestroy(c->own);
+    give_stream(device, c->own);
     delete c;
     return RTE_EHIP;
   }
@@ -203,8 +249,10 @@ int rte_destroy(rte_ctx* c) {
   if (!c) return RTE_OK;
   (void)hipSetDevice(c->device);
   if (c->stream) (void)hipStreamSynchronize(c->stream);
-  if (c->own) (void)hipStreamDestroy(c->own);
+  const int device = c->device;
+  const hipStream_t own = c->own;
   delete c;
+  if (own) give_stream(device, own);
   return RTE_OK;
 }
 
