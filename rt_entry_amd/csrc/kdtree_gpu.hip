@@ -42,13 +42,13 @@
 #include <vector>
 
 #include "ctx.h"
+#include "kd_chunk.h"
 
 namespace rte {
 
 namespace {
 
 constexpr int kKdSmall = 2048;   // nodes up to this size: one workgroup in LDS
-constexpr int kKdChunk = 2048;   // points per workgroup in the rounds' kernels
 constexpr int kKdMaxIter = 64;   // findxM ends within about 11 steps
 constexpr int kKdSteps = 4;      // of findxM in a launch
 constexpr int kKdPasses = 3;     // launches in a round
@@ -258,20 +258,20 @@ __global__ __launch_bounds__(256) void kd_count_kernel(KdWork w, int par, int pa
       br[2 * q + 1] = br[q];
     }
   }
-  const int s0 = n.l + ((int)blockIdx.x - n.blk0) * kKdChunk, s1 = min(n.r, s0 + kKdChunk);
+  const KdChunk ch = kd_chunk(n.l, n.r, (int)blockIdx.x - n.blk0);
   const float* x = reinterpret_cast<const float*>(w.rec[par]) + n.axis;
   constexpr int PER = kKdChunk / 256;
   float v[PER];
 #pragma unroll
   for (int k = 0; k < PER; ++k)  // past the end: above every midpoint, or NaN
-    v[k] = s0 + 256 * k + t < s1 ? x[4 * (int64_t)(s0 + 256 * k + t)] : INFINITY;
+    v[k] = 256 * k + t < ch.count ? x[4 * (int64_t)(ch.first + 256 * k + t)] : INFINITY;
   __syncthreads();
 #pragma unroll
   for (int q = 1; q <= kKdMids; ++q) {
     unsigned c = 0;
 #pragma unroll
     for (int k = 0; k < PER; ++k)
-      c += (unsigned)__popcll(__ballot(s0 + 256 * k + t < s1 && v[k] <= mid[q]));
+      c += (unsigned)__popcll(__ballot(256 * k + t < ch.count && v[k] <= mid[q]));
     if ((t & 63) == 0 && c) atomicAdd(&tot[q], c);
   }
   __syncthreads();
@@ -292,20 +292,20 @@ __global__ __launch_bounds__(256) void kd_partition_kernel(KdWork w, int par) {
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
   LevelNode& n = w.nodes[par][w.map[par][blockIdx.x]];
   const int l = n.l, r = n.r;
-  const int s0 = l + ((int)blockIdx.x - n.blk0) * kKdChunk, s1 = min(r, s0 + kKdChunk);
-  const float4* in = w.rec[par];
+  const KdChunk ch = kd_chunk(l, r, (int)blockIdx.x - n.blk0);
+  const float4* in = w.rec[par] + ch.first;
   float4* out = w.rec[par ^ 1];
   const KdState s = kd_walk(n, kKdPasses);
   float4 p[PER];
 #pragma unroll
   for (int k = 0; k < PER; ++k) {
-    const int i = s0 + 256 * k + t;
-    p[k] = i < s1 ? in[i] : make_float4(0.f, 0.f, 0.f, 0.f);
+    const int i = 256 * k + t;
+    p[k] = i < ch.count ? in[i] : make_float4(0.f, 0.f, 0.f, 0.f);
   }
   if (!s.done) {
 #pragma unroll
     for (int k = 0; k < PER; ++k)
-      if (s0 + 256 * k + t < s1) out[s0 + 256 * k + t] = p[k];
+      if (256 * k + t < ch.count) out[ch.first + 256 * k + t] = p[k];
     return;  // all threads
   }
   const int axis = n.axis;
@@ -316,7 +316,7 @@ __global__ __launch_bounds__(256) void kd_partition_kernel(KdWork w, int par) {
   unsigned nl = 0, nr = 0;        // this wave's counts (uniform)
 #pragma unroll
   for (int k = 0; k < PER; ++k) {
-    const bool valid = s0 + 256 * k + t < s1;
+    const bool valid = 256 * k + t < ch.count;
     const float x[3] = {p[k].x, p[k].y, p[k].z};
     const float xa = axis == 0 ? x[0] : axis == 1 ? x[1] : x[2];
     const bool left = valid && xa < s.xm;
@@ -425,7 +425,7 @@ __global__ __launch_bounds__(1024) void kd_plan_kernel(KdWork w, int par) {
             }
           }
       }
-      for (int k = 0; k < large; ++k) blocks += (c[k].r - c[k].l + kKdChunk - 1) / kKdChunk;
+      for (int k = 0; k < large; ++k) blocks += kd_chunks(c[k].r - c[k].l);
     }
     __syncthreads();
     sn[t] = large;
@@ -448,7 +448,7 @@ __global__ __launch_bounds__(1024) void kd_plan_kernel(KdWork w, int par) {
       for (int e = 0; e < 2; ++e)
         for (int a = 0; a < 6; ++a) d.key[e][a] = a < 3 ? 0xffffffffu : 0u;
       w.nodes[par ^ 1][at] = d;
-      for (int j = (d.r - d.l + kKdChunk - 1) / kKdChunk; j > 0; --j) w.map[par ^ 1][b++] = at;
+      for (int j = kd_chunks(d.r - d.l); j > 0; --j) w.map[par ^ 1][b++] = at;
       ++at;
     }
     base_n += sn[1023];
