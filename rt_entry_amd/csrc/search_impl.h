@@ -21,17 +21,17 @@
 //    one iteration issues its loads together and only for points that need a
 //    distance; a lane reads its half-wave's ids in 16-byte LDS reads and
 //    forms each row address with one 32x32->64 multiply-add;
-//  - a batch of which few elements enter the beam is merged by ranks through
-//    LDS instead of by the networks (rank_merge);
-//  - the FAST kernels (one row per iteration, whole 32-dim groups, 32-bit row
-//    offsets) have the graph row expected next on its way while the current
-//    distances are gathered.
+//  - in beams of up to 64 slots a batch of which few elements enter is merged by
+//    ranks through LDS instead of by the networks (rank_merge, use_ranks);
+//  - the FAST kernels (one row per iteration, whole 32-dim groups up to 256 dims,
+//    32-bit row offsets) have the graph row expected next on its way while the
+//    current distances are gathered.
 // Against kernels that ran both networks on every step, formed 64-bit row
 // addresses and requested each row when its node was taken: 1M x 128, 10k
-// queries at beam 256 877 -> 826 us and 20k uneven ones at 96-d 2504 -> 2396 us
-// (of waiting and issue in about equal parts), 100k x 128 with 1k queries 170
-// -> 156 us (latency), 10k at 64-d with rerank 631 -> 566 us; 10k at beam 64
-// unchanged at 571 us, which reads 3.9 GB through the L2s at 7.1 TB/s.
+// queries at beam 256 875 -> 794 us, 20k uneven ones at 96-d 2507 -> 2372 us,
+// 10k at 64-d with rerank 632 -> 566 us, 100 queries on 200k x 128 at beam 64 105
+// -> 96 us (latency); 10k at beam 64 unchanged at 571 us, which reads 3.9 GB
+// through the L2s at 7.1 TB/s.
 // Parity decisions P1-P7 match the CPU oracle (zeroed filter, all-ones first
 // mask, snapshot filter test per row, no row read for ids >= np,
 // barrier-separated substeps, REF/TUNED comparators).
@@ -593,8 +593,25 @@ constexpr int kRankMax = 24;
 
 constexpr int ilog2c(int x) { return x <= 1 ? 0 : 1 + ilog2c(x / 2); }
 
+// Beams of up to 64 slots (one register a lane) merge a batch of few entering
+// elements by ranks; with several waves a query, each of which repeats the merge,
+// beams of up to 32.  Past that the networks alone are as fast or faster, ranks
+// taking a second copy of the beam in registers and more LDS, but for TUNED's
+// two-key networks over batches of 128.  Networks alone -> with ranks, us: 100
+// queries at beam 16, d = 96, width 4 60 -> 52; 10k at beam 64, d = 64 in leaf order
+// 319 -> 304; 3k at beam 128, d = 100, width 4, TUNED 331 -> 324; but 100 at beam
+// 64, d = 128, four waves a query 104 -> 112; 10k at beam 128, d = 64 in leaf order
+// 369 -> 402 and d = 96, TUNED 616 -> 667; at beam 256, d = 64 622 -> 740 and at beam
+// 512, d = 128 1060 -> 1495.
+constexpr int kRanksWaves = 32;  // slots, for several waves a query
+template <bool TUNED, int NR, int MR>
+constexpr bool use_ranks() {
+  return NR == 1 || (TUNED && NR == 2 && MR == 2);
+}
+
 template <bool TUNED, int NR, int MR, int J, int WPQ, bool FAST>
 struct SearchCore {
+  static constexpr bool RANKS = use_ranks<TUNED, NR, MR>();
   // points per half-wave in one load group: all 16 when the vectors fit in
   // 64 VGPRs, so one iteration's gathers are issued together; with WPQ
   // waves per query each wave takes 1/WPQ of them
@@ -755,10 +772,9 @@ struct SearchCore {
   //
   // Bound by instruction issue: 2 VALU instructions per entering element and
   // register of L and B, against the full sort of B and merge of L whatever
-  // enters.  Elements that enter per step, measured on the CPU over mixtures
-  // of integer and of normalised vectors: 5 at beam 64, 8 at beam 256 (median
-  // 3 to 5; none in 6 to 40% of the steps).  At beam 256 a launch issues 472M
-  // VALU instructions without this path and 390M with it.
+  // enters.  At beam 64, 5 elements enter a step on average (median 3, none in 6 to
+  // 40% of the steps; counted on the CPU over mixtures of integer and of normalised
+  // vectors).
   template <class BeamT>
   static __device__ __forceinline__ bool rank_merge(const WaveLds& s, int lane, BeamT& L,
                                                     const float (&bd)[MR], const int (&bi)[MR],
@@ -914,7 +930,8 @@ struct SearchCore {
   // the networks (as does a point at distance kMaxD while seeding).
   //
   // `plain` is per query: false once a merge met equal keys or a NaN, after
-  // which the networks take every step (L may hold the tie, or be unsorted).
+  // which the networks take every step (L may hold the tie, or be unsorted), and
+  // from the start where ranks are not used.
   template <class BeamT>
   static __device__ __forceinline__ void merge_batch(const WaveLds& s, int lane, BeamT& L,
                                                      float (&bd)[MR], int (&bi)[MR], int n, int m,
@@ -922,7 +939,7 @@ struct SearchCore {
     const float last = L.last(n);
     uint64_t em[MR], any = 0;
     int cnt = 0;
-    bool ranks = plain;
+    bool ranks = RANKS && plain;
 #pragma unroll
     for (int r = 0; r < MR; ++r) {
       em[r] = __builtin_amdgcn_ballot_w64(bd[r] < last);
@@ -930,16 +947,21 @@ struct SearchCore {
       if constexpr (TUNED) {
         const uint64_t le = __builtin_amdgcn_ballot_w64(bd[r] <= last && bd[r] != kMaxD);
         any |= le;
-        if (le != em[r]) ranks = false;
-        if (!skip_max && __builtin_amdgcn_ballot_w64(bd[r] == kMaxD && bi[r] != npi)) ranks = false;
+        if constexpr (RANKS) {
+          if (le != em[r]) ranks = false;
+          if (!skip_max && __builtin_amdgcn_ballot_w64(bd[r] == kMaxD && bi[r] != npi))
+            ranks = false;
+        }
       } else {
         any |= em[r];
       }
     }
     if (!any) return;
-    if (ranks && cnt <= kRankMax) {
-      if (rank_merge(s, lane, L, bd, bi, em, cnt, n)) return;
-      plain = false;
+    if constexpr (RANKS) {
+      if (ranks && cnt <= kRankMax) {
+        if (rank_merge(s, lane, L, bd, bi, em, cnt, n)) return;
+        plain = false;
+      }
     }
     sort_desc<TUNED, MR>(bd, bi, m, lane);
 #pragma unroll
@@ -957,7 +979,8 @@ struct SearchCore {
     } else {
       exchange_merge(s, lane, L.d, L.i, n, m, skip_max);
     }
-    if (plain) plain = distinct(lane, L, n);
+    if constexpr (RANKS)
+      if (plain) plain = distinct(lane, L, n);
   }
 };
 
@@ -1079,19 +1102,19 @@ __host__ __device__ constexpr int filter_words(int w) { return (w + 3) & ~3; }
 // lie over them -- and for a beam held in LDS its queue of 64*NR (distance, id)
 // slots and one more, each array in whole 16 bytes
 constexpr int kRankWords = (kRankMax + 4) + kRankMax + 2 * kRankMax;
-template <int NR>
+template <int MR, int NR>
 __host__ __device__ constexpr int queue_words() {
-  return 64 * NR + 4;
+  return 64 * NR + (use_ranks<true, NR, MR>() ? 4 : 0);
 }
 template <int MR, int WPQ, int NR, bool LQ>
 __host__ __device__ constexpr int batch_words() {
   constexpr int batch = (WPQ > 1 ? 3 : 4) * 64 * MR;
-  constexpr int merge = kRankWords + (LQ ? 0 : 2 * 64 * NR + 4);
+  constexpr int merge = use_ranks<true, NR, MR>() ? kRankWords + (LQ ? 0 : 2 * 64 * NR + 4) : 0;
   return batch > merge ? batch : merge;
 }
 template <int MR, int WPQ, int NR, bool LQ>
 __host__ __device__ constexpr int lds_words_wave() {
-  return batch_words<MR, WPQ, NR, LQ>() + (LQ ? 2 * queue_words<NR>() : 0);
+  return batch_words<MR, WPQ, NR, LQ>() + (LQ ? 2 * queue_words<MR, NR>() : 0);
 }
 // LDS words a query shares between its waves (WPQ > 1): two distance
 // buffers (alternating batches) and the broadcast slot of the work queue
@@ -1100,17 +1123,8 @@ __host__ __device__ constexpr int lds_words_query() {
   return WPQ > 1 ? 2 * 64 * MR + 4 : 0;
 }
 
-// Waves per SIMD asked of the compiler: four of the FAST kernels with up to
-// 256 beam slots and 128 dims, which need just over the 128 VGPRs of four
-// waves when left alone (131 at beam 256, d = 128) and then run three.  At
-// 128 only values used once per query go to scratch.
-template <int NR, int J, bool FAST>
-constexpr int min_waves() {
-  return FAST && NR <= 4 && J <= 4 ? 4 : 1;
-}
-
 template <bool TUNED, int NR, int MR, int J, int WPQ, bool LQ, bool FAST>
-__global__ __launch_bounds__(256, (min_waves<NR, J, FAST>())) void search_kernel(SearchArgs a) {
+__global__ __launch_bounds__(256) void search_kernel(SearchArgs a) {
   using Core = SearchCore<TUNED, NR, MR, J, WPQ, FAST>;
   extern __shared__ uint32_t smem[];
   const int lane = threadIdx.x & 63;
@@ -1168,7 +1182,7 @@ __global__ __launch_bounds__(256, (min_waves<NR, J, FAST>())) void search_kernel
     s.es = (int2*)(s.eo + kRankMax);
     s.mbuf = LQ ? nullptr : s.es + kRankMax;
     s.qd = LQ ? (float*)(base_lds + fwords + batch_words<MR, WPQ, NR, LQ>()) : nullptr;
-    s.qi = LQ ? (int*)(s.qd + queue_words<NR>()) : nullptr;
+    s.qi = LQ ? (int*)(s.qd + queue_words<MR, NR>()) : nullptr;
     // the hash count is fixed per mode (kHashes), checked on the host
     Bloom<kHashes<TUNED>> bl{s.bloom, (uint32_t)bwords, (uint32_t)(31 - __clz(bwords)),
                              (uint32_t)bwords * 32u};
@@ -1199,7 +1213,8 @@ __global__ __launch_bounds__(256, (min_waves<NR, J, FAST>())) void search_kernel
     const int32_t* prow = a.pids + (int64_t)hit * a.cap;
     uint32_t seed = (uint32_t)(q * 64 + lane);  // :66
     int nE = 0, nX = 0;
-    bool plain = true;  // no equal keys met yet (merge_batch)
+    // no equal keys met yet (merge_batch)
+    bool plain = Core::RANKS && (WPQ == 1 || n <= kRanksWaves);
     int vpre = -1, gpre = npi;  // FAST: node whose graph row gpre holds or awaits
 
     // ---- entry seeding, :479-959
@@ -1396,10 +1411,12 @@ hipError_t launch_f(const SearchArgs& a, int grid, int wpb, hipStream_t st, int*
 // The FAST kernels: one row per iteration, whole 32-dim groups, 32-bit row
 // offsets from 24-bit ids and 24-bit row sizes.  The rest (wider search, other
 // dims, bases of 4 GiB, 16.7M rows or 16 MiB a row and more, several waves per
-// query) takes the general form.
+// query) takes the general form, and so does d = 960, where the launches are bound
+// by L2 misses: 10k queries in leaf order took 0.92 to 1.10 of the general form's
+// time with the FAST one, by how the queries happened to share rows.
 template <bool TUNED, int NR, int MR, int J, int WPQ, bool LQ>
 hipError_t launch_t(const SearchArgs& a, int grid, int wpb, hipStream_t st, int* occ) {
-  if constexpr (MR == 1 && WPQ == 1) {
+  if constexpr (MR == 1 && WPQ == 1 && J <= 8) {
     if (a.width == 1 && a.d == 32 * J && a.np < (1 << 24) && a.stride < (1 << 22) &&
         (uint64_t)a.np * (uint64_t)a.stride <= (1ull << 30))
       return launch_f<TUNED, NR, MR, J, WPQ, LQ, true>(a, grid, wpb, st, occ);
