@@ -164,6 +164,25 @@ int finish_out(rte_ctx* c, T* host, const T* dev, size_t count, int where) {
   return RTE_OK;
 }
 
+// the flag words of a kNN call, with an epoch of their own
+int knn_flags(rte_ctx* c, rte::KnnFlags* f) {
+  constexpr size_t bytes = rte::kKnnFlagWords * sizeof(uint32_t);
+  if (!c->knn_tested)
+    HIPCHK(c, hipEventCreateWithFlags(&c->knn_tested, hipEventDisableTiming), "hipEventCreate");
+  if (!c->knn_host)
+    HIPCHK(c, hipHostMalloc((void**)&c->knn_host, bytes,
+                            hipHostMallocMapped | hipHostMallocCoherent),
+           "hipHostMalloc(flags)");
+  HIPCHK(c, c->knn_dev.reserve(bytes), "hipMalloc(flags)");
+  if (c->knn_epoch == 0 || ++c->knn_epoch == 0) {  // new words, or every epoch used
+    memset(c->knn_host, 0, bytes);
+    HIPCHK(c, hipMemsetAsync(c->knn_dev.p, 0, bytes, c->stream), "clear flags");
+    c->knn_epoch = 1;
+  }
+  *f = rte::KnnFlags{c->knn_dev.as<uint32_t>(), c->knn_host, c->knn_epoch};
+  return RTE_OK;
+}
+
 int set_device(rte_ctx* c) {
   HIPCHK(c, hipSetDevice(c->device), "hipSetDevice");
   return RTE_OK;
@@ -378,51 +397,71 @@ int rte_knn_rows(rte_ctx* c, const float* X, int64_t np, int d, int64_t stride, 
   if (int r = stage_out(c, c->s_out, ids_out, (size_t)nrows * k, where, &di)) return r;
   if (dists_out)
     if (int r = stage_out(c, c->s_aux2, dists_out, (size_t)nrows * k, where, &dd)) return r;
-  // rows in launches of 128k (short kernels)
-  const int64_t step = 1 << 17;
   const int64_t npad = rte::knn_padded(np);
   int cus = 0;
   (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device);
   cus = std::max(cus, 1);
-  // norms | half | flag | bf16 rows | the whole-number kernel's scratch; without
-  // room for the last four (and half) the FP32 kernel runs
+  // The whole-number kernel's half | bf16 rows | scratch, in s_work: taken at once,
+  // and the bf16 rows written with the norms, where the context keeps that much;
+  // of a larger base after the test of its values.
   auto up = [](size_t n) { return (n + 255) & ~(size_t)255; };
   const size_t norm_bytes = up((size_t)npad * sizeof(float)),
                xb_bytes = up((size_t)npad * d * sizeof(uint16_t));
-  const bool room = np <= rte::kKnnWholeMax &&
-                    c->s_work.reserve(2 * norm_bytes + 256 + xb_bytes +
-                                      rte::knn_whole_bytes(np, d, nrows, cus)) == hipSuccess;
+  const bool test = np <= rte::kKnnWholeMax;
+  const size_t work_bytes =
+      norm_bytes + xb_bytes + (test ? rte::knn_whole_bytes(np, d, nrows, cus) : 0);
   WorkGuard guard{c};
-  if (!room) {
-    (void)hipGetLastError();
-    HIPCHK(c, c->s_work.reserve(norm_bytes), "hipMalloc(norms)");
-  }
-  char* w = c->s_work.as<char>();
-  float* norms = reinterpret_cast<float*>(w);
-  float* half = room ? reinterpret_cast<float*>(w + norm_bytes) : nullptr;
-  uint32_t* flag = room ? reinterpret_cast<uint32_t*>(w + 2 * norm_bytes) : nullptr;
-  uint16_t* xb = room ? reinterpret_cast<uint16_t*>(w + 2 * norm_bytes + 256) : nullptr;
-  void* work = room ? w + 2 * norm_bytes + 256 + xb_bytes : nullptr;
-  if (room) HIPCHK(c, hipMemsetAsync(flag, 0, sizeof(uint32_t), c->stream), "clear flag");
-  HIPCHK(c, rte::launch_row_norms(dx, np, d, stride, norms, xb, half, flag, c->stream),
-         "norms");
-  uint32_t bits = rte::kKnnNotWhole;
-  if (room) {
-    HIPCHK(c, hipMemcpyAsync(&bits, flag, sizeof bits, hipMemcpyDeviceToHost, c->stream),
-           "read flag");
-    HIPCHK(c, hipStreamSynchronize(c->stream), "sync norms");
-  }
+  HIPCHK(c, c->s_aux3.reserve(norm_bytes), "hipMalloc(norms)");
+  auto take_work = [&]() {
+    const bool ok = c->s_work.reserve(work_bytes) == hipSuccess;
+    if (!ok) (void)hipGetLastError();  // the FP32 kernel needs none
+    return ok;
+  };
+  bool room = test && work_bytes <= kWorkKeep && take_work();
+  rte::KnnFlags flags{};
+  if (test)
+    if (int r = knn_flags(c, &flags)) return r;
+  auto norms_of = [&](const rte::KnnFlags* f) {
+    char* w = c->s_work.as<char>();
+    return rte::launch_row_norms(dx, np, d, stride, c->s_aux3.as<float>(),
+                                 room ? reinterpret_cast<uint16_t*>(w + norm_bytes) : nullptr,
+                                 room ? reinterpret_cast<float*>(w) : nullptr, f, c->stream);
+  };
+  auto fp32 = [&](const rte::KnnFlags* unless) {
+    const int64_t step = 1 << 17;  // rows in launches of 128k (short kernels)
+    for (int64_t r0 = row0; r0 < row0 + nrows; r0 += step) {
+      const int64_t n = std::min<int64_t>(step, row0 + nrows - r0);
+      const hipError_t e = rte::launch_knn(dx, np, d, stride, c->s_aux3.as<float>(), r0, n, k,
+                                           di + (r0 - row0) * k,
+                                           dd ? dd + (r0 - row0) * k : nullptr, unless, c->stream);
+      if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
+  };
+  HIPCHK(c, norms_of(test ? &flags : nullptr), "norms");
+  // The FP32 kernel is queued behind the test and ends at once where that says
+  // whole numbers, so data of other kinds do not wait for the host to hear of it
+  // (65 points: 281 us with a read-back between the two, 264 without the test).
+  if (test) HIPCHK(c, hipEventRecord(c->knn_tested, c->stream), "record test");
+  HIPCHK(c, fp32(test ? &flags : nullptr), "knn launch");
   // whole numbers up to 256 with small norms: one bf16 product in place of an
   // FP32 one, exact either way (160k x 128, k = 64: 2.3 ms in clusters, 18 for
   // uniform values, 75.8 with the FP32 kernel)
-  const bool whole = rte::knn_whole_numbers(bits);
-  if (whole)
-    HIPCHK(c, rte::launch_knn_whole(xb, half, np, d, row0, nrows, k, cus, work, di, dd, c->stream),
-           "knn launch");
-  for (int64_t r0 = row0; !whole && r0 < row0 + nrows; r0 += step) {
-    const int64_t n = std::min<int64_t>(step, row0 + nrows - r0);
-    HIPCHK(c, rte::launch_knn(dx, np, d, stride, norms, r0, n, k, di + (r0 - row0) * k,
-                              dd ? dd + (r0 - row0) * k : nullptr, c->stream),
+  bool whole = false;
+  if (test) {
+    HIPCHK(c, hipEventSynchronize(c->knn_tested), "test values");
+    whole = rte::knn_whole_numbers(rte::knn_flag_bits(c->knn_host, flags.epoch));
+  }
+  if (whole && !room) {
+    room = take_work();
+    if (room) HIPCHK(c, norms_of(nullptr), "norms");
+    else HIPCHK(c, fp32(nullptr), "knn launch");
+  }
+  if (whole && room) {
+    char* w = c->s_work.as<char>();
+    HIPCHK(c, rte::launch_knn_whole(reinterpret_cast<uint16_t*>(w + norm_bytes),
+                                    reinterpret_cast<float*>(w), np, d, row0, nrows, k, cus,
+                                    w + norm_bytes + xb_bytes, di, dd, c->stream),
            "knn launch");
   }
   if (int r = finish_out(c, ids_out, di, (size_t)nrows * k, where)) return r;

@@ -84,6 +84,13 @@ struct rte_ctx {
   // scratch of the graph-building calls, which end with the stream idle
   DevBuf s_work;
 
+  // what a base's values rule out (knn.h, KnnFlags), once in device memory for the
+  // kernels behind the test and once in host memory for rte_knn_rows
+  DevBuf knn_dev;
+  uint32_t* knn_host = nullptr;
+  uint32_t knn_epoch = 0;
+  hipEvent_t knn_tested = nullptr;
+
   // batched search: per-query shapes, query order, work counter, and the
   // captured launch (reused while its key is unchanged)
   DevBuf b_k, b_beam, b_order, b_counter, b_kin, b_bin;
@@ -104,10 +111,11 @@ struct rte_ctx {
 // 1 ms of the 4 ms that lists and graph of 160k points take.  (The set-up calls
 // allocate for themselves: with their scratch kept a fit took 0.4 ms less, but the
 // first allocations of the queries after it 0.3 ms more.)
+constexpr size_t kWorkKeep = (size_t)256 << 20;
 struct WorkGuard {
   rte_ctx* c;
   ~WorkGuard() {
-    if (c->s_work.bytes > (size_t)256 << 20) c->s_work.release();  // hipFree waits for the device
+    if (c->s_work.bytes > kWorkKeep) c->s_work.release();  // hipFree waits for the device
   }
 };
 

@@ -10,10 +10,11 @@ constexpr int kKnnMaxD = 256;    // dims held in registers
 
 // ids/dists: nq x k (k <= kKnnK), the k nearest rows of X (np x d, row stride
 // `stride`) to each of rows [row0, row0 + nq) of X, excluding the row itself,
-// ordered by (squared distance, id).
+// ordered by (squared distance, id).  With `unless`, nothing for whole-number data.
+struct KnnFlags;
 hipError_t launch_knn(const float* X, int64_t np, int d, int64_t stride, const float* norms,
                       int64_t row0, int64_t nq, int k, int32_t* ids, float* dists,
-                      hipStream_t st);
+                      const KnnFlags* unless, hipStream_t st);
 // Search graph from kNN lists (np x kf, by (dist, id)): forward and reverse
 // (ranks < rev_rank) candidates, duplicates keep their smallest (rank, type),
 // each row keeps `degree` by (rank, type, id), padded with np.  `work` holds
@@ -21,17 +22,29 @@ hipError_t launch_knn(const float* X, int64_t np, int d, int64_t stride, const f
 hipError_t launch_graph_from_knn(const int32_t* knn, int64_t np, int kf, int degree, int rev_rank,
                                  int32_t* graph, void* work, hipStream_t st);
 size_t graph_from_knn_work_bytes(int64_t np, int kf, int rev_rank);
-// Row norms of X and what the whole-number kernel needs: the bf16 rows
-// (knn_padded(np) x d), half = -norm / 2 (-inf past np), and in *flag (zero
-// before the call) the bits that rule it out.
+// What rules the whole-number kernel out, a word a bit: the call's epoch where the
+// bit is set, so that nothing is cleared between calls.
 constexpr uint32_t kKnnNotWhole = 1, kKnnNegative = 2, kKnnLarge = 4, kKnnLargeSigned = 8;
-inline bool knn_whole_numbers(uint32_t flag) {
+constexpr int kKnnFlagWords = 4;
+struct KnnFlags {
+  uint32_t* dev;   // device memory
+  uint32_t* host;  // the same in mapped host memory
+  uint32_t epoch;
+};
+__host__ __device__ inline uint32_t knn_flag_bits(const uint32_t* words, uint32_t epoch) {
+  uint32_t bits = 0;
+  for (int b = 0; b < kKnnFlagWords; ++b) bits |= words[b] == epoch ? 1u << b : 0u;
+  return bits;
+}
+__host__ __device__ inline bool knn_whole_numbers(uint32_t flag) {
   return !(flag & (kKnnNotWhole | kKnnLarge)) &&
          (flag & (kKnnNegative | kKnnLargeSigned)) != (kKnnNegative | kKnnLargeSigned);
 }
 inline int64_t knn_padded(int64_t np) { return (np + 63) / 64 * 64; }
+// Row norms of X and, unless null, what the whole-number kernel needs: the bf16
+// rows (knn_padded(np) x d), half = -norm / 2 (-inf past np), and the flags.
 hipError_t launch_row_norms(const float* X, int64_t np, int d, int64_t stride, float* norms,
-                            uint16_t* Xb, float* half, uint32_t* flag, hipStream_t st);
+                            uint16_t* Xb, float* half, const KnnFlags* flags, hipStream_t st);
 // launch_knn for data of which knn_whole_numbers() holds and np <= kKnnWholeMax;
 // same lists, for rows [row0, row0 + nrows).  cus: the card's compute units;
 // `work` has knn_whole_bytes() bytes.

@@ -35,16 +35,15 @@ constexpr int kKnnCols = 64;   // base points per tile
 
 // |x|^2 per row (FP32, dims in order) and, for the whole-number kernel, the
 // bf16 copy of the rows (npad x d, zero past np), -|x|^2 / 2 (-inf past np) and
-// what rules that kernel out: flag bits are set when a value is no whole number
-// of magnitude <= 256 or a row's norm too large for exact sums
-// (knn_whole_numbers).  One workgroup takes 64 rows, staged through LDS so that
+// what rules that kernel out: flags are set when a value is no whole number of
+// magnitude <= 256 or a row's norm too large for exact sums (knn_whole_numbers).  One workgroup takes 64 rows, staged through LDS so that
 // the base is read in whole lines once; bound by that traffic.
 __global__ __launch_bounds__(256) void row_norms_kernel(const float* __restrict__ X, int64_t np,
                                                         int d, int64_t stride, int64_t npad,
                                                         float* __restrict__ norms,
                                                         uint16_t* __restrict__ Xb,
                                                         float* __restrict__ half,
-                                                        uint32_t* __restrict__ flag) {
+                                                        KnnFlags flags) {
   __shared__ float rows[64][128 + 1];
   const int t = threadIdx.x;
   const int64_t r0 = (int64_t)blockIdx.x * 64;
@@ -76,7 +75,15 @@ __global__ __launch_bounds__(256) void row_norms_kernel(const float* __restrict_
     if (half) half[r0 + t] = r0 + t < np ? -0.5f * s : -INFINITY;
   }
   for (int o = 32; o > 0; o >>= 1) bad |= __shfl_xor(bad, o, 64);
-  if (flag && (t & 63) == 0 && bad) atomicOr(flag, bad);
+  if (flags.dev && (t & 63) == 0)
+    for (int b = 0; b < kKnnFlagWords; ++b)
+      if ((bad >> b & 1u) &&
+          __hip_atomic_load(flags.dev + b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) !=
+              flags.epoch) {  // the first waves alone write to the host
+        __hip_atomic_store(flags.dev + b, flags.epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(flags.host + b, flags.epoch, __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_SYSTEM);
+      }
 }
 
 template <int S>  // S = d / 16 (float4 operands per lane)
@@ -84,7 +91,8 @@ __global__ __launch_bounds__(512) void knn_kernel(const float* __restrict__ X, i
                                                   int64_t stride, const float* __restrict__ norms,
                                                   int64_t row0, int64_t nq, int k,
                                                   int32_t* __restrict__ ids_out,
-                                                  float* __restrict__ dists_out) {
+                                                  float* __restrict__ dists_out, KnnFlags unless) {
+  if (unless.dev && knn_whole_numbers(knn_flag_bits(unless.dev, unless.epoch))) return;
   constexpr int LDB = 16 * S + 4;  // floats per point in LDS (padding breaks bank conflicts)
   __shared__ __attribute__((aligned(16))) float Bt[2][kKnnCols * LDB];
   __shared__ float Ld[kKnnRows * kKnnK];
@@ -412,21 +420,21 @@ size_t graph_from_knn_work_bytes(int64_t np, int kf, int rev_rank) {
 }
 
 hipError_t launch_row_norms(const float* X, int64_t np, int d, int64_t stride, float* norms,
-                            uint16_t* Xb, float* half, uint32_t* flag, hipStream_t st) {
+                            uint16_t* Xb, float* half, const KnnFlags* flags, hipStream_t st) {
   const int64_t npad = knn_padded(np);
   hipLaunchKernelGGL(row_norms_kernel, dim3((unsigned)(npad / 64)), dim3(256), 0, st, X, np, d,
-                     stride, npad, norms, Xb, half, flag);
+                     stride, npad, norms, Xb, half, flags ? *flags : KnnFlags{});
   return hipGetLastError();
 }
 
 hipError_t launch_knn(const float* X, int64_t np, int d, int64_t stride, const float* norms,
                       int64_t row0, int64_t nq, int k, int32_t* ids, float* dists,
-                      hipStream_t st) {
+                      const KnnFlags* unless, hipStream_t st) {
   if (nq <= 0) return hipSuccess;
   const dim3 grid((unsigned)((nq + kKnnRows - 1) / kKnnRows));
 #define KNN(S)                                                                                    \
   hipLaunchKernelGGL(knn_kernel<S>, grid, dim3(512), 0, st, X, np, d, stride, norms, row0, nq, k, \
-                     ids, dists)
+                     ids, dists, unless ? *unless : KnnFlags{})
   switch (d / 16) {
     case 2: KNN(2); break;
     case 4: KNN(4); break;

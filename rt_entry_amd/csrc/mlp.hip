@@ -1155,6 +1155,8 @@ void mlp_destroy(Mlp* m) { delete m; }
 rte_ctx::~rte_ctx() {
   rte::mlp_destroy(mlp);
   if (gexec) (void)hipGraphExecDestroy(gexec);
+  if (knn_host) (void)hipHostFree(knn_host);
+  if (knn_tested) (void)hipEventDestroy(knn_tested);
 }
 
 namespace {
