@@ -43,7 +43,6 @@ constexpr int kWnQueue = 416;  // queued points per wave: a block's 256 and some
 constexpr int kWnWaves = 4;    // of a workgroup
 constexpr int kWnRows = 32 * kWnWaves;
 constexpr int kWnPerCu = 2;    // workgroups
-constexpr int kWnGroup = 1;    // tiles between barriers
 constexpr int kWnKeys = 128;   // of a row: 64 list, 64 buffer
 constexpr int kWnPivots = 1024;
 constexpr int kWnBuckets = 32;  // of a cell, by distance from its pivot
@@ -386,7 +385,7 @@ __global__ __launch_bounds__(256) void wn_meta_kernel(WnLayout l) {
 // ---- the lists --------------------------------------------------------------
 // 64 lanes x 16 (or 4) bytes from global memory to LDS at `dst` + 16 (4) * lane.
 // As asm, so that the compiler does not wait for it before every LDS read that
-// might alias; the kernel waits once, before the group's barrier.
+// might alias; the kernel waits once, before the tile's barrier.
 __device__ __forceinline__ void wn_copy16(const void* src, uint32_t dst) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(dst), "v"(src)
                : "memory", "m0");
@@ -432,7 +431,8 @@ struct WnArgs {
 // tiles (16-byte units XOR-swizzled per point), one barrier a tile; two
 // workgroups a compute unit, since a wave's points to pick differ from tile to tile
 // and a workgroup waits for its slowest wave (one of eight waves, three tiles to a
-// barrier: 4.0 ms at 160k x 128, two: 2.6).  A point nearer than its row's threshold (the k-th best of the row's list) goes to the wave's queue -- writes
+// barrier: 4.0 ms at 160k x 128, two: 2.6).  A point nearer than its row's
+// threshold (the k-th best of the row's list) goes to the wave's queue -- writes
 // only, no round trip through LDS -- and 64 at a time to the rows' buffers.  A
 // buffer is sorted across the wave and merged with its row's sorted list when it
 // is full, in all rows at tiles 0, 1, 2, 4, ... times 1.8 (a point enters the k
@@ -448,7 +448,7 @@ __global__ __launch_bounds__(64 * kWnWaves, 2) void knn_whole_kernel(WnArgs a) {
   constexpr int D = 32 * KS;
   constexpr int ROWS = kWnRows;
   constexpr uint64_t kNone = ~0ull;
-  __shared__ __attribute__((aligned(16))) uint4 ring[2 * kWnGroup * W::SLOT];
+  __shared__ __attribute__((aligned(16))) uint4 ring[2 * W::SLOT];
   __shared__ uint2 qe[kWnWaves][kWnQueue];  // a wave's queue: product, row << 27 | id
   __shared__ int cnt[ROWS];
   __shared__ float thr[ROWS];  // -(k-th best distance) / 2 + |q|^2 / 2
@@ -465,7 +465,7 @@ __global__ __launch_bounds__(64 * kWnWaves, 2) void knn_whole_kernel(WnArgs a) {
   const int r = lane & 15, g = lane >> 4;
   const int lrow0 = 32 * wave;  // the wave's rows in the workgroup
   const uint32_t ring0 = (uint32_t)(uintptr_t)(lds_void_t*)ring;
-  constexpr uint32_t kHalf = 16u * kWnGroup * W::SLOT;
+  constexpr uint32_t kHalf = 16u * W::SLOT;
   const int ntile = a.l.cstart[a.l.pivots] / kWnCols;
   uint64_t* const keys = a.l.keys + ((int64_t)blockIdx.x * ROWS + lrow0) * kWnKeys + lane;
   while (true) {
@@ -654,28 +654,24 @@ __global__ __launch_bounds__(64 * kWnWaves, 2) void knn_whole_kernel(WnArgs a) {
       wave_sync();
       load_thr();
     };
-    // a tile's operands in registers: a step's are read again, for the next
-    // tile, as soon as its products are under way, so that LDS and the matrix
-    // unit work at the same time and the picking waits for neither
-    uint4 b[KS][4];
-    float hx[4];
-    auto fetch_half = [&](const uint4* Bt, float (&h)[4]) {
+    // one tile: products, then the points that pass.  All its operands are asked
+    // for before the first product: left to itself the compiler reads them between
+    // the products and waits for each (160k x 128 uniform 17.5 -> 19.1 ms).
+    auto tile = [&](const uint4* Bt) {
       const float* ht = reinterpret_cast<const float*>(Bt + W::UNITS);
+      uint4 b[KS][4];
+      float hx[4];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) h[j] = ht[16 * j + r];
-    };
-    auto fetch_step = [&](const uint4* Bt, int s) {
+      for (int j = 0; j < 4; ++j) hx[j] = ht[16 * j + r];
 #pragma unroll
-      for (int j = 0; j < 4; ++j)
-        b[s][j] = Bt[(16 * j + r) * W::CPR + ((4 * s + g) ^ (r & W::SWM))];
-    };
-    // one tile: products, then the points that pass
-    auto tile = [&](const uint4* Bt, const uint4* following) {
+      for (int s = 0; s < KS; ++s)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          b[s][j] = Bt[(16 * j + r) * W::CPR + ((4 * s + g) ^ (r & W::SWM))];
+      __builtin_amdgcn_sched_barrier(0);
       floatx4 acc[2][4];
-      float hn[4] = {0.f, 0.f, 0.f, 0.f};
-      fetch_half(following, hn);
 #pragma unroll
-      for (int s = 0; s < KS; ++s) {
+      for (int s = 0; s < KS; ++s)
 #pragma unroll
         for (int j = 0; j < 4; ++j)
 #pragma unroll
@@ -683,17 +679,11 @@ __global__ __launch_bounds__(64 * kWnWaves, 2) void knn_whole_kernel(WnArgs a) {
             acc[rb][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
                 __builtin_bit_cast(bf16x8, A[rb][s]), __builtin_bit_cast(bf16x8, b[s][j]),
                 s ? acc[rb][j] : floatx4{hx[j], hx[j], hx[j], hx[j]}, 0, 0, 0);
-        __builtin_amdgcn_sched_barrier(0);
-        fetch_step(following, s);
-        __builtin_amdgcn_sched_barrier(0);
-      }
       int idx[4];
 #pragma unroll
       for (int j = 0; j < 4; ++j)
         idx[j] = reinterpret_cast<const int*>(Bt + W::UNITS + 16)[16 * j + r];
       asm volatile("" ::: "memory");  // the reads stay here
-#pragma unroll
-      for (int j = 0; j < 4; ++j) hx[j] = hn[j];
       // points that pass, block (rb, v) by block; a block that the queue may
       // have no room for (the first tiles) is left for the loop below.  What
       // is done with them lies out of line: a tile's branches fall through
@@ -800,36 +790,25 @@ __global__ __launch_bounds__(64 * kWnWaves, 2) void knn_whole_kernel(WnArgs a) {
         __syncthreads();
         const int n = __builtin_amdgcn_readfirstlane(listed);
         if (n == 0) continue;
-        auto copy_group = [&](int g0, uint32_t dst) {
-#pragma unroll 1
-          for (int j = 0; j < kWnGroup && g0 + j < n; ++j)
-            wn_copy_tile<KS>(a.l.Xs, a.l.hs, a.l.sid,
-                                 (int64_t)__builtin_amdgcn_readfirstlane(list[g0 + j]) * kWnCols,
-                                 dst + 16u * (uint32_t)(j * W::SLOT), wave, lane);
+        auto copy_tile = [&](int i, uint32_t dst) {
+          wn_copy_tile<KS>(a.l.Xs, a.l.hs, a.l.sid,
+                           (int64_t)__builtin_amdgcn_readfirstlane(list[i]) * kWnCols, dst, wave,
+                           lane);
         };
-        copy_group(0, ring0);
-        uint32_t here = 0;  // the ring's half that holds the group
-        for (int g0 = 0; g0 < n; g0 += kWnGroup) {
-          // the group's copies have landed (each wave waits for its own) and
+        copy_tile(0, ring0);
+        uint32_t here = 0;  // the ring's half that holds the tile
+        for (int i = 0; i < n; ++i) {
+          // the tile's copies have landed (each wave waits for its own) and
           // every wave is done with the other half
           __builtin_amdgcn_s_waitcnt(0x0f70);
           __syncthreads();
-          if (g0 + kWnGroup < n) copy_group(g0 + kWnGroup, ring0 + (kHalf - here));
-          const int m = min(kWnGroup, n - g0);
-          const uint4* Bt = ring + here / 16;
-          fetch_half(Bt, hx);
-#pragma unroll
-          for (int s = 0; s < KS; ++s) fetch_step(Bt, s);
-#pragma unroll 1
-          for (int j = 0; j < m; ++j) {
-            tile(Bt, j + 1 < m ? Bt + W::SLOT : Bt);  // past the group's last: not used
-            Bt += W::SLOT;
-            if (seen >= next) {
-              flush_all();
-              next = seen + 1 + 8 * seen / 10;
-            }
-            ++seen;
+          if (i + 1 < n) copy_tile(i + 1, ring0 + (kHalf - here));
+          tile(ring + here / 16);
+          if (seen >= next) {
+            flush_all();
+            next = seen + 1 + 8 * seen / 10;
           }
+          ++seen;
           here = kHalf - here;
         }
         flush_all();
