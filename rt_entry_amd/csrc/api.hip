@@ -179,7 +179,7 @@ int knn_flags(rte_ctx* c, rte::KnnFlags* f) {
     HIPCHK(c, hipMemsetAsync(c->knn_dev.p, 0, bytes, c->stream), "clear flags");
     c->knn_epoch = 1;
   }
-  *f = rte::KnnFlags{c->knn_dev.as<uint32_t>(), c->knn_host, c->knn_epoch};
+  *f = rte::KnnFlags{c->knn_dev.as<uint32_t>(), c->knn_host, c->knn_epoch, false};
   return RTE_OK;
 }
 
@@ -421,6 +421,7 @@ int rte_knn_rows(rte_ctx* c, const float* X, int64_t np, int d, int64_t stride, 
   rte::KnnFlags flags{};
   if (test)
     if (int r = knn_flags(c, &flags)) return r;
+  flags.varied = rte::knn_varied_only(np, cus);
   auto norms_of = [&](const rte::KnnFlags* f) {
     char* w = c->s_work.as<char>();
     return rte::launch_row_norms(dx, np, d, stride, c->s_aux3.as<float>(),
@@ -450,7 +451,7 @@ int rte_knn_rows(rte_ctx* c, const float* X, int64_t np, int d, int64_t stride, 
   bool whole = false;
   if (test) {
     HIPCHK(c, hipEventSynchronize(c->knn_tested), "test values");
-    whole = rte::knn_whole_numbers(rte::knn_flag_bits(c->knn_host, flags.epoch));
+    whole = rte::knn_whole_numbers(rte::knn_flag_bits(c->knn_host, flags.epoch), flags.varied);
   }
   if (whole && !room) {
     room = take_work();

@@ -36,7 +36,9 @@ constexpr int kKnnCols = 64;   // base points per tile
 // |x|^2 per row (FP32, dims in order) and, for the whole-number kernel, the
 // bf16 copy of the rows (npad x d, zero past np), -|x|^2 / 2 (-inf past np) and
 // what rules that kernel out: flags are set when a value is no whole number of
-// magnitude <= 256 or a row's norm too large for exact sums (knn_whole_numbers).  One workgroup takes 64 rows, staged through LDS so that
+// magnitude <= 256 or a row's norm too large for exact sums (knn_whole_numbers),
+// and when a workgroup's rows differ: fewer than a seventh of 192 pairs of them have
+// equal norms, pairs at least 11 rows apart (a point and its copies may be closer).  One workgroup takes 64 rows, staged through LDS so that
 // the base is read in whole lines once; bound by that traffic.
 __global__ __launch_bounds__(256) void row_norms_kernel(const float* __restrict__ X, int64_t np,
                                                         int d, int64_t stride, int64_t npad,
@@ -73,6 +75,10 @@ __global__ __launch_bounds__(256) void row_norms_kernel(const float* __restrict_
       bad |= s < 4194304.f ? 0u : kKnnLargeSigned;  // 2^22
     }
     if (half) half[r0 + t] = r0 + t < np ? -0.5f * s : -INFINITY;
+    int equal = 0;
+    for (int o : {32, 53, 42})
+      equal += __popcll(__builtin_amdgcn_ballot_w64(s == __shfl_xor(s, o, 64)));
+    if (equal < 28 && r0 + 64 <= np) bad |= kKnnVaried;  // of 192
   }
   for (int o = 32; o > 0; o >>= 1) bad |= __shfl_xor(bad, o, 64);
   if (flags.dev && (t & 63) == 0)
@@ -92,7 +98,8 @@ __global__ __launch_bounds__(512) void knn_kernel(const float* __restrict__ X, i
                                                   int64_t row0, int64_t nq, int k,
                                                   int32_t* __restrict__ ids_out,
                                                   float* __restrict__ dists_out, KnnFlags unless) {
-  if (unless.dev && knn_whole_numbers(knn_flag_bits(unless.dev, unless.epoch))) return;
+  if (unless.dev && knn_whole_numbers(knn_flag_bits(unless.dev, unless.epoch), unless.varied))
+    return;
   constexpr int LDB = 16 * S + 4;  // floats per point in LDS (padding breaks bank conflicts)
   __shared__ __attribute__((aligned(16))) float Bt[2][kKnnCols * LDB];
   __shared__ float Ld[kKnnRows * kKnnK];
