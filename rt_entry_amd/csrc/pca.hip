@@ -310,6 +310,61 @@ __global__ __launch_bounds__(512) void pca_rotate_kernel(const float* __restrict
   }
 }
 
+// The same for few columns, four or eight a wave: all four waves stage the rows, the
+// next 64 columns of X on their way during the products, and R's come from LDS,
+// widened there, so one launch does it.  The kernel above has a wave or two a
+// workgroup here, which stage 64 rows alone and wait for scalar loads at every column
+// of X.  Bound by the launch and a few round trips at 1000 x 128 to 3 columns (34 us
+// with both copies to the device, 70 with the kernel above), by memory and LDS (three
+// reads for 8 operations a wave) at 1M x 96 to 3: 174 us, 2.3 TB/s.
+template <int C>  // columns a wave
+__global__ __launch_bounds__(256) void pca_rotate_narrow_kernel(
+    const float* __restrict__ X, int64_t n, int d, int64_t stride, const float* __restrict__ R,
+    const float* __restrict__ mu, int d_out, float* __restrict__ out) {
+  constexpr int kPitch = kRotRows + 1, kPer = kRotRows / 4, kCols = 4 * C;
+  __shared__ double xs[kRotK * kPitch];
+  __shared__ __attribute__((aligned(16))) double rs[kRotK * kCols];
+  const int t = threadIdx.x, lane = t & 63;
+  const int w = __builtin_amdgcn_readfirstlane(t >> 6), c0 = C * w;
+  const int64_t row0 = (int64_t)blockIdx.x * kRotRows;
+  double acc[C];
+#pragma unroll
+  for (int i = 0; i < C; ++i) acc[i] = 0.0;
+  float v[kPer];
+  auto load = [&](int j0) {  // at clamped, valid addresses
+    const int j = min(j0 + lane, d - 1);
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) v[i] = X[min(row0 + w + 4 * i, n - 1) * stride + j];
+  };
+  load(0);
+  for (int j0 = 0; j0 < d; j0 += kRotK) {
+    const int jn = d - j0 < kRotK ? d - j0 : kRotK;
+    const double m = (double)mu[min(j0 + lane, d - 1)];
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) xs[lane * kPitch + w + 4 * i] = (double)v[i] - m;
+    for (int e = t; e < kRotK * kCols; e += 256) {
+      const int k = e / kCols, c = e % kCols;
+      rs[e] = k < jn && c < d_out ? (double)R[(int64_t)(j0 + k) * d_out + c] : 0.0;
+    }
+    __syncthreads();
+    if (j0 + kRotK < d) load(j0 + kRotK);
+    if (c0 < d_out) {
+#pragma unroll 8
+      for (int k = 0; k < jn; ++k) {
+        const double x = xs[k * kPitch + lane];
+#pragma unroll
+        for (int i = 0; i < C; ++i) acc[i] = acc[i] + x * rs[k * kCols + c0 + i];
+      }
+    }
+    __syncthreads();
+  }
+  const int64_t row = row0 + lane;
+  if (row < n)
+#pragma unroll
+    for (int i = 0; i < C; ++i)
+      if (c0 + i < d_out) out[row * d_out + c0 + i] = (float)acc[i];
+}
+
 // Symmetric eigen-decomposition (FP64): the published EISPACK method,
 // tred2 (Householder reduction to tridiagonal form, accumulating the
 // transformations) followed by tql2 (QL iterations with implicit shifts on
@@ -573,9 +628,13 @@ int rte_pca_rotate(rte_ctx* c, const float* X, int64_t n, int d, int64_t stride,
     dx = xin.as<float>();
     dout = ob.as<float>();
   }
-  // R (d x d_out) and mu (d) are host arrays; R widened comes first
+  // R (d x d_out) and mu (d) are host arrays; R widened, where it is, comes first
+  // up to 16 columns at any n (1M x 96 to 3: 460 -> 174 us, 20k x 960 to 3: 365 -> 82);
+  // up to 32 while there are too few rows to hide the wide kernel's chain (20k x 960
+  // to 32: 340 -> 225, 1000 x 128 to 17: 67 -> 50; but 1M x 32 to 32 192 -> 272)
+  const bool narrow = d_out <= 16 || (d_out <= 32 && n <= 65536);
   const int ldr = (d_out + rte::kRotCols - 1) / rte::kRotCols * rte::kRotCols;
-  const size_t wide = (size_t)(d + 1) * ldr;
+  const size_t wide = narrow ? 0 : (size_t)(d + 1) * ldr;
   if (int r = ck(rm.reserve(wide * sizeof(double) + ((size_t)d * d_out + d) * sizeof(float)),
                  "hipMalloc"))
     return r;
@@ -586,13 +645,20 @@ int rte_pca_rotate(rte_ctx* c, const float* X, int64_t n, int d, int64_t stride,
     return r;
   if (int r = ck(hipMemcpyAsync(dmu, mu, (size_t)d * 4, hipMemcpyHostToDevice, st), "copy"))
     return r;
-  hipLaunchKernelGGL(rte::widen_kernel, dim3((unsigned)((wide + 255) / 256)), dim3(256), 0, st, dR,
-                     d, d_out, ldr, dW);
-  dim3 grid((unsigned)((n + rte::kRotRows - 1) / rte::kRotRows),
-            (unsigned)((d_out + rte::kPcaTile - 1) / rte::kPcaTile));
-  const int waves = std::min(ldr, rte::kPcaTile) / rte::kRotCols;
-  hipLaunchKernelGGL(rte::pca_rotate_kernel, grid, dim3(64 * waves), 0, st, dx, n, d, stride, dW,
-                     ldr, dmu, d_out, dout);
+  const unsigned blocks = (unsigned)((n + rte::kRotRows - 1) / rte::kRotRows);
+  if (narrow) {
+    auto* kernel =
+        d_out <= 16 ? rte::pca_rotate_narrow_kernel<4> : rte::pca_rotate_narrow_kernel<8>;
+    hipLaunchKernelGGL(kernel, dim3(blocks), dim3(256), 0, st, dx, n, d, stride, dR, dmu, d_out,
+                       dout);
+  } else {
+    hipLaunchKernelGGL(rte::widen_kernel, dim3((unsigned)((wide + 255) / 256)), dim3(256), 0, st,
+                       dR, d, d_out, ldr, dW);
+    const int waves = std::min(ldr, rte::kPcaTile) / rte::kRotCols;
+    hipLaunchKernelGGL(rte::pca_rotate_kernel,
+                       dim3(blocks, (unsigned)((d_out + rte::kPcaTile - 1) / rte::kPcaTile)),
+                       dim3(64 * waves), 0, st, dx, n, d, stride, dW, ldr, dmu, d_out, dout);
+  }
   if (int r = ck(hipGetLastError(), "pca_rotate kernel")) return r;
   if (where == RTE_HOST) {
     if (int r = ck(hipMemcpyAsync(out, dout, obytes, hipMemcpyDeviceToHost, st), "copy")) return r;
