@@ -746,7 +746,8 @@ int rte_build_kdtree_gpu(rte_ctx* c, const float* pts, int64_t np, int64_t strid
   for (int64_t n = np; n > kKdSmall; n = (n + 1) / 2) ++rounds;
   if (rounds) ++rounds;
   Header hh{};
-  for (int r = 0;; ++r) {
+  hh.ns = 1;  // a root that is a small node needs no rounds and no read-back
+  for (int r = 0; rounds > 0; ++r) {
     const int par = r & 1;
     if (r >= rounds) {
       KCK(hipGetLastError(), "kd-tree kernels");
