@@ -98,7 +98,8 @@ typedef struct rte_params {
 /* Replaces Graph::Graph + cublasCreate (graph.cu:32-64). */
 int rte_create(rte_ctx** ctx, int device);
 /* Replaces Graph::CleanUp / OptiXRT::CleanUp (graph.cu:339-342,
- * raytracing.cpp:263-281). */
+ * raytracing.cpp:263-281).  The context's own stream is kept idle for a later
+ * context on the device (at most 64 are). */
 int rte_destroy(rte_ctx* ctx);
 const char* rte_last_error(const rte_ctx* ctx);
 /* Use the caller's HIP stream (hipStream_t) instead of the context's own;
@@ -202,8 +203,12 @@ int rte_pca_rotate(rte_ctx* ctx, const float* X, int64_t n, int d, int64_t strid
 /* ---- graph construction ------------------------------------------------ */
 /* Exact k nearest neighbours of every row of X (np x d, row stride `stride`)
  * among the rows of X, itself excluded, ordered by (squared L2 distance,
- * id): ids_out/dists_out np x k (dists may be NULL).  FP32 MFMA distances
- * |q|^2 + |x|^2 - 2 q.x; exact for integer-valued data with |x|^2 < 2^24.
+ * id): ids_out/dists_out np x k (dists may be NULL).  Distances |q|^2 + |x|^2 -
+ * 2 q.x in FP32, exact for integer-valued data with |x|^2 < 2^24.  Whole numbers
+ * of magnitude <= 256 with |x|^2 < 2^23 (2^22 with negative ones) and np <= 2^27
+ * take one bf16 product over points grouped by cells, where its scratch (about
+ * 4 d + 30 bytes a point and up to 70 MB) can be allocated: same lists and distances.
+ * A context keeps up to 256 MiB of scratch for the next call.
  * d in {32, 64, 96, 128}, k <= 64, stride % 4 == 0.  No reference
  * counterpart: the reference loads prebuilt .nsw graphs and leaves graph
  * building as a TODO (graph.cu:114-139). */
@@ -211,7 +216,8 @@ int rte_knn(rte_ctx* ctx, const float* X, int64_t np, int d, int64_t stride, int
             int32_t* ids_out, float* dists_out, int where);
 
 /* rte_knn for the rows [row0, row0 + nrows) of X only, still against all np
- * rows: ids_out/dists_out nrows x k.  A large build can run in pieces
+ * rows: ids_out/dists_out nrows x k; whole numbers are grouped anew in every
+ * call.  A large build can run in pieces
  * (progress between calls, bounded output staging) or split its row ranges
  * across devices that each hold X.  No reference counterpart (as rte_knn). */
 int rte_knn_rows(rte_ctx* ctx, const float* X, int64_t np, int d, int64_t stride, int64_t row0,

@@ -589,10 +589,8 @@ int rte_set_pca(rte_ctx* c, const float* R, const float* mu, int d, int r_cols, 
   HIPCHK(c, c->rot.reserve((size_t)d * d_out * sizeof(float)), "hipMalloc(rot)");
   HIPCHK(c, c->bias.reserve((size_t)d_out * sizeof(float)), "hipMalloc(bias)");
   const hipMemcpyKind kind = where == RTE_HOST ? hipMemcpyHostToDevice : hipMemcpyDeviceToDevice;
-  // keep the first d_out columns (graph.cu:196 CopyHostToDevice(..., DIM)).  A
-  // host matrix is packed here and copied flat: under a profiler's queue
-  // interception a 2D copy from the host left L2 with what the memory held
-  // before (the covariance of a fit that had just been freed).
+  // keep the first d_out columns (graph.cu:196 CopyHostToDevice(..., DIM)); a
+  // host matrix is packed here and copied flat
   std::vector<float> packed;
   if (where == RTE_HOST && r_cols > d_out) {
     packed.resize((size_t)d * d_out);
