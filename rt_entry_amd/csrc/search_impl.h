@@ -21,8 +21,8 @@
 //    one iteration issues its loads together and only for points that need a
 //    distance; a lane reads its half-wave's ids in 16-byte LDS reads and
 //    forms each row address with one 32x32->64 multiply-add;
-//  - in beams of up to 64 slots a batch of which few elements enter is merged by
-//    ranks through LDS instead of by the networks (rank_merge, use_ranks);
+//  - a batch of which few elements enter is merged by ranks through LDS instead of
+//    by the networks where that is faster (rank_merge, use_ranks);
 //  - the FAST kernels (one row per iteration, whole 32-dim groups up to 256 dims,
 //    32-bit row offsets) have the graph row expected next on its way while the
 //    current distances are gathered.
@@ -421,14 +421,17 @@ struct Beam<NR, false> {
     return __int_as_float(s.mbuf[s0 + slot].x);
   }
   __device__ __forceinline__ void undo(int, int, const float (&)[NR], const int (&)[NR]) const {}
+  __device__ __forceinline__ void take_slot(int r, int n, int lane, float v, int id) {
+    const bool in = lane < n - r * 64;  // lanes past the beam stay kMaxD
+    d[r] = in ? v : d[r];
+    i[r] = in ? id : i[r];
+  }
   __device__ __forceinline__ void take_merged(int n, int lane, const float (&nd)[NR],
                                               const int (&ni)[NR]) {
 #pragma unroll
     for (int r = 0; r < NR; ++r) {
       if (r * 64 >= n) continue;
-      const bool in = lane < n - r * 64;  // lanes past the beam stay kMaxD
-      d[r] = in ? nd[r] : d[r];
-      i[r] = in ? ni[r] : i[r];
+      take_slot(r, n, lane, nd[r], ni[r]);
     }
   }
 };
@@ -593,25 +596,29 @@ constexpr int kRankMax = 24;
 
 constexpr int ilog2c(int x) { return x <= 1 ? 0 : 1 + ilog2c(x / 2); }
 
-// Beams of up to 64 slots (one register a lane) merge a batch of few entering
-// elements by ranks; with several waves a query, each of which repeats the merge,
-// beams of up to 32.  Past that the networks alone are as fast or faster, ranks
-// taking a second copy of the beam in registers and more LDS, but for TUNED's
-// two-key networks over batches of 128.  Networks alone -> with ranks, us: 100
-// queries at beam 16, d = 96, width 4 60 -> 52; 10k at beam 64, d = 64 in leaf order
-// 319 -> 304; 3k at beam 128, d = 100, width 4, TUNED 331 -> 324; but 100 at beam
-// 64, d = 128, four waves a query 104 -> 112; 10k at beam 128, d = 64 in leaf order
-// 369 -> 402 and d = 96, TUNED 616 -> 667; at beam 256, d = 64 622 -> 740 and at beam
-// 512, d = 128 1060 -> 1495.
-constexpr int kRanksWaves = 32;  // slots, for several waves a query
-template <bool TUNED, int NR, int MR>
+// Where a batch of few entering elements is merged by ranks: they take a second
+// copy of the beam in registers and more LDS, against networks that grow with the
+// beam and cost TUNED, which compares two keys, twice.
+//  - beams of up to 64 slots (REF with several waves a query, each of which
+//    repeats the merge: up to 32);
+//  - TUNED up to 128 slots, with the beam in LDS at any size, and in the FAST
+//    kernels up to 256 slots while four waves per SIMD are left (d up to 128: 88,
+//    105 and 121 VGPRs).
+// Networks alone -> with ranks, us.  100 queries at beam 16, d = 96, width 4 60 -> 52;
+// 10k in leaf order at beam 64, d = 64 319 -> 304; TUNED on unit vectors, beam 128, d =
+// 64 601 -> 546 and d = 96 583 -> 570, beam 256, d = 96 839 -> 794 and d = 128 859 -> 815.
+// But REF: 100 at beam 64, d = 128, four waves a query 104 -> 112; 10k at beam 128, d =
+// 64 369 -> 402, at beam 256 622 -> 740, at beam 512, d = 128 1060 -> 1495.  TUNED on
+// mixtures of whole numbers, where few steps have an element that enters, loses up
+// to 13% (d = 96, beam 128) by the registers that ranks take.
+constexpr int kRanksWaves = 32;  // slots
+template <bool TUNED, int NR, int MR, int J, bool LQ, bool FAST>
 constexpr bool use_ranks() {
-  return NR == 1 || (TUNED && NR == 2 && MR == 2);
+  return NR == 1 || (TUNED && (NR == 2 || LQ || (NR == 4 && FAST && J <= 4)));
 }
 
-template <bool TUNED, int NR, int MR, int J, int WPQ, bool FAST>
+template <bool TUNED, int NR, int MR, int J, int WPQ, bool FAST, bool RANKS>
 struct SearchCore {
-  static constexpr bool RANKS = use_ranks<TUNED, NR, MR>();
   // points per half-wave in one load group: all 16 when the vectors fit in
   // 64 VGPRs, so one iteration's gathers are issued together; with WPQ
   // waves per query each wave takes 1/WPQ of them
@@ -835,13 +842,9 @@ struct SearchCore {
       const int o = in ? s.eo[rk[r]] : 0;
       odd |= __builtin_amdgcn_ballot_w64(in && o != ci[r]);
     }
+    // slot r*64 + lane: its beam key f, moved, and what the beam then has there
     int holes = 0;
-    float nd[NR], top = -1.0f;  // top: slot r*64 - 1
-    int ni[NR];
-#pragma unroll
-    for (int r = 0; r < NR; ++r) {
-      if (r * 64 >= n) continue;
-      float f;
+    auto merged = [&](int r, float& f, float& v, int& id) {
       int fi;
       L.get(s, r * 64, lane, f, fi);
       const bool hole = lane < n - r * 64 && f < 0.0f;
@@ -851,8 +854,17 @@ struct SearchCore {
       holes += __popcll(hm);
       // read by every lane (k <= cnt is inside the buffers), used by the holes
       const int2 x = s.es[k];
-      nd[r] = hole ? __int_as_float(x.x) : f;
-      ni[r] = hole ? x.y : fi;
+      v = hole ? __int_as_float(x.x) : f;
+      id = hole ? x.y : fi;
+      return hole;
+    };
+    float nd[NR], top = -1.0f;  // top: slot r*64 - 1
+    int ni[NR];
+#pragma unroll
+    for (int r = 0; r < NR; ++r) {
+      if (r * 64 >= n) continue;
+      float f;
+      const bool hole = merged(r, f, nd[r], ni[r]);
       // a beam key equal to the element in a hole is in the slot below it
       const float below = prev_lane(f, top);
       odd |= __builtin_amdgcn_ballot_w64(hole && below == nd[r]);
@@ -861,7 +873,24 @@ struct SearchCore {
     // slot n, the first that drops out
     if (L.dist_in(s, n, 0) < 0.0f)
       odd |= __builtin_amdgcn_ballot_w64(L.dist_in(s, n - 1, 0) == __int_as_float(s.es[holes].x));
-    wave_sync();  // the slots are read before anything is written over them
+    if constexpr (!BeamT::kInLds && NR >= 4) {
+      // formed again from LDS, so that the old slots and the new ones are not in
+      // registers together
+      if (!odd) {
+        holes = 0;
+#pragma unroll
+        for (int r = 0; r < NR; ++r) {
+          if (r * 64 >= n) continue;
+          float f, v;
+          int id;
+          merged(r, f, v, id);
+          L.take_slot(r, n, lane, v, id);
+        }
+      }
+      wave_sync();  // the slots are read before anything is written over them
+      return !odd;
+    }
+    wave_sync();
     if (odd) {
       L.undo(n, lane, ld, li);
       return false;
@@ -1102,19 +1131,19 @@ __host__ __device__ constexpr int filter_words(int w) { return (w + 3) & ~3; }
 // lie over them -- and for a beam held in LDS its queue of 64*NR (distance, id)
 // slots and one more, each array in whole 16 bytes
 constexpr int kRankWords = (kRankMax + 4) + kRankMax + 2 * kRankMax;
-template <int MR, int NR>
+template <int NR, bool RANKS>
 __host__ __device__ constexpr int queue_words() {
-  return 64 * NR + (use_ranks<true, NR, MR>() ? 4 : 0);
+  return 64 * NR + (RANKS ? 4 : 0);
 }
-template <int MR, int WPQ, int NR, bool LQ>
+template <int MR, int WPQ, int NR, bool LQ, bool RANKS>
 __host__ __device__ constexpr int batch_words() {
   constexpr int batch = (WPQ > 1 ? 3 : 4) * 64 * MR;
-  constexpr int merge = use_ranks<true, NR, MR>() ? kRankWords + (LQ ? 0 : 2 * 64 * NR + 4) : 0;
+  constexpr int merge = RANKS ? kRankWords + (LQ ? 0 : 2 * 64 * NR + 4) : 0;
   return batch > merge ? batch : merge;
 }
-template <int MR, int WPQ, int NR, bool LQ>
+template <int MR, int WPQ, int NR, bool LQ, bool RANKS>
 __host__ __device__ constexpr int lds_words_wave() {
-  return batch_words<MR, WPQ, NR, LQ>() + (LQ ? 2 * queue_words<MR, NR>() : 0);
+  return batch_words<MR, WPQ, NR, LQ, RANKS>() + (LQ ? 2 * queue_words<NR, RANKS>() : 0);
 }
 // LDS words a query shares between its waves (WPQ > 1): two distance
 // buffers (alternating batches) and the broadcast slot of the work queue
@@ -1125,7 +1154,8 @@ __host__ __device__ constexpr int lds_words_query() {
 
 template <bool TUNED, int NR, int MR, int J, int WPQ, bool LQ, bool FAST>
 __global__ __launch_bounds__(256) void search_kernel(SearchArgs a) {
-  using Core = SearchCore<TUNED, NR, MR, J, WPQ, FAST>;
+  constexpr bool RANKS = use_ranks<TUNED, NR, MR, J, LQ, FAST>();
+  using Core = SearchCore<TUNED, NR, MR, J, WPQ, FAST, RANKS>;
   extern __shared__ uint32_t smem[];
   const int lane = threadIdx.x & 63;
   // one value per wave: as a scalar it keeps the query's slot, its addresses
@@ -1133,7 +1163,7 @@ __global__ __launch_bounds__(256) void search_kernel(SearchArgs a) {
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int sub = wave % WPQ;  // this wave's share of the query's distances
   const int fwords = filter_words(a.bloom_words_max);
-  const int region = fwords + lds_words_wave<MR, WPQ, NR, LQ>();
+  const int region = fwords + lds_words_wave<MR, WPQ, NR, LQ, RANKS>();
   uint32_t* base_lds = smem + wave * region;
   // shared by the query's waves (WPQ > 1; one query per workgroup)
   uint32_t* qshared = smem + (blockDim.x >> 6) * region;
@@ -1181,8 +1211,8 @@ __global__ __launch_bounds__(256) void search_kernel(SearchArgs a) {
     s.eo = (int*)(s.ed + kRankMax + 4);
     s.es = (int2*)(s.eo + kRankMax);
     s.mbuf = LQ ? nullptr : s.es + kRankMax;
-    s.qd = LQ ? (float*)(base_lds + fwords + batch_words<MR, WPQ, NR, LQ>()) : nullptr;
-    s.qi = LQ ? (int*)(s.qd + queue_words<MR, NR>()) : nullptr;
+    s.qd = LQ ? (float*)(base_lds + fwords + batch_words<MR, WPQ, NR, LQ, RANKS>()) : nullptr;
+    s.qi = LQ ? (int*)(s.qd + queue_words<NR, RANKS>()) : nullptr;
     // the hash count is fixed per mode (kHashes), checked on the host
     Bloom<kHashes<TUNED>> bl{s.bloom, (uint32_t)bwords, (uint32_t)(31 - __clz(bwords)),
                              (uint32_t)bwords * 32u};
@@ -1214,7 +1244,7 @@ __global__ __launch_bounds__(256) void search_kernel(SearchArgs a) {
     uint32_t seed = (uint32_t)(q * 64 + lane);  // :66
     int nE = 0, nX = 0;
     // no equal keys met yet (merge_batch)
-    bool plain = Core::RANKS && (WPQ == 1 || n <= kRanksWaves);
+    bool plain = RANKS && (TUNED || WPQ == 1 || n <= kRanksWaves);
     int vpre = -1, gpre = npi;  // FAST: node whose graph row gpre holds or awaits
 
     // ---- entry seeding, :479-959
@@ -1390,15 +1420,17 @@ __global__ __launch_bounds__(256) void search_kernel(SearchArgs a) {
   }
 }
 
-template <int MR, int WPQ, int NR, bool LQ>
+template <int MR, int WPQ, int NR, bool LQ, bool RANKS>
 size_t search_lds_bytes(int bloom_words_max, int wpb) {
-  return ((size_t)wpb * (filter_words(bloom_words_max) + lds_words_wave<MR, WPQ, NR, LQ>()) +
+  return ((size_t)wpb * (filter_words(bloom_words_max) + lds_words_wave<MR, WPQ, NR, LQ, RANKS>()) +
           lds_words_query<MR, WPQ>()) * 4;
 }
 
 template <bool TUNED, int NR, int MR, int J, int WPQ, bool LQ, bool FAST>
 hipError_t launch_f(const SearchArgs& a, int grid, int wpb, hipStream_t st, int* occ) {
-  const size_t lds = search_lds_bytes<MR, WPQ, NR, LQ>(a.bloom_words_max, wpb);
+  const size_t lds =
+      search_lds_bytes<MR, WPQ, NR, LQ, use_ranks<TUNED, NR, MR, J, LQ, FAST>()>(
+          a.bloom_words_max, wpb);
   if (occ) {  // resident workgroups per CU for this shape
     return hipOccupancyMaxActiveBlocksPerMultiprocessor(
         occ, search_kernel<TUNED, NR, MR, J, WPQ, LQ, FAST>, 64 * wpb, lds);
@@ -1413,12 +1445,17 @@ hipError_t launch_f(const SearchArgs& a, int grid, int wpb, hipStream_t st, int*
 // dims, bases of 4 GiB, 16.7M rows or 16 MiB a row and more, several waves per
 // query) takes the general form, and so does d = 960, where the launches are bound
 // by L2 misses: 10k queries in leaf order took 0.92 to 1.10 of the general form's
-// time with the FAST one, by how the queries happened to share rows.
+// time with the FAST one, by how the queries happened to share rows.  TUNED with
+// 256 slots beside a filter of more than 1024 words takes it too: with the ranks' LDS
+// three workgroups of four waves fit a CU there, without it four (1178 against 1058
+// us at 2048 words, d = 128).
 template <bool TUNED, int NR, int MR, int J, int WPQ, bool LQ>
 hipError_t launch_t(const SearchArgs& a, int grid, int wpb, hipStream_t st, int* occ) {
   if constexpr (MR == 1 && WPQ == 1 && J <= 8) {
     if (a.width == 1 && a.d == 32 * J && a.np < (1 << 24) && a.stride < (1 << 22) &&
-        (uint64_t)a.np * (uint64_t)a.stride <= (1ull << 30))
+        (uint64_t)a.np * (uint64_t)a.stride <= (1ull << 30) &&
+        !(NR == 4 && !LQ && use_ranks<TUNED, NR, MR, J, LQ, true>() &&
+          a.bloom_words_max > 1024))
       return launch_f<TUNED, NR, MR, J, WPQ, LQ, true>(a, grid, wpb, st, occ);
   }
   return launch_f<TUNED, NR, MR, J, WPQ, LQ, false>(a, grid, wpb, st, occ);
